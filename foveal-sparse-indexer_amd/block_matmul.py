@@ -191,11 +191,64 @@ def _expand_tiles(m: Tensor, N: int, K: int, block_k: int, block_n: int) -> Tens
     return m.view(nkb, nnb).t().repeat_interleave(block_n, 0).repeat_interleave(block_k, 1)
 
 
+def _tile_bwd_supported(M: int, N: int, groups: int, rpg: int, block_k: int, block_n: int) -> bool:
+    """Tilings fsi_blockwise_matmul_bwd takes (include/fsi.h) and is the faster form of.
+
+    One row group is the only form in which the library runs two whole dense products
+    instead of two per group.  Its 128 x 128 output tiles hold up to four 64-wide mask tiles
+    there, so at density 0.5 nearly all of them have work, and many rows hide the library
+    form's masking passes: 64 x 64 tiles of 8192 x 8192 at density 0.5, forward and both
+    gradients, 0.57 / 0.72 / 1.27 ms here and 0.72 / 0.84 / 1.16 ms there for 512 / 1024 /
+    2048 rows (4096 x 4096: 0.23 / 0.26 / 0.345 and 0.245 / 0.27 / 0.34); 128 x 128 tiles
+    0.66 and 1.00 ms for 2048 rows."""
+    block = lambda b: b == 64 or b % 128 == 0  # noqa: E731
+    used = -(-M // rpg) if groups > 1 else 1
+    if groups == 1 and 64 in (block_k, block_n) and M > 1024:
+        return False
+    return (M > 0 and block(block_k) and block(block_n) and (groups == 1 or rpg % 128 == 0) and used <= 2048
+            and N // block_n <= 2048)
+
+
+def _aligned16(t: Tensor) -> Tensor:
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+def _blockwise_bwd_fake(x2d, weight, dy, m8, block_k, block_n, rpg, want_dx, want_dw):
+    return (x2d.new_empty(x2d.shape if want_dx else (0,)), weight.new_empty(weight.shape if want_dw else (0,)))
+
+
+@_lib.fsi_op("blockwise_matmul_bwd", _blockwise_bwd_fake)
+def _blockwise_bwd_op(x2d: Tensor, weight: Tensor, dy: Tensor, m8: Tensor, block_k: int, block_n: int, rpg: int,
+                      want_dx: bool, want_dw: bool) -> Tuple[Tensor, Tensor]:
+    """fsi_blockwise_matmul_bwd: (dx, dW), each empty unless wanted."""
+    what = "blockwise_matmul backward"
+    dev = _lib.require_gpu(x2d, weight, dy, m8, what=what)
+    x2d, weight, dy = _aligned16(x2d), _aligned16(weight), _aligned16(dy)
+    M, K = x2d.shape
+    N = weight.shape[0]
+    groups = m8.shape[0]
+    L = _lib.lib()
+    code = _lib.dtype_code(x2d.dtype, what)
+    dx = torch.empty((M, K) if want_dx else (0,), dtype=x2d.dtype, device=dev)
+    dw = torch.empty((N, K) if want_dw else (0,), dtype=weight.dtype, device=dev)
+    # scratch of this call alone: it is as large as the operands, so it is not kept
+    ws = torch.empty(L.fsi_blockwise_matmul_bwd_workspace_size(M, N, K, groups, rpg, code, want_dx, want_dw),
+                     dtype=torch.uint8, device=dev)
+    st = L.fsi_blockwise_matmul_bwd(x2d.data_ptr(), K, weight.data_ptr(), K, dy.data_ptr(), N, m8.data_ptr(), groups,
+                                    rpg, block_k, block_n, M, N, K, code, dx.data_ptr() if want_dx else None, K,
+                                    dw.data_ptr() if want_dw else None, K, ws.data_ptr(), ws.numel(),
+                                    _lib.stream_handle(dev))
+    _lib.check(st, what)
+    return dx, dw
+
+
 class _BlockwiseMatmulFn(torch.autograd.Function):
     """2-D tile-sparse matmul on the HIP kernels with the gradients of the
     reference's per-tile F.linear sum (block_matmul.py:381-392), i.e. of
-    x (W o M)^T: dx = dy (W o M), dW = (dy^T x) o M, row group by row group —
-    library GEMMs in the backward."""
+    x (W o M)^T: dx = dy (W o M), dW = (dy^T x) o M.  Tiles of 64 or multiples
+    of 128 run the HIP backward; other tilings, and a backward that is itself
+    differentiated, run row group by row group on library GEMMs."""
 
     @staticmethod
     def forward(ctx, x2d, weight, m8, block_k, block_n, rpg):
@@ -210,6 +263,10 @@ class _BlockwiseMatmulFn(torch.autograd.Function):
         block_k, block_n, rpg = ctx.meta
         N, K = weight.shape
         M = x2d.shape[0]
+        if not torch.is_grad_enabled() and _tile_bwd_supported(M, N, m8.shape[0], rpg, block_k, block_n):
+            want_dx, want_dw = ctx.needs_input_grad[:2]
+            dx, dw = _blockwise_bwd_op(x2d, weight, dy.to(x2d.dtype), m8, block_k, block_n, rpg, want_dx, want_dw)
+            return dx if want_dx else None, dw if want_dw else None, None, None, None, None
         dx = torch.zeros_like(x2d)
         dw = torch.zeros_like(weight)
         for g in range(m8.shape[0]):  # the groups cover every row (checked in blockwise_matmul)

@@ -89,7 +89,9 @@ struct TileArgs {
   const void* bias;  // optional, block_k == K only: added on the columns of active n blocks
   int64_t lda, ldb, ldc;
   int M, N, K;
-  const uint8_t* mask;  // [groups][nkb * nnb], tile id k_b * nnb + n_b
+  // byte of (row group g, k block kb, n block nb): mask[g ms_g + kb ms_k + nb ms_n]
+  const uint8_t* mask;
+  int64_t ms_g, ms_k, ms_n;
   int groups, rows_per_group, nkb, nnb, block_k, block_n;
   int m_tiles, n_tiles;
   const int32_t* order;  // tile ids heaviest first (tile_order_kernel), or null: dispatch order
@@ -159,21 +161,23 @@ __device__ int tile_kcount_chunk(const TileArgs& g, int mt, int nt, int kb0) {
   const int nsub = g.block_n < TT ? TT / g.block_n : 1;
   const int nb0 = nt * TT / g.block_n;
   const int cnt = (nb0 + nsub < g.nnb ? nb0 + nsub : g.nnb) - nb0;  // 1 .. TT / 16 (block_n >= 16)
-  const uint8_t* col = g.mask + static_cast<int64_t>(grp) * g.nkb * g.nnb + nb0;
+  const uint8_t* col = g.mask + grp * g.ms_g + nb0 * g.ms_n;
   // branch-free: rows past nkb re-read the last row and are not counted, so the
   // chunk's loads issue together
   uint32_t any[ORDER_KB_CHUNK];
 #pragma unroll
   for (int k = 0; k < ORDER_KB_CHUNK; ++k) {
     const int kb = kb0 + k < g.nkb ? kb0 + k : g.nkb - 1;
-    any[k] = col[static_cast<int64_t>(kb) * g.nnb];
+    any[k] = col[kb * g.ms_k];
   }
-  if (cnt > 1) {
+  const int msub = g.rows_per_group < TT ? 2 : 1;  // QUAD tiles: 64-row groups
+  if (cnt > 1 || msub > 1) {
 #pragma unroll
     for (int k = 0; k < ORDER_KB_CHUNK; ++k) {
       const int kb = kb0 + k < g.nkb ? kb0 + k : g.nkb - 1;
-      const uint8_t* row = col + static_cast<int64_t>(kb) * g.nnb;
-      for (int j = 1; j < cnt; ++j) any[k] |= row[j];
+      for (int i = 0; i < msub; ++i)
+        for (int j = 0; j < cnt; ++j)
+          if (grp + i < g.groups) any[k] |= col[kb * g.ms_k + i * g.ms_g + j * g.ms_n];
     }
   }
   int n = 0;
@@ -257,8 +261,14 @@ __global__ __launch_bounds__(ORDER_THREADS) void tile_order_kernel(TileArgs g, i
 // values, a fragment read 8 bf16 (one v_mfma_f32_16x16x32_bf16) or 4 fp32 (four
 // v_mfma_f32_16x16x4_f32, k-step kk taking k = 4 (lane / 16) + kk: A and B use the
 // same k order, so the four steps together cover the 16 k of the row).
-template <typename T, bool MASKED>
+// MASK: NONE one mask byte decides the whole output tile per k block; NSUB several n
+// blocks in the tile; QUAD row groups and n blocks of 64 or more, either below 128: each
+// wave's 64 x 64 quarter lies in one (row group, n block) pair.
+enum TileMask : int { MASK_NONE = 0, MASK_NSUB = 1, MASK_QUAD = 2 };
+template <typename T, int MASK>
 __global__ __launch_bounds__(NTHREADS, WG_PER_CU) void tile_list_gemm_kernel(TileArgs g) {
+  constexpr bool MASKED = MASK != MASK_NONE;
+  static_assert(MASK != MASK_QUAD || NW == 4, "a wave per quarter");
   constexpr bool F32 = sizeof(T) == 4;
   constexpr int KSE = 64 / static_cast<int>(sizeof(T));  // K-step in elements (64 bytes of a row)
   constexpr int CE = 16 / static_cast<int>(sizeof(T));   // elements per 16-byte chunk
@@ -279,8 +289,8 @@ __global__ __launch_bounds__(NTHREADS, WG_PER_CU) void tile_list_gemm_kernel(Til
   // ---- active k blocks of this tile -> klist -----------------------------------
   int grp = m0 / g.rows_per_group;
   grp = grp < g.groups ? grp : g.groups - 1;
-  const uint8_t* gmask = g.mask + static_cast<int64_t>(grp) * g.nkb * g.nnb;
-  const int nsub = MASKED ? TT / g.block_n : 1;
+  const uint8_t* gmask = g.mask + grp * g.ms_g;
+  const int nsub = MASK == MASK_NSUB ? TT / g.block_n : 1;
   const int nb0 = n0 / g.block_n;
   const int rounds = (g.nkb + NTHREADS - 1) / NTHREADS;  // <= LIST_MAX / NTHREADS
   constexpr int MAX_ROUNDS = LIST_MAX / NTHREADS;
@@ -292,9 +302,17 @@ __global__ __launch_bounds__(NTHREADS, WG_PER_CU) void tile_list_gemm_kernel(Til
     if (i < rounds) {
       const int kb = i * NTHREADS + tid;
       if (kb < g.nkb) {
-        const uint8_t* row = gmask + static_cast<int64_t>(kb) * g.nnb + nb0;
-        for (int j = 0; j < nsub; ++j)
-          if (nb0 + j < g.nnb && row[j]) bits[i] |= 1u << j;
+        if constexpr (MASK == MASK_QUAD) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {  // quarter (j / 2, j % 2)
+            const int rg = (m0 + 64 * (j >> 1)) / g.rows_per_group, nb = (n0 + 64 * (j & 1)) / g.block_n;
+            if (rg < g.groups && nb < g.nnb && g.mask[rg * g.ms_g + kb * g.ms_k + nb * g.ms_n]) bits[i] |= 1u << j;
+          }
+        } else {
+          const uint8_t* row = gmask + kb * g.ms_k + nb0 * g.ms_n;
+          for (int j = 0; j < nsub; ++j)
+            if (nb0 + j < g.nnb && row[j * g.ms_n]) bits[i] |= 1u << j;
+        }
       }
     }
   }
@@ -372,7 +390,8 @@ __global__ __launch_bounds__(NTHREADS, WG_PER_CU) void tile_list_gemm_kernel(Til
   const int frow = lane & 15, fchunk = lane >> 4;
   int fsub[FB];  // n block (within the tile) of each B fragment
 #pragma unroll
-  for (int f = 0; f < FB; ++f) fsub[f] = MASKED ? (WCOLS * wn + 16 * f) / g.block_n : 0;
+  for (int f = 0; f < FB; ++f)
+    fsub[f] = MASK == MASK_QUAD ? 2 * wm + wn : MASK == MASK_NSUB ? (WCOLS * wn + 16 * f) / g.block_n : 0;
   auto read_frags = [&](int stage, u32x4_t (&fa)[4], u32x4_t (&fb)[FB]) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -396,6 +415,9 @@ __global__ __launch_bounds__(NTHREADS, WG_PER_CU) void tile_list_gemm_kernel(Til
 #pragma unroll
       for (int f = 0; f < FB; ++f)
         if (!((on >> fsub[f]) & 1u)) fb[f] = u32x4_t{0u, 0u, 0u, 0u};
+      if (MASK == MASK_QUAD && !((on >> fsub[0]) & 1u))
+#pragma unroll
+        for (int i = 0; i < 4; ++i) fa[i] = u32x4_t{0u, 0u, 0u, 0u};
     }
   };
   auto mfmas = [&](const u32x4_t (&fa)[4], const u32x4_t (&fb)[FB]) {
@@ -487,14 +509,14 @@ __global__ __launch_bounds__(NTHREADS, WG_PER_CU) void tile_list_gemm_kernel(Til
   T* C = static_cast<T*>(g.C);
   if (g.bias) {  // block_k == K: the bias of the columns whose n block is active
     const T* bias = static_cast<const T*>(g.bias);
-    const uint8_t* row0 = g.mask + static_cast<int64_t>(grp) * g.nkb * g.nnb;
+    const uint8_t* row0 = g.mask + grp * g.ms_g;
 #pragma unroll
     for (int f = 0; f < FB; ++f)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int n = ccol + 16 * f + j;
         float bv = 0.f;
-        if (n < g.N && row0[n / g.block_n]) {
+        if (n < g.N && row0[n / g.block_n * g.ms_n]) {
           if constexpr (F32) bv = bias[n];
           else bv = bf16_to_f32(bias[n]);
         }
@@ -537,6 +559,43 @@ __global__ __launch_bounds__(NTHREADS, WG_PER_CU) void tile_list_gemm_kernel(Til
   }
 }
 
+// dst[c][r] = src[r][c] for r < R, 0 for R <= r < ldd: the operand layout of a product
+// that contracts over src's rows.  64 x 64 tiles through LDS, 16-byte loads and stores
+// on both sides (C a multiple of 64, ldd of 16 / sizeof(T), 16-byte aligned rows).
+template <typename T>
+__global__ __launch_bounds__(256) void transpose_pad_kernel(const T* __restrict__ src, int64_t ld, int R,
+                                                            T* __restrict__ dst, int64_t ldd) {
+  constexpr int V = 16 / static_cast<int>(sizeof(T)), LS = 64 + V;  // LS: 16-byte aligned rows, shifted banks
+  __shared__ __attribute__((aligned(16))) T tile[64 * LS];          // [c][r]
+  const int r0 = blockIdx.x * 64, c0 = blockIdx.y * 64;
+  constexpr int CV = 64 / V;  // vectors per row
+  for (int i = threadIdx.x; i < 64 * CV; i += 256) {
+    // rows fastest: one wave writes a vector's columns as 64 consecutive elements each
+    const int r = i & 63, c = i / 64 * V;
+    u32x4_t v = u32x4_t{0u, 0u, 0u, 0u};
+    if (r0 + r < R) v = *reinterpret_cast<const u32x4_t*>(src + static_cast<int64_t>(r0 + r) * ld + c0 + c);
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      if constexpr (sizeof(T) == 2) tile[(c + e) * LS + r] = static_cast<T>(v[e / 2] >> (16 * (e & 1)));
+      else tile[(c + e) * LS + r] = __builtin_bit_cast(T, static_cast<uint32_t>(v[e]));
+    }
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < 64 * CV; i += 256) {
+    const int c = i / CV, r = i % CV * V;
+    if (r0 + r < ldd)
+      *reinterpret_cast<u32x4_t*>(dst + static_cast<int64_t>(c0 + c) * ldd + r0 + r) =
+          *reinterpret_cast<const u32x4_t*>(&tile[c * LS + r]);
+  }
+}
+
+// Rows of a product that contracts over x's rows: whole row groups (of rows_per_group), or
+// M rounded up to a K-step when one group covers every row.
+int64_t padded_rows(int64_t M, int64_t groups, int64_t rows_per_group) {
+  const int64_t u = groups > 1 ? rows_per_group : KS;
+  return (M + u - 1) / u * u;
+}
+
 }  // namespace
 
 namespace fsi_tile {
@@ -546,15 +605,18 @@ namespace fsi_tile {
 // row groups of whole 128-row tiles, 16-byte aligned rows.  Returns 1 when the
 // shape does not fit (the caller runs the generic kernel), else an FSI status.
 // `order_ws` (tiles int32, may be null) takes the heaviest-first tile order.
-int tile_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, const uint8_t* mask,
-              int64_t groups, int64_t rows_per_group, int64_t block_k, int64_t block_n, int64_t M, int64_t N,
-              int64_t K, int dtype, void* out, int64_t ldo, int32_t* order_ws, hipStream_t st) {
+int tile_gemm_strided(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, const uint8_t* mask,
+                      int64_t ms_g, int64_t ms_k, int64_t ms_n, int64_t groups, int64_t rows_per_group,
+                      int64_t block_k, int64_t block_n, int64_t M, int64_t N, int64_t K, int dtype, void* out,
+                      int64_t ldo, int32_t* order_ws, hipStream_t st) {
   using namespace fsi_host;
   const int64_t esz = dtype == FSI_DTYPE_F32 ? 4 : 2;
   const int64_t kse = 64 / esz, ce = 16 / esz;
   const int64_t nkb = K / block_k, nnb = N / block_n;
+  // 64-row groups (the weight gradient's rows are one n block's): quarters of a tile
+  const bool quad = groups > 1 && rows_per_group % TT != 0 && (rows_per_group == 64 && (block_n == 64 || block_n % TT == 0));
   const bool tiles_ok = block_k % kse == 0 && (block_n % TT == 0 || (TT % block_n == 0 && block_n >= 16)) &&
-                        nkb <= LIST_MAX && (rows_per_group % TT == 0 || groups == 1) &&
+                        nkb <= LIST_MAX && (rows_per_group % TT == 0 || groups == 1 || quad) &&
                         (bias == nullptr || nkb == 1);
   const bool aligned = ldx % ce == 0 && ldw % ce == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
                        (reinterpret_cast<uintptr_t>(w) & 15) == 0;  // 16-byte direct-to-LDS loads
@@ -571,6 +633,9 @@ int tile_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, const void
   a.N = (int)N;
   a.K = (int)K;
   a.mask = mask;
+  a.ms_g = ms_g;
+  a.ms_k = ms_k;
+  a.ms_n = ms_n;
   a.groups = (int)groups;
   a.rows_per_group = (int)(rows_per_group < 0x7fffffff ? rows_per_group : 0x7fffffff);
   a.nkb = (int)nkb;
@@ -593,15 +658,27 @@ int tile_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, const void
     a.order = order_ws;
   }
   if (dtype == FSI_DTYPE_F32) {
-    if (block_n < TT) tile_list_gemm_kernel<float, true><<<grid, NTHREADS, 0, st>>>(a);
-    else tile_list_gemm_kernel<float, false><<<grid, NTHREADS, 0, st>>>(a);
+    if (quad) tile_list_gemm_kernel<float, MASK_QUAD><<<grid, NTHREADS, 0, st>>>(a);
+    else if (block_n < TT) tile_list_gemm_kernel<float, MASK_NSUB><<<grid, NTHREADS, 0, st>>>(a);
+    else tile_list_gemm_kernel<float, MASK_NONE><<<grid, NTHREADS, 0, st>>>(a);
   } else {
-    if (block_n < TT) tile_list_gemm_kernel<bf16_t, true><<<grid, NTHREADS, 0, st>>>(a);
-    else tile_list_gemm_kernel<bf16_t, false><<<grid, NTHREADS, 0, st>>>(a);
+    if (quad) tile_list_gemm_kernel<bf16_t, MASK_QUAD><<<grid, NTHREADS, 0, st>>>(a);
+    else if (block_n < TT) tile_list_gemm_kernel<bf16_t, MASK_NSUB><<<grid, NTHREADS, 0, st>>>(a);
+    else tile_list_gemm_kernel<bf16_t, MASK_NONE><<<grid, NTHREADS, 0, st>>>(a);
   }
   const hipError_t e = hipGetLastError();
   FSI_CHECK_ARG(e == hipSuccess, FSI_ERR_HIP, "blockwise_matmul: launch failed: %s", hipGetErrorString(e));
   return FSI_OK;
+}
+
+// The forward's form: mask tile id k_b nnb + n_b, groups of whole 128-row tiles.
+int tile_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, const uint8_t* mask,
+              int64_t groups, int64_t rows_per_group, int64_t block_k, int64_t block_n, int64_t M, int64_t N,
+              int64_t K, int dtype, void* out, int64_t ldo, int32_t* order_ws, hipStream_t st) {
+  if (groups > 1 && rows_per_group % TT != 0) return 1;
+  const int64_t nkb = K / block_k, nnb = N / block_n;
+  return tile_gemm_strided(x, ldx, w, ldw, bias, mask, nkb * nnb, nnb, 1, groups, rows_per_group, block_k, block_n, M,
+                           N, K, dtype, out, ldo, order_ws, st);
 }
 
 }  // namespace fsi_tile
@@ -651,6 +728,117 @@ FSI_API int fsi_blockwise_matmul(const void* x, int64_t ldx, const void* w, int6
   // tilings the list kernel does not take: the generic kernel
   return fsi_bs_generic::tile_gemm(x, ldx, w, ldw, nullptr, tile_mask, groups, rows_per_group, block_k, block_n, M,
                                    N, K, dtype, out, ldo, st);
+}
+
+}  // extern "C"
+
+namespace {
+
+bool tile_bwd_block(int64_t b) { return b == 64 || (b > 0 && b % TT == 0); }
+
+int64_t tile_count(int64_t R, int64_t C) { return ((R + TT - 1) / TT) * ((C + TT - 1) / TT); }
+
+// Byte offsets of the backward's workspace after the counter area: the tile order, then
+// W^T (K x N), dy^T (N x Mp) and x^T (K x Mp), as far as they are needed.
+struct TileBwdWs {
+  size_t order, wt, dyt, xt, end;
+};
+TileBwdWs tile_bwd_ws(int64_t M, int64_t N, int64_t K, int64_t Mp, int64_t esz, bool dx, bool dw) {
+  using fsi_host::align_up;
+  TileBwdWs o{};
+  o.order = FSI_WORKSPACE_COUNTER_BYTES;
+  const int64_t tx = dx ? tile_count(M, K) : 0, tw = dw ? tile_count(N, K) : 0;
+  o.wt = o.order + align_up(static_cast<size_t>(tx > tw ? tx : tw) * sizeof(int32_t), 256);
+  o.dyt = o.wt + (dx ? align_up(static_cast<size_t>(K * N * esz), 256) : 0);
+  o.xt = o.dyt + (dw ? align_up(static_cast<size_t>(N * Mp * esz), 256) : 0);
+  o.end = o.xt + (dw ? align_up(static_cast<size_t>(K * Mp * esz), 256) : 0);
+  return o;
+}
+
+template <typename T>
+void transpose_launch(const void* src, int64_t ld, int64_t R, int64_t C, void* dst, int64_t ldd, hipStream_t st) {
+  transpose_pad_kernel<T><<<dim3(static_cast<unsigned>((ldd + 63) / 64), static_cast<unsigned>(C / 64)), 256, 0, st>>>(
+      static_cast<const T*>(src), ld, static_cast<int>(R), static_cast<T*>(dst), ldd);
+}
+
+}  // namespace
+
+extern "C" {
+
+FSI_API size_t fsi_blockwise_matmul_bwd_workspace_size(int64_t M, int64_t N, int64_t K, int64_t groups,
+                                                       int64_t rows_per_group, int dtype, int want_dx, int want_dw) {
+  if (M <= 0 || N <= 0 || K <= 0 || groups <= 0 || rows_per_group <= 0) return FSI_WORKSPACE_COUNTER_BYTES;
+  return tile_bwd_ws(M, N, K, padded_rows(M, groups, rows_per_group), dtype == FSI_DTYPE_F32 ? 4 : 2, want_dx != 0,
+                     want_dw != 0)
+      .end;
+}
+
+// Gradients of fsi_blockwise_matmul on the same list-driven GEMM: dx = dy (W o T) contracts
+// over the n blocks active for its row group and k block, dW = (dy^T x) o T over the row
+// groups whose mask has the tile, so both do the forward's operations and sum in fp32 (the
+// masked dense products of the library form do 1 / density times as many and write W o T
+// for every group).  4096 x 8192 x 8192 at 25 % in 32 groups: 15.0 -> 0.52 ms for both
+// gradients, 225 us for each GEMM (610 TFLOP/s, as the forward: the operand stream of its
+// 128 x 128 tiles bounds it).  The GEMM wants both operands contraction-major, so W (for
+// dx), dy and x (for dW) are transposed first, 128 of the 520 us (4.2 TB/s).
+FSI_API int fsi_blockwise_matmul_bwd(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* dy,
+                                     int64_t lddy, const uint8_t* tile_mask, int64_t groups, int64_t rows_per_group,
+                                     int64_t block_k, int64_t block_n, int64_t M, int64_t N, int64_t K, int dtype,
+                                     void* dx, int64_t lddx, void* dw, int64_t lddw, void* workspace,
+                                     size_t workspace_bytes, void* stream) {
+  using namespace fsi_host;
+  FSI_CHECK_ARG(dtype == FSI_DTYPE_BF16 || dtype == FSI_DTYPE_F32, FSI_ERR_DTYPE, "blockwise_matmul_bwd: dtype %d",
+                dtype);
+  FSI_CHECK_ARG(M > 0 && N > 0 && K > 0 && groups > 0 && rows_per_group > 0 && M <= 0x7fffff00 && N <= 0x7fffff00 &&
+                    K <= 0x7fffff00 && K / 64 <= 65535 && N / 64 <= 65535,
+                FSI_ERR_SHAPE, "blockwise_matmul_bwd: bad sizes");
+  FSI_CHECK_ARG(tile_bwd_block(block_k) && tile_bwd_block(block_n) && K % block_k == 0 && N % block_n == 0,
+                FSI_ERR_SHAPE, "blockwise_matmul_bwd: tiles %lldx%lld (64 or a multiple of 128, dividing K and N)",
+                (long long)block_k, (long long)block_n);
+  FSI_CHECK_ARG(groups == 1 || (rows_per_group % TT == 0 && groups * rows_per_group >= M), FSI_ERR_SHAPE,
+                "blockwise_matmul_bwd: %lld row groups of %lld rows", (long long)groups, (long long)rows_per_group);
+  const int64_t used = groups > 1 ? (M + rows_per_group - 1) / rows_per_group : 1;
+  FSI_CHECK_ARG(used <= LIST_MAX && N / block_n <= LIST_MAX, FSI_ERR_CAPACITY,
+                "blockwise_matmul_bwd: %lld groups, %lld column blocks", (long long)used, (long long)(N / block_n));
+  FSI_CHECK_ARG(dy && tile_mask && (dx || dw) && (!dx || w) && (!dw || x), FSI_ERR_INVALID_ARG,
+                "blockwise_matmul_bwd: null pointer");
+  const int64_t esz = dtype == FSI_DTYPE_F32 ? 4 : 2, ce = 16 / esz;
+  auto rows_ok = [&](const void* p, int64_t ld, int64_t cols) {
+    return !p || (reinterpret_cast<uintptr_t>(p) % 16 == 0 && ld % ce == 0 && ld >= cols);
+  };
+  FSI_CHECK_ARG(rows_ok(x, ldx, K) && rows_ok(w, ldw, K) && rows_ok(dy, lddy, N) && (!dx || lddx >= K) &&
+                    (!dw || lddw >= K),
+                FSI_ERR_ALIGN, "blockwise_matmul_bwd: rows must be 16-byte aligned");
+  const int64_t Mp = padded_rows(M, groups, rows_per_group);
+  const TileBwdWs o = tile_bwd_ws(M, N, K, Mp, esz, dx != nullptr, dw != nullptr);
+  FSI_CHECK_ARG(workspace && workspace_bytes >= o.end && reinterpret_cast<uintptr_t>(workspace) % 16 == 0,
+                FSI_ERR_WORKSPACE, "blockwise_matmul_bwd: workspace %zu < %zu (or misaligned)", workspace_bytes, o.end);
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  char* ws = static_cast<char*>(workspace);
+  int32_t* order = reinterpret_cast<int32_t*>(ws + o.order);
+  const int64_t nkb = K / block_k, nnb = N / block_n;
+  auto transpose = [&](const void* src, int64_t ld, int64_t R, int64_t C, void* dst, int64_t ldd) {
+    if (esz == 4) transpose_launch<float>(src, ld, R, C, dst, ldd, st);
+    else transpose_launch<bf16_t>(src, ld, R, C, dst, ldd, st);
+  };
+  if (dx) {
+    transpose(w, ldw, N, K, ws + o.wt, N);
+    const int rc = fsi_tile::tile_gemm_strided(dy, lddy, ws + o.wt, N, nullptr, tile_mask, nkb * nnb, 1, nnb, groups,
+                                               rows_per_group, block_n, block_k, M, K, N, dtype, dx, lddx, order, st);
+    FSI_CHECK_ARG(rc <= 0, FSI_ERR_SHAPE, "blockwise_matmul_bwd: tiling");
+    if (rc != FSI_OK) return rc;
+  }
+  if (dw) {
+    transpose(dy, lddy, M, N, ws + o.dyt, Mp);
+    transpose(x, ldx, M, K, ws + o.xt, Mp);
+    const int rc = fsi_tile::tile_gemm_strided(ws + o.dyt, Mp, ws + o.xt, Mp, nullptr, tile_mask, 1, nkb * nnb, nnb,
+                                               nnb, block_n, groups > 1 ? rows_per_group : Mp, block_k, N, K, Mp, dtype,
+                                               dw, lddw, order, st);
+    FSI_CHECK_ARG(rc <= 0, FSI_ERR_SHAPE, "blockwise_matmul_bwd: tiling");
+    if (rc != FSI_OK) return rc;
+  }
+  FSI_HIP_LAUNCH_CHECK("blockwise_matmul_bwd");
+  return FSI_OK;
 }
 
 }  // extern "C"

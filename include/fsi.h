@@ -581,6 +581,21 @@ FSI_API int fsi_blockwise_matmul(const void* x, int64_t ldx, const void* w, int6
                                  int64_t block_n, int64_t M, int64_t N, int64_t K, int dtype, void* out, int64_t ldo,
                                  void* workspace, size_t workspace_bytes, void* stream);
 
+/* Gradients of fsi_blockwise_matmul: dx = dy (w o T) and dw = (dy^T x) o T (autograd of
+ * block_matmul.py:381-392), fp32 sums, each written if its pointer is given (x is read for
+ * dw, w for dx).  block_k and block_n 64 or a multiple of 128; rows_per_group a multiple of
+ * 128 unless groups = 1; at most 2048 row groups and 2048 column blocks; 16-byte aligned
+ * x, w and dy rows.  Workspace: fsi_blockwise_matmul_bwd_workspace_size bytes (transposed
+ * copies of the operands that are contracted over their rows). */
+FSI_API size_t fsi_blockwise_matmul_bwd_workspace_size(int64_t M, int64_t N, int64_t K, int64_t groups,
+                                                       int64_t rows_per_group, int dtype, int want_dx, int want_dw);
+
+FSI_API int fsi_blockwise_matmul_bwd(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* dy,
+                                     int64_t lddy, const uint8_t* tile_mask, int64_t groups, int64_t rows_per_group,
+                                     int64_t block_k, int64_t block_n, int64_t M, int64_t N, int64_t K, int dtype,
+                                     void* dx, int64_t lddx, void* dw, int64_t lddw, void* workspace,
+                                     size_t workspace_bytes, void* stream);
+
 /* 2-D tile routing of BlockwiseMatMul2D (foveal_indexer/block_matmul.py:355-377).
  * Per row r of scores (rows x n_tiles, row stride ld_scores, fp32 or bf16):
  * p = softmax(row) (rounded to bf16 for bf16 rows), tiles ranked by p
