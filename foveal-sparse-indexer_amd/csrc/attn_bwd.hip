@@ -60,9 +60,10 @@ struct AbParams {
   int64_t cs_b, cs_q;
   float scale;
   int nb;             // blocks of the pattern: ceil(T / block)
+  int64_t tp;         // T rounded up to whole tiles
   bool vec4;          // head_dim one of the tile widths (16 / 32 / 64 / 128), rows 4-element aligned
   int32_t* map;       // (B, nb, nb) weight classes
-  float* stat_m;      // (B, Hq, T)
+  float* stat_m;      // (B, Hq, T); the bf16 kernels: lse2 and D, (B, Hq, tp)
   float* stat_l;
   float* stat_d;
   float* dq;          // (B, Hq, T, hd) fp32, contiguous
@@ -538,88 +539,105 @@ __global__ __launch_bounds__(AB_THREADS) void sab_kv_kernel(AbParams P) {
 }
 
 // ---------------------------------------------------------------------------
-// bf16 inputs with head_dim 32 / 64 / 128 and 4-element-aligned rows: every
-// product on v_mfma_f32_16x16x32_bf16.  Tiles sit in LDS as bf16, row-major at
-// stride HD + 8 (the 8 rows a 128-bit read serves at once start on distinct
-// bank quads) and, where a product contracts over the tile's rows, transposed
-// as well at stride 64 + 4 (the 16 rows of a 64-bit read on distinct bank
-// pairs).  P and dS enter their products as a pair of bf16 operands hi + lo
-// (hi = the value rounded to bf16, lo = the remainder rounded): the pair holds
-// the value to ~2^-17 relative, the other operand is an exact bf16 input and
-// the MFMA accumulates in fp32.
+// bf16 inputs with head_dim 32 / 64 / 128 and 8-element-aligned rows: every product on
+// v_mfma_f32_16x16x32_bf16 over 64-row tiles moved straight into LDS (no staging
+// registers), double-buffered: the next tile's loads run while this one is used.
 //
-// A lane's k slots 8 kg + e of a 32-row product: rows 4 kg + e (e < 4) and
-// 16 + 4 kg + e - 4 (e >= 4) of the 32, i.e. the rows its two 16 x 16
-// accumulators of P / dS hold, so those enter the MFMA where they are; the
-// transposed tile is read at the same rows.
+// What bounds these kernels is LDS, not the matrix cores: an operand fragment is 1 KiB
+// (8 LDS clocks) and feeds a 16-clock MFMA on one of four SIMDs, so a fragment has to
+// serve two MFMAs at least.  Each wave therefore owns 32 rows (two 16-row operands in
+// registers) of its side, and P / dS enter their products as a pair of bf16 operands
+// hi + lo (hi = the value rounded to bf16, lo = the remainder rounded; ~2^-17 relative,
+// the other operand an exact bf16 input, fp32 accumulation), which makes it four there.
+// The tiles are stored row-major only: products that contract over a tile's rows read it
+// with ds_read_b64_tr_b16, so no transposed copy is written.
+// 8192 tokens, 32 / 8 heads of 128, window 1024 + 32 pages: sab_q 1521 -> 1026 us,
+// sab_kv 1763 -> 1125 us against 16 rows a wave over padded row-major and
+// transposed tiles staged in registers (four heads a workgroup in sab_q: 2 % slower).
+// Sub-tile classes: block 16, 2 x 4096 tokens, 8 / 2 heads of 128 2480 -> 925 us.
+//
+// 16-byte piece p of row r sits at piece p ^ sab_swz(r): the 8 rows a 128-bit read serves
+// at once fall on distinct bank quads, and the 4 rows x 32 bytes that 16 lanes of a
+// transposing read cover fill one bank period (head_dim 32: two rows share a period and
+// the transposing reads conflict pairwise).
+//
+// A lane's k slots of a 32-row product: rows 4 kg + e (e < 4) and 16 + 4 kg + e - 4
+// (e >= 4), i.e. the rows its two 16 x 16 accumulators of P / dS hold, so those enter the
+// MFMA where they are; the transposing reads take the same rows.
 // ---------------------------------------------------------------------------
-constexpr int BF_TS = AB_T + 4;  // transposed-tile row stride (bf16 elements)
+typedef __attribute__((address_space(3))) void ab_lds_t;
+typedef __attribute__((address_space(1))) void ab_glb_t;
+typedef __attribute__((__vector_size__(4 * sizeof(short)))) short s16x4_t;
+typedef __attribute__((address_space(3))) s16x4_t ab_tr_t;
 
-// Rows [r0, r0 + 64) of a (T, HD) bf16 matrix move in two halves, so the next
-// tile's loads can be in flight while the current tile is used: bf_load reads
-// them into registers (thread = 4-row group x 4-dim group, one 8-byte load per
-// row; rows past T read as 0), bf_store writes them to the row-major tile rt
-// and, when TR, to the transposed tile tt after a 4 x 4 transpose in registers.
-// Transposed rows d hold their 4-column groups in the order g ^ ((d >> 4) & 3):
-// the 16 rows 4 apart that one store instruction writes then land on distinct
-// banks, and the 16 consecutive rows of an operand read (one swizzle value)
-// stay on distinct bank pairs.
 template <int HD>
-constexpr int bf_rounds() { return HD >= 64 ? HD / 64 : 1; }
-
-// Rows past T re-read row T - 1: every product that uses them is multiplied by
-// a zero P / dS or masked, so they only need to be finite.
-template <int HD>
-__device__ __forceinline__ void bf_load(const bf16_t* base, int64_t rs, int r0, int T, uint2 (&x)[bf_rounds<HD>()][4]) {
-  constexpr int DGN = HD / 4, QG = AB_THREADS / DGN;
-  const int dg = threadIdx.x % DGN;
-  const int qg0 = QG * bf_rounds<HD>() > AB_T / 4 ? (threadIdx.x / DGN) % (AB_T / 4) : threadIdx.x / DGN;
-  if (r0 + AB_T <= T) {
-    // every row inside: a scalar row base and 32-bit lane offsets (row strides
-    // below 2^24 elements, host-checked), one add per load
-    const char* rb = reinterpret_cast<const char*>(base + static_cast<int64_t>(r0) * rs);
-    const uint32_t rsb = static_cast<uint32_t>(rs) * 2u;
-    const uint32_t lo = static_cast<uint32_t>(4 * qg0) * rsb + 8u * static_cast<uint32_t>(dg);
-#pragma unroll
-    for (int rr = 0; rr < bf_rounds<HD>(); ++rr)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        x[rr][j] = *reinterpret_cast<const uint2*>(rb + (lo + static_cast<uint32_t>(4 * rr * QG + j) * rsb));
-    return;
-  }
-#pragma unroll
-  for (int rr = 0; rr < bf_rounds<HD>(); ++rr)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int r = r0 + 4 * (qg0 + rr * QG) + j;
-      x[rr][j] = *reinterpret_cast<const uint2*>(base + static_cast<int64_t>(r < T ? r : T - 1) * rs + 4 * dg);
-    }
+__device__ __forceinline__ int sab_swz(int row) {
+  return HD >= 64 ? ((row & 3) << 1) | ((row >> 2) & 1) : (row >> 1) & 3;
 }
 
-template <int HD, bool TR>
-__device__ __forceinline__ void bf_store(const uint2 (&x)[bf_rounds<HD>()][4], bf16_t* rt, bf16_t* tt) {
-  constexpr int DGN = HD / 4, QG = AB_THREADS / DGN;
-  const int dg = threadIdx.x % DGN, qg0 = threadIdx.x / DGN;
+template <int HD>
+constexpr int sab_tile_bytes() { return AB_T * HD * 2; }
+
+// Rows [r0, r0 + 64) of a (T, HD) bf16 matrix at row stride rs into the LDS tile, by NT
+// threads; rows past T re-read row T - 1 (every product that uses them is multiplied by a
+// zero P / dS or never stored, so they only need to be finite).  Row strides are below
+// 2^24 elements (host-checked): a scalar row base and 32-bit lane offsets.
+template <int HD, int NT>
+__device__ __forceinline__ void sab_dma(const bf16_t* base, int64_t rs, int r0, int T, char* tile) {
+  constexpr int PC = HD / 8, ROWS = NT / PC, N = AB_T / ROWS > 0 ? AB_T / ROWS : 1;
+  static_assert(ROWS % 8 == 0, "a thread's rows share their swizzle");
+  if (NT > AB_T * PC && threadIdx.x >= AB_T * PC) return;
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));  // offsets are formed here, not kept in registers over the caller's loop
+  const int row = tid / PC, lp = (tid % PC) ^ sab_swz<HD>(row);
+  const uint32_t rsb = static_cast<uint32_t>(rs) * 2u;
+  const char* rb = reinterpret_cast<const char*>(base + static_cast<int64_t>(r0) * rs);
+  char* dst = tile + (threadIdx.x & ~63u) * 16;
+  if (r0 + AB_T <= T) {
+    // scalar bases and one lane offset: nothing else is kept in registers over the loop
+    const uint32_t lo = static_cast<uint32_t>(row) * rsb + 16u * static_cast<uint32_t>(lp);
 #pragma unroll
-  for (int rr = 0; rr < bf_rounds<HD>(); ++rr) {
-    const int qg = qg0 + rr * QG;
-    if (QG * bf_rounds<HD>() > AB_T / 4 && qg >= AB_T / 4) continue;
+    for (int j = 0; j < N; ++j)
+      __builtin_amdgcn_global_load_lds((ab_glb_t*)(rb + static_cast<uint64_t>(j * ROWS) * rsb + lo),
+                                       (ab_lds_t*)(dst + j * NT * 16), 16, 0, 0);
+  } else {
+    const int last = T - 1 - r0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) *reinterpret_cast<uint2*>(&rt[(4 * qg + j) * (HD + 8) + 4 * dg]) = x[rr][j];
-    if constexpr (TR) {
-      constexpr uint32_t LO = 0x05040100u, HI = 0x07060302u;  // low / high bf16 of each source
-      const uint2* y = x[rr];
-      bf16_t* t = &tt[4 * dg * BF_TS + 4 * (qg ^ ((dg >> 2) & 3))];
-      *reinterpret_cast<uint2*>(t) =
-          make_uint2(__builtin_amdgcn_perm(y[1].x, y[0].x, LO), __builtin_amdgcn_perm(y[3].x, y[2].x, LO));
-      *reinterpret_cast<uint2*>(t + BF_TS) =
-          make_uint2(__builtin_amdgcn_perm(y[1].x, y[0].x, HI), __builtin_amdgcn_perm(y[3].x, y[2].x, HI));
-      *reinterpret_cast<uint2*>(t + 2 * BF_TS) =
-          make_uint2(__builtin_amdgcn_perm(y[1].y, y[0].y, LO), __builtin_amdgcn_perm(y[3].y, y[2].y, LO));
-      *reinterpret_cast<uint2*>(t + 3 * BF_TS) =
-          make_uint2(__builtin_amdgcn_perm(y[1].y, y[0].y, HI), __builtin_amdgcn_perm(y[3].y, y[2].y, HI));
+    for (int j = 0; j < N; ++j) {
+      const uint32_t lo = static_cast<uint32_t>(min(j * ROWS + row, last)) * rsb + 16u * static_cast<uint32_t>(lp);
+      __builtin_amdgcn_global_load_lds((ab_glb_t*)(rb + lo), (ab_lds_t*)(dst + j * NT * 16), 16, 0, 0);
     }
   }
+}
+
+// LDS byte offsets of a lane's reads inside a tile: every fragment's address is one of
+// these plus the tile's, xored with its step's piece, plus a constant, so a loop keeps two
+// registers of them and not one per fragment.
+//   row: row (lane & 15) of the 128-bit operand reads (32-dim step ks in bits 6 and up);
+//   tr: row 4 kg + r / 4, 4-dim group r % 4 of the transposing reads (dims 16 dt in bits 5 and up).
+template <int HD>
+__device__ __forceinline__ uint32_t sab_row_off(int r, int kg) {
+  return r * (HD * 2) + 16 * (kg ^ sab_swz<HD>(r));
+}
+template <int HD>
+__device__ __forceinline__ uint32_t sab_tr_off(int r, int kg) {
+  const int row = 4 * kg + (r >> 2);
+  return row * (HD * 2) + 16 * (((r >> 1) & 1) ^ sab_swz<HD>(row)) + 8 * (r & 1);
+}
+// The operand at a row offset (16 rows from a multiple of 16, `at` the constant part) for step ks.
+__device__ __forceinline__ u32x4_t sab_row(const char* smem, uint32_t off, int ks, int at) {
+  typedef __attribute__((address_space(3))) const u32x4_t lds_u32x4_t;
+  typedef __attribute__((address_space(3))) const char lds_char_t;
+  return *(lds_u32x4_t*)((lds_char_t*)smem + ((off ^ (64u * (ks & 1))) + 128 * (ks >> 1) + at));
+}
+// Dims 16 dt + (lane & 15) at the lane's k slots of 32 rows.
+template <int HD>
+__device__ __forceinline__ u32x4_t sab_trow(char* smem, uint32_t off, int dt, int at) {
+  typedef __attribute__((address_space(3))) char lds_char_t;
+  lds_char_t* p = (lds_char_t*)smem + ((off ^ (32u * (dt & 3))) + 128 * (dt >> 2) + at);
+  const u32x2_t x = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((ab_tr_t*)p));
+  const u32x2_t y = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((ab_tr_t*)(p + 16 * HD * 2)));
+  return u32x4_t{x[0], x[1], y[0], y[1]};
 }
 
 // Class of the tile pair (queries [t0, t0 + 64), keys [s0, s0 + 64)) computed by
@@ -634,41 +652,120 @@ __device__ __forceinline__ int sab_pair_class(const AbParams& P, const int32_t* 
   return live ? -1 : 0;
 }
 
-// sab_logits in log2 units for the bf16 kernels: x2 = scale log2(e) q.k + log2(w)
-// (sl2 = scale log2(e)), -inf where the weight is 0 or the query / key is past
-// T.  Tiles of one weight with every query and key inside T take one fma per score.
-__device__ __forceinline__ void sab_logits2(const AbParams& P, const int32_t* map_b, int tq, int kg, int t0, int s0,
-                                            int tcls, float sl2, f32x4_t (&st)[4]) {
-  if (tcls > 0 && (P.mode == FSI_SATTN_BLOCK_LIST || (tcls & 2))) {
-    const float lw2 = P.mode == FSI_SATTN_BLOCK_LIST ? __log2f(static_cast<float>(tcls)) : 0.f;
-    if (t0 + AB_T <= P.T && s0 + AB_T <= P.T) {
+// The live tiles of one tile row (ROW: the query tile at fixed0, key tiles vary) or column,
+// ascending: next() moves to the next one and returns false after the last.  Every wave
+// walks the same list (64 classes a time in a register, the live ones a ballot), so no LDS
+// and no barrier is spent on it.
+template <bool ROW>
+struct SabTiles {
+  const AbParams& P;
+  const int32_t* map_b;
+  int fixed0, ntiles, c0, cls_lane;
+  uint64_t live;
+  int tile, cls;
+  __device__ SabTiles(const AbParams& p, const int32_t* m, int f0, int n) : P(p), map_b(m), fixed0(f0), ntiles(n) {
+    c0 = -64;
+    live = 0;
+  }
+  __device__ __forceinline__ bool next() {
+    while (live == 0) {
+      c0 += 64;
+      if (c0 >= ntiles) return false;
+      const int i = c0 + static_cast<int>(threadIdx.x & 63);
+      cls_lane = 0;
+      if (i < ntiles)
+        cls_lane = ROW ? sab_pair_class(P, map_b, fixed0, i * AB_T) : sab_pair_class(P, map_b, i * AB_T, fixed0);
+      live = __ballot(cls_lane != 0);
+    }
+    const int i = __builtin_ctzll(live);
+    live &= live - 1;
+    tile = c0 + i;
+    cls = __builtin_amdgcn_readlane(cls_lane, i);
+    return true;
+  }
+};
+
+// How a 64 x 64 tile's weights are found (by the pattern's block, host-chosen): one block
+// pair per tile; one per 16 x 16 sub-tile (block a multiple of 16, the class a scalar load);
+// or looked up per element.
+enum SabMix : int { SAB_TILE = 0, SAB_SUB = 1, SAB_ELEM = 2 };
+template <int MIX>
+using sab_mix_t = std::integral_constant<int, MIX>;
+
+// Class of the 16 x 16 sub-tile at queries t0, keys s0 (both wave-uniform); 0 past T.  The
+// constant address space makes it a scalar load, which the vector loads in flight don't delay.
+__device__ __forceinline__ int sab_sub_class(const AbParams& P, const int32_t* map_b, int t0, int s0) {
+  typedef __attribute__((address_space(4))) const int32_t const_i32_t;
+  if (t0 >= P.T || s0 >= P.T) return 0;
+  return ((const_i32_t*)map_b)[static_cast<int64_t>(t0 / P.block) * P.nb + s0 / P.block];
+}
+
+// Logits in log2 units of 4 keys sb + e against query tq (S^T accumulator st) in a tile or
+// sub-tile of class cls > 0: x2 = scale log2(e) q.k + log2(w) (sl2 = scale log2(e)), -inf where
+// the weight is 0 or the query / key is past T.  inner: all of it lies inside T; one weight
+// then takes one fma per score.
+__device__ __forceinline__ void sab_logits4(const AbParams& P, int tq, int sb, int cls, bool inner, float sl2,
+                                            f32x4_t& st) {
+  if (P.mode == FSI_SATTN_BLOCK_LIST || (cls & 2)) {
+    const float lw2 = P.mode == FSI_SATTN_BLOCK_LIST ? __log2f(static_cast<float>(cls)) : 0.f;
+    if (inner) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) st[t][e] = fmaf(st[t][e], sl2, lw2);
+      for (int e = 0; e < 4; ++e) st[e] = fmaf(st[e], sl2, lw2);
     } else {
       const int lim = tq < P.T ? P.T : 0;
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          st[t][e] = s0 + 16 * t + 4 * kg + e < lim ? fmaf(st[t][e], sl2, lw2) : -INFINITY;
+      for (int e = 0; e < 4; ++e) st[e] = sb + e < lim ? fmaf(st[e], sl2, lw2) : -INFINITY;
     }
-  } else if (tcls > 0) {
+  } else {
     const int hi = tq < P.T ? tq : -1, lo = tq - P.window;
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int e = 0; e < 4; ++e) st[e] = sb + e <= hi && sb + e > lo ? st[e] * sl2 : -INFINITY;
+  }
+}
+
+// How the weights of a tile or sub-tile of class cls >= 0 are applied: one weight (all, its
+// log2 lw2), the window only (win), or nothing attended.
+struct SabWeight {
+  bool all, win;
+  float lw2;
+};
+__device__ __forceinline__ SabWeight sab_weight_of(const AbParams& P, int cls) {
+  const bool list = P.mode == FSI_SATTN_BLOCK_LIST;
+  const bool all = cls > 0 && (list || (cls & 2));
+  return {all, cls > 0 && !all, all && list ? __log2f(static_cast<float>(cls)) : 0.f};
+}
+// P of query t and key sk from the raw score and the query's log2 denominator (+inf past T: P = 0).
+__device__ __forceinline__ float sab_p(const AbParams& P, const SabWeight& w, int t, int sk, bool inner, float sl2,
+                                       float lse, float s) {
+  float p = 0.f;
+  if (w.all) {
+    p = __builtin_amdgcn_exp2f(fmaf(s, sl2, w.lw2 - lse));
+    if (!inner) p = sk < P.T ? p : 0.f;
+  } else if (w.win) {
+    const float x = __builtin_amdgcn_exp2f(fmaf(s, sl2, -lse));
+    p = sk <= t && sk > t - P.window ? x : 0.f;
+  }
+  return p;
+}
+
+// sab_logits4 for keys sb + 16 t + 4 kg + e of a tile of class tcls against query tq0 + r.
+template <int N, int MIX>
+__device__ __forceinline__ void sab_logits2(const AbParams& P, const int32_t* map_b, int tq0, int r, int kg, int sb,
+                                            int tcls, bool inner, float sl2, f32x4_t (&st)[N]) {
+  const int tq = tq0 + r;
+#pragma unroll
+  for (int t = 0; t < N; ++t) {
+    const int s0 = sb + 16 * t;
+    if (MIX == SAB_TILE || tcls > 0) {
+      sab_logits4(P, tq, s0 + 4 * kg, tcls, inner, sl2, st[t]);
+    } else if constexpr (MIX == SAB_SUB) {
+      const int cls = sab_sub_class(P, map_b, tq0, s0);
+      if (cls > 0) sab_logits4(P, tq, s0 + 4 * kg, cls, inner, sl2, st[t]);
+      else st[t] = f32x4_t{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    } else {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int sk = s0 + 16 * t + 4 * kg + e;
-        st[t][e] = sk <= hi && sk > lo ? st[t][e] * sl2 : -INFINITY;
-      }
-  } else {
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int sk = s0 + 16 * t + 4 * kg + e;
+        const int sk = s0 + 4 * kg + e;
         float x = -INFINITY;
         if (tq < P.T && sk < P.T) {
           const float w = sab_tile_weight(P, map_b, tcls, tq, sk);
@@ -676,49 +773,8 @@ __device__ __forceinline__ void sab_logits2(const AbParams& P, const int32_t* ma
         }
         st[t][e] = x;
       }
+    }
   }
-}
-
-// The live tiles among [c0, c0 + 256) of one tile row (ROW: the query tile t0 is
-// fixed, key tiles vary) or column (the key tile is fixed), ascending, with their
-// classes, compacted into idx / cls; returns their number (every thread).
-template <bool ROW>
-__device__ __forceinline__ int sab_live_chunk(const AbParams& P, const int32_t* map_b, int fixed0, int c0, int ntiles,
-                                              int* idx, int* cls, int* wcount) {
-  const int i = c0 + static_cast<int>(threadIdx.x), lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int c = 0;
-  if (i < ntiles) c = ROW ? sab_pair_class(P, map_b, fixed0, i * AB_T) : sab_pair_class(P, map_b, i * AB_T, fixed0);
-  const uint64_t bal = __ballot(c != 0);
-  if (lane == 0) wcount[wave] = __popcll(bal);
-  __syncthreads();
-  int base = 0, total = 0;
-#pragma unroll
-  for (int w = 0; w < AB_THREADS / 64; ++w) {
-    base += w < wave ? wcount[w] : 0;
-    total += wcount[w];
-  }
-  if (c != 0) {
-    const int pos = base + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(bal >> 32),
-                                                     __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(bal), 0));
-    idx[pos] = i;
-    cls[pos] = c;
-  }
-  __syncthreads();
-  return total;
-}
-
-// Row `row` of a row-major tile as the lane's operand of a 32-dim step ks.
-template <int HD>
-__device__ __forceinline__ u32x4_t bf_row(const bf16_t* rt, int row, int ks, int kg) {
-  return *reinterpret_cast<const u32x4_t*>(&rt[row * (HD + 8) + 32 * ks + 8 * kg]);
-}
-// Row `row` of a transposed tile at the lane's k slots of the 32 columns
-// [32 j, 32 j + 32): column groups 8 j + kg and 8 j + 4 + kg, stored swizzled.
-__device__ __forceinline__ u32x4_t bf_trow(const bf16_t* tt, int row, int j, int kg) {
-  const int sw = kg ^ ((row >> 4) & 3);
-  const uint2 a = *reinterpret_cast<const uint2*>(&tt[row * BF_TS + 32 * j + 4 * sw]);
-  const uint2 b = *reinterpret_cast<const uint2*>(&tt[row * BF_TS + 32 * j + 16 + 4 * sw]);
-  return u32x4_t{a.x, a.y, b.x, b.y};
 }
 
 __device__ __forceinline__ uint32_t bf_cvt2(float a, float b) {
@@ -737,21 +793,23 @@ __device__ __forceinline__ void bf_split8(const f32x4_t& a, const f32x4_t& b, u3
   }
 }
 
-// dQ and the row statistics (as sab_q_kernel) with K, V as bf16 tiles, K also
-// transposed for dQ^T = K^T dS^T.
-template <int HD>
-__global__ __launch_bounds__(AB_THREADS, 2) void sab_q_bf_kernel(AbParams P) {
-  constexpr int DG = HD / 16, KS32 = HD / 32, RS = HD + 8;
-  __shared__ __attribute__((aligned(16))) bf16_t Kr[AB_T * RS], Vr[AB_T * RS], Kt[HD * BF_TS];
-  __shared__ int lt_idx[AB_THREADS], lt_cls[AB_THREADS], wcount[AB_THREADS / 64];
-  const int ntiles = (P.T + AB_T - 1) / AB_T;
-  const int t0 = (ntiles - 1 - static_cast<int>(blockIdx.x / P.Hq)) * AB_T;
-  const int b = blockIdx.y, h = blockIdx.x % P.Hq;
-  const int g = h / (P.Hq / P.Hkv);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// dQ and the row statistics (as sab_q_kernel).  A workgroup is HP query heads of one KV head
+// (they share the K / V tiles and the block lists) at 64 queries; wave (head, half) owns 32
+// of them.  Consecutive workgroups are consecutive KV heads (one XCD each when there are
+// eight), the latest query tiles first.
+template <int HD, int HP, int MIX>
+__global__ __launch_bounds__(128 * HP, 2) void sab_q_bf_kernel(AbParams P) {
+  constexpr int DG = HD / 16, KS32 = HD / 32, NT = 128 * HP, TB = sab_tile_bytes<HD>();
+  // one array: separate ones get alias scopes, and every LDS read would then wait for the
+  // direct loads in flight
+  __shared__ __attribute__((aligned(1024))) char smem[4 * TB];  // [stage][K, V]
+  const int ntiles = (P.T + AB_T - 1) / AB_T, nhp = P.Hq / HP;
+  const int t0 = (ntiles - 1 - static_cast<int>(blockIdx.x) / nhp) * AB_T;
+  const int hp = static_cast<int>(blockIdx.x) % nhp, g = hp % P.Hkv;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int b = blockIdx.y, h = g * (P.Hq / P.Hkv) + hp / P.Hkv * HP + (wave >> 1);
   const int r = lane & 15, kg = lane >> 4;
-  const int tq = t0 + 16 * wave + r;
-  const int tql = tq < P.T ? tq : P.T - 1;
+  const int tw = t0 + 32 * (wave & 1);  // this wave's queries tw + 16 i + r
   const bf16_t* q = static_cast<const bf16_t*>(P.q) + b * P.qs_b + h * P.qs_h;
   const bf16_t* o = static_cast<const bf16_t*>(P.o) + b * P.os_b + h * P.os_h;
   const bf16_t* dout = static_cast<const bf16_t*>(P.dout) + b * P.ds_b + h * P.ds_h;
@@ -759,262 +817,319 @@ __global__ __launch_bounds__(AB_THREADS, 2) void sab_q_bf_kernel(AbParams P) {
   const bf16_t* v = static_cast<const bf16_t*>(P.v) + b * P.vs_b + g * P.vs_h;
   const int32_t* map_b = P.map + static_cast<int64_t>(b) * P.nb * P.nb;
 
-  u32x4_t qb[KS32], db[KS32];
-  sab_row_frag_bf<bf16_t, HD>(q, P.qs_t, tql, P.hd, kg, qb);
-  sab_row_frag_bf<bf16_t, HD>(dout, P.ds_t, tql, P.hd, kg, db);
-  float dd;  // D = dout . out of query r
-  {
+  u32x4_t qb[2][KS32], db[2][KS32];
+  float dd[2];  // D = dout . out of query tw + 16 i + r
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int tq = tw + 16 * i + r, tql = tq < P.T ? tq : P.T - 1;
+    sab_row_frag_bf<bf16_t, HD>(q, P.qs_t, tql, HD, kg, qb[i]);
+    sab_row_frag_bf<bf16_t, HD>(dout, P.ds_t, tql, HD, kg, db[i]);
     f32x4_t of[DG], df[DG];
-    sab_row_frag<bf16_t, HD>(o, P.os_t, tql, P.hd, kg, of);
-    sab_row_frag<bf16_t, HD>(dout, P.ds_t, tql, P.hd, kg, df);
+    sab_row_frag<bf16_t, HD>(o, P.os_t, tql, HD, kg, of);
+    sab_row_frag<bf16_t, HD>(dout, P.ds_t, tql, HD, kg, df);
     float part = 0.f;
 #pragma unroll
     for (int d = 0; d < DG; ++d)
 #pragma unroll
       for (int kk = 0; kk < 4; ++kk) part = fmaf(df[d][kk], of[d][kk], part);
-    dd = sum_rows4(part);
+    dd[i] = sum_rows4(part);
   }
-  auto scores = [&](f32x4_t (&st)[4], const bf16_t* Xr, const u32x4_t (&bb)[KS32]) {
+  const uint32_t row_off = sab_row_off<HD>(r, kg), tr_off = sab_tr_off<HD>(r, kg);
+  // S^T (dP^T) of 32 keys of a tile against this wave's queries
+  auto scores = [&](f32x4_t (&st)[2][2], uint32_t off, const u32x4_t (&bb)[2][KS32]) {
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      st[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < 2; ++t) {
+      st[0][t] = st[1][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int ks = 0; ks < KS32; ++ks) st[t] = mfma16x16x32(bf_row<HD>(Xr, 16 * t + r, ks, kg), bb[ks], st[t]);
+      for (int ks = 0; ks < KS32; ++ks) {
+        const u32x4_t a = sab_row(smem, off, ks, 16 * t * HD * 2);
+        st[0][t] = mfma16x16x32(a, bb[0][ks], st[0][t]);
+        st[1][t] = mfma16x16x32(a, bb[1][ks], st[1][t]);
+      }
     }
   };
 
-  // pass 1: row maximum and sum (log2 units) over the live key tiles (listed 256
-  // at a time; the next tile's K rows load while this one's scores run)
+  // pass 1: row maximum and sum (log2 units) over the live key tiles
   const float sl2 = P.scale * 1.4426950408889634f;
-  float m = -INFINITY, lpart = 0.f;
-  uint2 xk[bf_rounds<HD>()][4], xv[bf_rounds<HD>()][4];
-  for (int c0 = 0; c0 < ntiles; c0 += AB_THREADS) {
-   const int n = sab_live_chunk<true>(P, map_b, t0, c0, ntiles, lt_idx, lt_cls, wcount);
-   if (n > 0) bf_load<HD>(k, P.ks_t, lt_idx[0] * AB_T, P.T, xk);
-   for (int li = 0; li < n; ++li) {
-    const int s0 = __builtin_amdgcn_readfirstlane(lt_idx[li]) * AB_T;
-    const int tcls = __builtin_amdgcn_readfirstlane(lt_cls[li]);
-    bf_store<HD, false>(xk, Kr, nullptr);
+  float m[2] = {-INFINITY, -INFINITY}, lpart[2] = {0.f, 0.f};
+  {
+    SabTiles<true> it(P, map_b, t0, ntiles);
+    bool more = it.next();
+    if (more) sab_dma<HD, NT>(k, P.ks_t, it.tile * AB_T, P.T, smem);
+    int stage = 0;
     __syncthreads();
-    if (li + 1 < n) bf_load<HD>(k, P.ks_t, lt_idx[li + 1] * AB_T, P.T, xk);
-    f32x4_t st[4];
-    scores(st, Kr, qb);
-    sab_logits2(P, map_b, tq, kg, t0, s0, tcls, sl2, st);
-    float cm = -INFINITY;
+    while (more) {
+      const int s0 = it.tile * AB_T, tcls = it.cls;
+      const uint32_t ko = row_off + stage * 2 * TB;
+      stage ^= 1;
+      more = it.next();
+      if (more) sab_dma<HD, NT>(k, P.ks_t, it.tile * AB_T, P.T, smem + stage * 2 * TB);
+      const bool inner = t0 + AB_T <= P.T && s0 + AB_T <= P.T;
+      f32x4_t st[2][4];
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+      for (int j = 0; j < 2; ++j) {
+        f32x4_t x[2][2];
+        scores(x, ko + 32 * j * HD * 2, qb);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) cm = fmaxf(cm, st[t][e]);
-    cm = max_rows4(cm);
-    if (cm > -INFINITY) {
-      const float mn = fmaxf(m, cm);
-      float add = 0.f;
+        for (int i = 0; i < 2; ++i) {
+          st[i][2 * j] = x[i][0];
+          st[i][2 * j + 1] = x[i][1];
+        }
+      }
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+      for (int i = 0; i < 2; ++i) {
+        sab_logits2<4, MIX>(P, map_b, tw + 16 * i, r, kg, s0, tcls, inner, sl2, st[i]);
+        float cm = -INFINITY;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) add += __builtin_amdgcn_exp2f(st[t][e] - mn);
-      lpart = (m > -INFINITY ? lpart * __builtin_amdgcn_exp2f(m - mn) : 0.f) + add;
-      m = mn;
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) cm = fmaxf(cm, st[i][t][e]);
+        cm = max_rows4(cm);
+        if (cm > -INFINITY) {
+          const float mn = fmaxf(m[i], cm);
+          float add = 0.f;
+#pragma unroll
+          for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) add += __builtin_amdgcn_exp2f(st[i][t][e] - mn);
+          lpart[i] = (m[i] > -INFINITY ? lpart[i] * __builtin_amdgcn_exp2f(m[i] - mn) : 0.f) + add;
+          m[i] = mn;
+        }
+      }
+      __syncthreads();
     }
-    __syncthreads();
-   }
   }
-  const float l = sum_rows4(lpart);
-  // log2 of the row's softmax denominator: P = exp2(x2 - lse2); +inf for a row
-  // with no key (every P 0, no NaN)
-  const float lse2 = l > 0.f ? m + __log2f(l) : INFINITY;
+  // log2 of the row's softmax denominator: P = exp2(x2 - lse2); +inf for a row with no key
+  // or past T (every P 0, no NaN)
+  float lse2[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const float l = sum_rows4(lpart[i]);
+    lse2[i] = l > 0.f && tw + 16 * i + r < P.T ? m[i] + __log2f(l) : INFINITY;
+  }
 
   // pass 2: dQ^T[dim][query] = sum_key K^T[dim][key] dS^T[key][query]
-  f32x4_t dqa[DG];
+  f32x4_t dqa[2][DG];
 #pragma unroll
-  for (int dt = 0; dt < DG; ++dt) dqa[dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  for (int c0 = 0; c0 < ntiles; c0 += AB_THREADS) {
-   const int n = sab_live_chunk<true>(P, map_b, t0, c0, ntiles, lt_idx, lt_cls, wcount);
-   if (n > 0) {
-     bf_load<HD>(k, P.ks_t, lt_idx[0] * AB_T, P.T, xk);
-     bf_load<HD>(v, P.vs_t, lt_idx[0] * AB_T, P.T, xv);
-   }
-   for (int li = 0; li < n; ++li) {
-    const int s0 = __builtin_amdgcn_readfirstlane(lt_idx[li]) * AB_T;
-    const int tcls = __builtin_amdgcn_readfirstlane(lt_cls[li]);
-    bf_store<HD, true>(xk, Kr, Kt);
-    bf_store<HD, false>(xv, Vr, nullptr);
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int dt = 0; dt < DG; ++dt) dqa[i][dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  {
+    SabTiles<true> it(P, map_b, t0, ntiles);
+    auto load = [&](int stage) {
+      sab_dma<HD, NT>(k, P.ks_t, it.tile * AB_T, P.T, smem + stage * 2 * TB);
+      sab_dma<HD, NT>(v, P.vs_t, it.tile * AB_T, P.T, smem + stage * 2 * TB + TB);
+    };
+    bool more = it.next();
+    if (more) load(0);
+    int stage = 0;
     __syncthreads();
-    if (li + 1 < n) {
-      bf_load<HD>(k, P.ks_t, lt_idx[li + 1] * AB_T, P.T, xk);
-      bf_load<HD>(v, P.vs_t, lt_idx[li + 1] * AB_T, P.T, xv);
-    }
-    f32x4_t st[4], dp[4];
-    scores(st, Kr, qb);
-    scores(dp, Vr, db);  // dP^T = V dout^T
-    sab_logits2(P, map_b, tq, kg, t0, s0, tcls, sl2, st);
+    while (more) {
+      const int s0 = it.tile * AB_T, tcls = it.cls;
+      const int cur = stage * 2 * TB;
+      stage ^= 1;
+      more = it.next();
+      if (more) load(stage);
+      const bool inner = t0 + AB_T <= P.T && s0 + AB_T <= P.T;
+#pragma unroll 1
+      for (int j = 0; j < 2; ++j) {  // 32 keys at a time (not unrolled: register budget)
+        f32x4_t st[2][2], dp[2][2];
+        const uint32_t at = cur + 32 * j * HD * 2;
+        scores(st, row_off + at, qb);
+        scores(dp, row_off + at + TB, db);  // dP^T = V dout^T
+        u32x4_t hi[2], lo[2];
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+        for (int i = 0; i < 2; ++i) {
+          sab_logits2<2, MIX>(P, map_b, tw + 16 * i, r, kg, s0 + 32 * j, tcls, inner, sl2, st[i]);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float p = __builtin_amdgcn_exp2f(st[t][e] - lse2);
-        st[t][e] = p * (dp[t][e] - dd);  // dS^T
+          for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              st[i][t][e] = __builtin_amdgcn_exp2f(st[i][t][e] - lse2[i]) * (dp[i][t][e] - dd[i]);  // dS^T
+          bf_split8(st[i][0], st[i][1], hi[i], lo[i]);
+        }
+#pragma unroll
+        for (int dt = 0; dt < DG; ++dt) {
+          const u32x4_t a = sab_trow<HD>(smem, tr_off + at, dt, 0);
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            dqa[i][dt] = mfma16x16x32(a, hi[i], dqa[i][dt]);
+            dqa[i][dt] = mfma16x16x32(a, lo[i], dqa[i][dt]);
+          }
+        }
       }
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      u32x4_t hi, lo;
-      bf_split8(st[2 * j], st[2 * j + 1], hi, lo);
-#pragma unroll
-      for (int dt = 0; dt < DG; ++dt) {
-        const u32x4_t a = bf_trow(Kt, 16 * dt + r, j, kg);
-        dqa[dt] = mfma16x16x32(a, hi, dqa[dt]);
-        dqa[dt] = mfma16x16x32(a, lo, dqa[dt]);
-      }
+      __syncthreads();
     }
-    __syncthreads();
-   }
   }
-  const int64_t rowbase = (static_cast<int64_t>(b) * P.Hq + h) * P.T;
-  if (tq < P.T) {
+  const int64_t row0 = static_cast<int64_t>(b) * P.Hq + h;
 #pragma unroll
-    for (int dt = 0; dt < DG; ++dt)
+  for (int i = 0; i < 2; ++i) {
+    const int tq = tw + 16 * i + r;
+    if (tq < P.T) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) P.dq[(rowbase + tq) * P.hd + 16 * dt + 4 * kg + e] = dqa[dt][e] * P.scale;
-    if (kg == 0) {
-      P.stat_m[rowbase + tq] = lse2;  // the bf16 kernels keep log2 units
-      P.stat_l[rowbase + tq] = l;
-      P.stat_d[rowbase + tq] = dd;
+      for (int dt = 0; dt < DG; ++dt)
+        *reinterpret_cast<f32x4_t*>(&P.dq[(row0 * P.T + tq) * HD + 16 * dt + 4 * kg]) = dqa[i][dt] * P.scale;
+    }
+    if (kg == 0) {  // statistics of whole tiles: rows past T get P = 0
+      P.stat_m[row0 * P.tp + tq] = lse2[i];
+      P.stat_d[row0 * P.tp + tq] = dd[i];
     }
   }
 }
 
-// dK and dV (as sab_kv_kernel) with Q and dout as bf16 tiles, both also
-// transposed for dK^T = Q^T dS and dV^T = dout^T P.
-template <int HD>
+// dK and dV (as sab_kv_kernel): wave (query half, key half) owns 32 keys and, of every
+// query tile, 32 queries; the two query halves' sums meet in LDS at the end.
+template <int HD, int MIX>
 __global__ __launch_bounds__(AB_THREADS, 2) void sab_kv_bf_kernel(AbParams P) {
-  constexpr int DG = HD / 16, KS32 = HD / 32, RS = HD + 8;
-  __shared__ __attribute__((aligned(16))) bf16_t Qr[AB_T * RS], Dr[AB_T * RS], Qt[HD * BF_TS], Dt[HD * BF_TS];
-  __shared__ float row_lse[AB_T], row_d[AB_T];  // log2 softmax denominators (+inf past T), D
-  __shared__ int lt_idx[AB_THREADS], lt_cls[AB_THREADS], wcount[AB_THREADS / 64];
+  constexpr int DG = HD / 16, KS32 = HD / 32, TB = sab_tile_bytes<HD>();
+  constexpr int STAGE = 2 * TB + 2 * AB_T * 4;  // Q, dout, then lse2 and D of the rows
+  constexpr int SUMS = 2 * 2 * 2 * DG * 64 * 16;  // two waves' dK and dV accumulators
+  __shared__ __attribute__((aligned(1024))) char smem[2 * STAGE > SUMS ? 2 * STAGE : SUMS];
   const int ntiles = (P.T + AB_T - 1) / AB_T;
   const int s0 = static_cast<int>(blockIdx.x / P.Hkv) * AB_T;
   const float sl2 = P.scale * 1.4426950408889634f;
   const int b = blockIdx.y, g = blockIdx.x % P.Hkv;
   const int G = P.Hq / P.Hkv;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, kg = lane >> 4;
-  const int sk = s0 + 16 * wave + r;
-  const int skl = sk < P.T ? sk : P.T - 1;
+  const int wq = wave >> 1, sw = s0 + 32 * (wave & 1);  // this wave's keys sw + 16 kt + r
   const bf16_t* k = static_cast<const bf16_t*>(P.k) + b * P.ks_b + g * P.ks_h;
   const bf16_t* v = static_cast<const bf16_t*>(P.v) + b * P.vs_b + g * P.vs_h;
   const int32_t* map_b = P.map + static_cast<int64_t>(b) * P.nb * P.nb;
-  u32x4_t kb[KS32], vb[KS32];
-  sab_row_frag_bf<bf16_t, HD>(k, P.ks_t, skl, P.hd, kg, kb);
-  sab_row_frag_bf<bf16_t, HD>(v, P.vs_t, skl, P.hd, kg, vb);
-  f32x4_t dka[DG], dva[DG];
+  u32x4_t kb[2][KS32], vb[2][KS32];
+  f32x4_t dka[2][DG], dva[2][DG];
 #pragma unroll
-  for (int dt = 0; dt < DG; ++dt) dka[dt] = dva[dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int kt = 0; kt < 2; ++kt) {
+    const int sk = sw + 16 * kt + r, skl = sk < P.T ? sk : P.T - 1;
+    sab_row_frag_bf<bf16_t, HD>(k, P.ks_t, skl, HD, kg, kb[kt]);
+    sab_row_frag_bf<bf16_t, HD>(v, P.vs_t, skl, HD, kg, vb[kt]);
+#pragma unroll
+    for (int dt = 0; dt < DG; ++dt) dka[kt][dt] = dva[kt][dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
 
-  // (live query tile, query head of the group) pairs, the tiles listed 256 at a
-  // time; the next pair's Q and dout rows and row statistics load while this
-  // pair's products run
-  uint2 xq[bf_rounds<HD>()][4], xd[bf_rounds<HD>()][4];
-  float nlse = INFINITY, nd = 0.f;
-  auto load_pair = [&](int li, int hh) {
-    const int t0 = __builtin_amdgcn_readfirstlane(lt_idx[li]) * AB_T, h = g * G + hh;
-    bf_load<HD>(static_cast<const bf16_t*>(P.q) + b * P.qs_b + h * P.qs_h, P.qs_t, t0, P.T, xq);
-    bf_load<HD>(static_cast<const bf16_t*>(P.dout) + b * P.ds_b + h * P.ds_h, P.ds_t, t0, P.T, xd);
-    const int64_t rowbase = (static_cast<int64_t>(b) * P.Hq + h) * P.T;
-    const int t = t0 + tid;
-    if (tid < AB_T && t < P.T) {
-      nlse = P.stat_m[rowbase + t];
-      nd = P.stat_d[rowbase + t];
-    } else {
-      nlse = INFINITY;
-      nd = 0.f;
+  const uint32_t row_off = sab_row_off<HD>(r, kg) + 32 * wq * HD * 2;
+  const uint32_t tr_off = sab_tr_off<HD>(r, kg) + 32 * wq * HD * 2;
+  // (live query tile, query head of the group) pairs
+  SabTiles<false> it(P, map_b, s0, ntiles);
+  int hh = G - 1;
+  auto next = [&]() {
+    if (++hh < G) return true;
+    hh = 0;
+    return it.next();
+  };
+  auto load = [&](int stage) {
+    char* S = smem + stage * STAGE;
+    const int h = g * G + hh, t0 = it.tile * AB_T;
+    sab_dma<HD, AB_THREADS>(static_cast<const bf16_t*>(P.q) + b * P.qs_b + h * P.qs_h, P.qs_t, t0, P.T, S);
+    sab_dma<HD, AB_THREADS>(static_cast<const bf16_t*>(P.dout) + b * P.ds_b + h * P.ds_h, P.ds_t, t0, P.T, S + TB);
+    if (wave < 2) {  // the statistics cover whole tiles
+      const float* st = (wave ? P.stat_d : P.stat_m) + (static_cast<int64_t>(b) * P.Hq + h) * P.tp + t0 + lane;
+      __builtin_amdgcn_global_load_lds((ab_glb_t*)st, (ab_lds_t*)(S + 2 * TB + wave * AB_T * 4), 4, 0, 0);
     }
   };
-  for (int c0 = 0; c0 < ntiles; c0 += AB_THREADS) {
-   const int n = sab_live_chunk<false>(P, map_b, s0, c0, ntiles, lt_idx, lt_cls, wcount);
-   if (n > 0) load_pair(0, 0);
-   for (int it = 0; it < n * G; ++it) {
-    const int li = it / G;
-    const int t0 = __builtin_amdgcn_readfirstlane(lt_idx[li]) * AB_T;
-    const int tcls = __builtin_amdgcn_readfirstlane(lt_cls[li]);
-    // one weight for the whole tile (all: log2 weight lw2; inner: every query and
-    // key inside T), the window only (win), or per element
-    const bool all = tcls > 0 && (P.mode == FSI_SATTN_BLOCK_LIST || (tcls & 2));
-    const bool win = tcls > 0 && !all;
+  bool more = next();
+  if (more) load(0);
+  int stage = 0;
+  __syncthreads();
+  while (more) {
+    const int t0 = it.tile * AB_T, tcls = it.cls;
     const bool inner = t0 + AB_T <= P.T && s0 + AB_T <= P.T;
-    const float lw2 = all && P.mode == FSI_SATTN_BLOCK_LIST ? __log2f(static_cast<float>(tcls)) : 0.f;
-    {
-      bf_store<HD, true>(xq, Qr, Qt);
-      bf_store<HD, true>(xd, Dr, Dt);
-      if (tid < AB_T) {
-        row_lse[tid] = nlse;
-        row_d[tid] = nd;
-      }
-      __syncthreads();
-      if (it + 1 < n * G) load_pair((it + 1) / G, (it + 1) % G);
-      // two 16-query sub-tiles at a time (not unrolled: the operand reads of all
-      // four would be hoisted past the register budget)
-#pragma unroll 1
-      for (int j = 0; j < 2; ++j) {
-        f32x4_t pp[2], ds[2];  // P, dS [query 32 j + 16 i + 4 kg + e][key r]
+    const SabWeight wt = sab_weight_of(P, tcls);
+    const int cur = stage * STAGE;
+    stage ^= 1;
+    more = next();
+    if (more) load(stage);
+    f32x4_t s[2][2], dp[2][2];  // [key half][16-query part]: query 32 wq + 16 i + 4 kg + e, key r
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const int qt = 2 * j + i;
-          f32x4_t s = f32x4_t{0.f, 0.f, 0.f, 0.f}, dp = s;
+    for (int i = 0; i < 2; ++i) {
+      s[0][i] = s[1][i] = dp[0][i] = dp[1][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int ks = 0; ks < KS32; ++ks) {
-            s = mfma16x16x32(bf_row<HD>(Qr, 16 * qt + r, ks, kg), kb[ks], s);
-            dp = mfma16x16x32(bf_row<HD>(Dr, 16 * qt + r, ks, kg), vb[ks], dp);
-          }
+      for (int ks = 0; ks < KS32; ++ks) {
+        const u32x4_t aq = sab_row(smem, row_off + cur, ks, 16 * i * HD * 2);
+        const u32x4_t ad = sab_row(smem, row_off + cur, ks, 16 * i * HD * 2 + TB);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int rq = 16 * qt + 4 * kg + e, t = t0 + rq;
-            const float lse = row_lse[rq];  // +inf past T: P = 0
-            float p;
-            if (all) {
-              p = __builtin_amdgcn_exp2f(fmaf(s[e], sl2, lw2 - lse));
-              if (!inner) p = sk < P.T ? p : 0.f;
-            } else if (win) {
-              const float x = __builtin_amdgcn_exp2f(fmaf(s[e], sl2, -lse));
-              p = sk <= t && sk > t - P.window ? x : 0.f;
-            } else {
-              p = 0.f;
-              if (t < P.T && sk < P.T) {
-                const float w = sab_tile_weight(P, map_b, tcls, t, sk);
-                if (w > 0.f) p = __builtin_amdgcn_exp2f(fmaf(s[e], sl2, __log2f(w) - lse));
-              }
-            }
-            pp[i][e] = p;
-            ds[i][e] = p * (dp[e] - row_d[rq]);
-          }
-        }
-        // dV^T[dim][key] += dout^T[dim][query] P[query][key], dK^T += Q^T dS
-        u32x4_t ph, pl, dh, dl;
-        bf_split8(pp[0], pp[1], ph, pl);
-        bf_split8(ds[0], ds[1], dh, dl);
-#pragma unroll
-        for (int dt = 0; dt < DG; ++dt) {
-          const u32x4_t ad = bf_trow(Dt, 16 * dt + r, j, kg);
-          const u32x4_t aq = bf_trow(Qt, 16 * dt + r, j, kg);
-          dva[dt] = mfma16x16x32(ad, ph, dva[dt]);
-          dva[dt] = mfma16x16x32(ad, pl, dva[dt]);
-          dka[dt] = mfma16x16x32(aq, dh, dka[dt]);
-          dka[dt] = mfma16x16x32(aq, dl, dka[dt]);
+        for (int kt = 0; kt < 2; ++kt) {
+          s[kt][i] = mfma16x16x32(aq, kb[kt][ks], s[kt][i]);
+          dp[kt][i] = mfma16x16x32(ad, vb[kt][ks], dp[kt][i]);
         }
       }
-      __syncthreads();
     }
-   }
-  }
-  const int64_t kbase = (static_cast<int64_t>(b) * P.Hkv + g) * P.T;
-  if (sk < P.T) {
+    __builtin_amdgcn_sched_barrier(0);  // register budget: keep the phases apart
 #pragma unroll
-    for (int dt = 0; dt < DG; ++dt)
+    for (int i = 0; i < 2; ++i) {
+      const int rq = 32 * wq + 16 * i + 4 * kg;
+      const float* rows = reinterpret_cast<const float*>(smem + cur + 2 * TB) + rq;
+      const f32x4_t lse = *reinterpret_cast<const f32x4_t*>(rows);  // +inf past T: P = 0
+      const f32x4_t rd = *reinterpret_cast<const f32x4_t*>(rows + AB_T);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int d = 16 * dt + 4 * kg + e;
-        P.dk[(kbase + sk) * P.hd + d] = dka[dt][e] * P.scale;
-        P.dv[(kbase + sk) * P.hd + d] = dva[dt][e];
+      for (int kt = 0; kt < 2; ++kt) {
+        const int sk0 = sw + 16 * kt, sk = sk0 + r, t = t0 + rq;
+        SabWeight w = wt;
+        if (MIX == SAB_SUB && tcls < 0)
+          w = sab_weight_of(P, sab_sub_class(P, map_b, t0 + 32 * wq + 16 * i, sk0));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float p;
+          if (MIX == SAB_ELEM && tcls < 0) {
+            p = 0.f;
+            if (t + e < P.T && sk < P.T) {
+              const float we = sab_tile_weight(P, map_b, tcls, t + e, sk);
+              if (we > 0.f) p = __builtin_amdgcn_exp2f(fmaf(s[kt][i][e], sl2, __log2f(we) - lse[e]));
+            }
+          } else {
+            p = sab_p(P, w, t + e, sk, inner, sl2, lse[e], s[kt][i][e]);
+          }
+          s[kt][i][e] = p;
+          dp[kt][i][e] = p * (dp[kt][i][e] - rd[e]);  // dS
+        }
       }
+    }
+    __builtin_amdgcn_sched_barrier(0);  // register budget: keep the phases apart
+    // dV^T[dim][key] += dout^T[dim][query] P[query][key], dK^T += Q^T dS
+    u32x4_t ph[2], pl[2], dh[2], dl[2];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+      bf_split8(s[kt][0], s[kt][1], ph[kt], pl[kt]);
+      bf_split8(dp[kt][0], dp[kt][1], dh[kt], dl[kt]);
+    }
+#pragma unroll
+    for (int dt = 0; dt < DG; ++dt) {
+      const u32x4_t ad = sab_trow<HD>(smem, tr_off + cur, dt, TB);
+      const u32x4_t aq = sab_trow<HD>(smem, tr_off + cur, dt, 0);
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt) {
+        dva[kt][dt] = mfma16x16x32(ad, ph[kt], dva[kt][dt]);
+        dva[kt][dt] = mfma16x16x32(ad, pl[kt], dva[kt][dt]);
+        dka[kt][dt] = mfma16x16x32(aq, dh[kt], dka[kt][dt]);
+        dka[kt][dt] = mfma16x16x32(aq, dl[kt], dka[kt][dt]);
+      }
+    }
+    __syncthreads();
+  }
+  // the second query half hands its sums over, the first stores
+  f32x4_t* sums = reinterpret_cast<f32x4_t*>(smem) + (wave & 1) * (4 * DG * 64) + lane;
+  if (wq == 1) {
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int dt = 0; dt < DG; ++dt) {
+        sums[(2 * (kt * DG + dt)) * 64] = dka[kt][dt];
+        sums[(2 * (kt * DG + dt) + 1) * 64] = dva[kt][dt];
+      }
+  }
+  __syncthreads();
+  if (wq == 1) return;
+  const int64_t kbase = (static_cast<int64_t>(b) * P.Hkv + g) * P.T;
+#pragma unroll
+  for (int kt = 0; kt < 2; ++kt) {
+    const int sk = sw + 16 * kt + r;
+    if (sk >= P.T) continue;
+#pragma unroll
+    for (int dt = 0; dt < DG; ++dt) {
+      const int64_t at = (kbase + sk) * HD + 16 * dt + 4 * kg;
+      *reinterpret_cast<f32x4_t*>(&P.dk[at]) = (dka[kt][dt] + sums[(2 * (kt * DG + dt)) * 64]) * P.scale;
+      *reinterpret_cast<f32x4_t*>(&P.dv[at]) = dva[kt][dt] + sums[(2 * (kt * DG + dt) + 1) * 64];
+    }
   }
 }
 
@@ -1024,14 +1139,18 @@ size_t sab_map_bytes(int64_t B, int64_t T, int64_t block) {
   return fsi_host::align_up(sizeof(int32_t) * static_cast<size_t>(B * nb * nb), 256);
 }
 
+// One statistic of every query row, T rounded up to whole tiles.
+size_t sab_stat_bytes(int64_t B, int64_t Hq, int64_t T) {
+  return fsi_host::align_up(sizeof(float) * static_cast<size_t>(B * Hq * ((T + AB_T - 1) / AB_T * AB_T)), 256);
+}
+
 }  // namespace
 
 extern "C" {
 
 FSI_API size_t fsi_sparse_attn_bwd_workspace_size(int64_t B, int64_t Hq, int64_t T, int64_t block) {
   if (B <= 0 || Hq <= 0 || T <= 0 || block <= 0) return 0;
-  return FSI_WORKSPACE_COUNTER_BYTES + sab_map_bytes(B, T, block) +
-         3 * fsi_host::align_up(sizeof(float) * static_cast<size_t>(B * Hq * T), 256);
+  return FSI_WORKSPACE_COUNTER_BYTES + sab_map_bytes(B, T, block) + 3 * sab_stat_bytes(B, Hq, T);
 }
 
 FSI_API int fsi_sparse_attn_bwd(const void* q, int64_t qs_b, int64_t qs_h, int64_t qs_t, const void* k, int64_t ks_b,
@@ -1114,7 +1233,8 @@ FSI_API int fsi_sparse_attn_bwd(const void* q, int64_t qs_b, int64_t qs_h, int64
   }
   char* ws = static_cast<char*>(workspace) + FSI_WORKSPACE_COUNTER_BYTES;
   P.map = reinterpret_cast<int32_t*>(ws);
-  const size_t st_bytes = align_up(sizeof(float) * static_cast<size_t>(B * Hq * T), 256);
+  P.tp = (T + AB_T - 1) / AB_T * AB_T;
+  const size_t st_bytes = sab_stat_bytes(B, Hq, T);
   P.stat_m = reinterpret_cast<float*>(ws + sab_map_bytes(B, T, block));
   P.stat_l = reinterpret_cast<float*>(ws + sab_map_bytes(B, T, block) + st_bytes);
   P.stat_d = reinterpret_cast<float*>(ws + sab_map_bytes(B, T, block) + 2 * st_bytes);
@@ -1134,12 +1254,25 @@ FSI_API int fsi_sparse_attn_bwd(const void* q, int64_t qs_b, int64_t qs_h, int64
       sab_kv_kernel<float, HD><<<gkv, AB_THREADS, 0, st>>>(P);
     } else {
       if constexpr (HD >= 32) {
-        // the bf16 kernels address a tile's rows with 32-bit offsets: row strides below 2^24
-        const bool short_rows = qs_t < (int64_t(1) << 24) && ks_t < (int64_t(1) << 24) &&
-                                vs_t < (int64_t(1) << 24) && ds_t < (int64_t(1) << 24);
-        if (head_dim == HD && P.vec4 && short_rows) {
-          sab_q_bf_kernel<HD><<<gq, AB_THREADS, 0, st>>>(P);
-          sab_kv_bf_kernel<HD><<<gkv, AB_THREADS, 0, st>>>(P);
+        // the bf16 kernels move 16-byte pieces and address a tile's rows with 32-bit
+        // offsets: rows 8-element aligned, row strides below 2^24
+        auto al8 = [&](const void* p, int64_t sb, int64_t sh, int64_t stt) {
+          return reinterpret_cast<uintptr_t>(p) % 16 == 0 && sb % 8 == 0 && sh % 8 == 0 && stt % 8 == 0 &&
+                 stt >= 0 && stt < (int64_t(1) << 24);
+        };
+        const bool out16 = reinterpret_cast<uintptr_t>(dq) % 16 == 0 && reinterpret_cast<uintptr_t>(dk) % 16 == 0 &&
+                           reinterpret_cast<uintptr_t>(dv) % 16 == 0;
+        if (head_dim == HD && out16 && al8(q, qs_b, qs_h, qs_t) && al8(k, ks_b, ks_h, ks_t) &&
+            al8(v, vs_b, vs_h, vs_t) && al8(dout, ds_b, ds_h, ds_t)) {
+          auto launch = [&](auto mix_tag) {
+            constexpr int MIX = decltype(mix_tag)::value;
+            if ((Hq / Hkv) % 2 == 0) sab_q_bf_kernel<HD, 2, MIX><<<dim3(gq.x / 2, gq.y), 256, 0, st>>>(P);
+            else sab_q_bf_kernel<HD, 1, MIX><<<gq, 128, 0, st>>>(P);
+            sab_kv_bf_kernel<HD, MIX><<<gkv, AB_THREADS, 0, st>>>(P);
+          };
+          if (block % AB_T == 0) launch(sab_mix_t<SAB_TILE>{});
+          else if (block % 16 == 0) launch(sab_mix_t<SAB_SUB>{});
+          else launch(sab_mix_t<SAB_ELEM>{});
           return;
         }
       }
