@@ -199,6 +199,28 @@ SIGNATURES: dict[str, tuple] = {
         [_c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int,
          _c_ptr, _c_i64, _c_ptr, _c_size, _c_ptr],
     ),
+    "fsi_mlp_train_route_workspace_size": (_c_size, [_c_i64, _c_i64, _c_int]),
+    "fsi_mlp_train_route": (
+        _c_int,
+        [_c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, ctypes.c_float, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
+         _c_size, _c_ptr],
+    ),
+    "fsi_mlp_train_route_bwd": (
+        _c_int,
+        [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, ctypes.c_float, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_size,
+         _c_ptr],
+    ),
+    "fsi_mlp_train_gather": (
+        _c_int,
+        [_c_ptr, _c_ptr, _c_i64, _c_ptr, _c_i64, _c_int, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_ptr,
+         _c_ptr, _c_ptr],
+    ),
+    "fsi_mlp_train_scatter": (
+        _c_int,
+        [_c_ptr, _c_ptr, _c_int, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr],
+    ),
+    "fsi_swiglu_pair": (_c_int, [_c_ptr, _c_i64, _c_i64, _c_int, _c_ptr, _c_ptr]),
+    "fsi_swiglu_pair_bwd": (_c_int, [_c_ptr, _c_ptr, _c_i64, _c_i64, _c_int, _c_ptr, _c_ptr]),
     "fsi_blockwise_matmul_bwd_workspace_size": (_c_size, [_c_i64] * 5 + [_c_int] * 3),
     "fsi_blockwise_matmul_bwd": (
         _c_int,

@@ -30,6 +30,7 @@ from .pattention import (
     PACKED_PREFILL_MIN_M,
     PackedPattentionWeights,
     dense_block_targets,
+    _aligned_rows,
     _weights_key,
     pack_pattention_weights,
     packed_decode_supported,
@@ -133,6 +134,241 @@ class _SavedGU:
 
     def __init__(self, g: Tensor, u: Tensor):
         self.saved_tensors = (g.contiguous(), u.contiguous())
+
+
+# -- training path on the HIP kernels of csrc/mlp_train.hip -----------------------------
+
+
+def _train_route_fake(q, keys, base, remote, temperature):
+    return (q.new_empty((q.shape[0], keys.shape[0])), torch.empty_like(q),
+            q.new_empty((base + remote,), dtype=torch.int32))
+
+
+@_lib.fsi_op("mlp_train_route", _train_route_fake)
+def _train_route_op(q: Tensor, keys: Tensor, base: int, remote: int,
+                    temperature: float) -> Tuple[Tensor, Tensor, Tensor]:
+    """fsi_mlp_train_route: (scores (M, n_blocks), context (M, 16), active blocks int32)."""
+    what = "FovealPattentionMLP training routing"
+    dev = _lib.require_gpu(q, keys, what=what)
+    q, keys = q.contiguous(), keys.contiguous()
+    M, nb = q.shape[0], keys.shape[0]
+    L = _lib.lib()
+    stream = _lib.stream_handle(dev)
+    scores = torch.empty((M, nb), dtype=q.dtype, device=dev)
+    ctx = torch.empty_like(q)
+    active = torch.empty(base + remote, dtype=torch.int32, device=dev)
+    ws = _lib.workspace(dev, L.fsi_mlp_train_route_workspace_size(M, nb, 0), stream)
+    st = L.fsi_mlp_train_route(q.data_ptr(), keys.data_ptr(), M, nb, base, remote, temperature,
+                               _lib.dtype_code(q.dtype, what), scores.data_ptr(), ctx.data_ptr(), active.data_ptr(),
+                               ws.data_ptr(), ws.numel(), stream)
+    _lib.check(st, what)
+    return scores, ctx, active
+
+
+@_lib.fsi_op("mlp_train_route_bwd", lambda q, keys, dscores, dctx, temperature: (torch.empty_like(q),
+                                                                               torch.empty_like(keys)))
+def _train_route_bwd_op(q: Tensor, keys: Tensor, dscores: Optional[Tensor], dctx: Optional[Tensor],
+                        temperature: float) -> Tuple[Tensor, Tensor]:
+    """fsi_mlp_train_route_bwd: (dq, dkeys)."""
+    what = "FovealPattentionMLP training routing backward"
+    dev = _lib.require_gpu(q, keys, what=what)
+    q, keys = q.contiguous(), keys.contiguous()
+    ds = dscores.to(q.dtype).contiguous() if dscores is not None else None
+    dc = dctx.to(q.dtype).contiguous() if dctx is not None else None
+    M, nb = q.shape[0], keys.shape[0]
+    L = _lib.lib()
+    stream = _lib.stream_handle(dev)
+    dq, dkeys = torch.empty_like(q), torch.empty_like(keys)
+    ws = _lib.workspace(dev, L.fsi_mlp_train_route_workspace_size(M, nb, 1), stream)
+    st = L.fsi_mlp_train_route_bwd(q.data_ptr(), keys.data_ptr(), _lib.ptr(ds), _lib.ptr(dc), M, nb, temperature,
+                                   _lib.dtype_code(q.dtype, what), dq.data_ptr(), dkeys.data_ptr(), ws.data_ptr(),
+                                   ws.numel(), stream)
+    _lib.check(st, what)
+    return dq, dkeys
+
+
+def _router_scores(q: Tensor, keys: Tensor) -> Tensor:
+    return torch.matmul(F.rms_norm(q, (q.shape[-1],)), keys.t()) / math.sqrt(q.shape[-1])
+
+
+class _TrainRouteFn(torch.autograd.Function):
+    """Router scores, 16-D context and active blocks from the projected queries
+    (foveal_pattention.py:257-262, 292-299, 338-341).  A backward that is itself
+    differentiated runs on torch ops."""
+
+    @staticmethod
+    def forward(ctx, q, keys, base, remote, temperature):
+        scores, context, active = _train_route_op(q, keys, base, remote, temperature)
+        ctx.save_for_backward(q, keys)
+        ctx.temperature = temperature
+        ctx.mark_non_differentiable(active)
+        ctx.set_materialize_grads(False)
+        return scores, context, active
+
+    @staticmethod
+    def backward(ctx, dscores, dcontext, _):
+        q, keys = ctx.saved_tensors
+        if dscores is None and dcontext is None:
+            return None, None, None, None, None
+        if torch.is_grad_enabled():
+            s = _router_scores(q, keys)
+            outs = [(s, dscores), (torch.matmul(F.softmax(s / ctx.temperature, dim=-1), keys), dcontext)]
+            outs = [o for o in outs if o[1] is not None]
+            wanted = [t for t, need in zip((q, keys), ctx.needs_input_grad) if need]
+            got = iter(torch.autograd.grad([o[0] for o in outs], wanted, [o[1] for o in outs], create_graph=True))
+            dq, dkeys = (next(got) if need else None for need in ctx.needs_input_grad[:2])
+        else:
+            dq, dkeys = _train_route_bwd_op(q, keys, dscores, dcontext, ctx.temperature)
+        return dq, dkeys, None, None, None
+
+
+def _v_transposed(v: Tensor) -> bool:
+    return v.stride(0) == 1 and v.stride(1) >= v.shape[0] and v.shape[1] > 1
+
+
+def _train_gather_fake(k_gate, k_up, v, active, block, v_t):
+    n, D = active.shape[0] * block, k_gate.shape[1]
+    return k_gate.new_empty((2 * n, D)), v.new_empty((D, n) if v_t else (n, D))
+
+
+@_lib.fsi_op("mlp_train_gather", _train_gather_fake)
+def _train_gather_op(k_gate: Tensor, k_up: Tensor, v: Tensor, active: Tensor, block: int,
+                     v_t: bool) -> Tuple[Tensor, Tensor]:
+    """fsi_mlp_train_gather: the active rows of [k_gate; k_up] and of v ((D, n) with v_t)."""
+    what = "FovealPattentionMLP training"
+    dev = _lib.require_gpu(k_gate, k_up, v, active, what=what)
+    kg, ku, vv = _aligned_rows(k_gate), _aligned_rows(k_up), _aligned_rows(v.t() if v_t else v)
+    if kg.stride(0) != ku.stride(0):
+        kg, ku = kg.contiguous(), ku.contiguous()
+    D, n = kg.shape[1], active.numel() * block
+    kgu = torch.empty((2 * n, D), dtype=kg.dtype, device=dev)
+    vs = torch.empty((D, n) if v_t else (n, D), dtype=kg.dtype, device=dev)
+    st = _lib.lib().fsi_mlp_train_gather(kg.data_ptr(), ku.data_ptr(), kg.stride(0), vv.data_ptr(), vv.stride(0),
+                                         int(v_t), active.data_ptr(), active.numel(), block, kg.shape[0] // block, D,
+                                         _lib.dtype_code(kg.dtype, what), kgu.data_ptr(), vs.data_ptr(),
+                                         _lib.stream_handle(dev))
+    _lib.check(st, what)
+    return kgu, vs
+
+
+def _train_scatter_fake(dkgu, dvs, active, block, n_blocks, D, v_t, gate, up, v):
+    like = dkgu if dkgu is not None else dvs
+    np_ = n_blocks * block
+    return (like.new_empty((np_, D) if gate else (0,)), like.new_empty((np_, D) if up else (0,)),
+            like.new_empty(((D, np_) if v_t else (np_, D)) if v else (0,)))
+
+
+@_lib.fsi_op("mlp_train_scatter", _train_scatter_fake)
+def _train_scatter_op(dkgu: Optional[Tensor], dvs: Optional[Tensor], active: Tensor, block: int, n_blocks: int, D: int,
+                      v_t: bool, gate: bool, up: bool, v: bool) -> Tuple[Tensor, Tensor, Tensor]:
+    """fsi_mlp_train_scatter: dense gradients of k_gate, k_up and v ((D, N_p) with v_t), each
+    empty unless wanted."""
+    what = "FovealPattentionMLP training backward"
+    like = dkgu if dkgu is not None else dvs
+    dev = like.device
+    np_ = n_blocks * block
+    dg, du, dv = (torch.empty(s if w else (0,), dtype=like.dtype, device=dev) for s, w in
+                  (((np_, D), gate), ((np_, D), up), ((D, np_) if v_t else (np_, D), v)))
+    dk = _aligned_rows(dkgu) if dkgu is not None else None
+    dvs = _aligned_rows(dvs) if dvs is not None else None
+    dk = dk.contiguous() if dk is not None else None
+    dvs = dvs.contiguous() if dvs is not None else None
+    st = _lib.lib().fsi_mlp_train_scatter(_lib.ptr(dk), _lib.ptr(dvs), int(v_t), active.data_ptr(), active.numel(),
+                                          block, n_blocks, D, _lib.dtype_code(like.dtype, what),
+                                          dg.data_ptr() if gate else None, du.data_ptr() if up else None,
+                                          dv.data_ptr() if v else None, _lib.stream_handle(dev))
+    _lib.check(st, what)
+    return dg, du, dv
+
+
+class _TrainGatherFn(torch.autograd.Function):
+    """The active blocks' rows of [k_gate; k_up] and v, as copies (foveal_pattention.py:115-122)."""
+
+    @staticmethod
+    def forward(ctx, k_gate, k_up, v, active, block):
+        v_t = _v_transposed(v)
+        kgu, vs = _train_gather_op(k_gate, k_up, v, active, block, v_t)
+        ctx.save_for_backward(active)
+        ctx.meta = (block, k_gate.shape[0] // block, k_gate.shape[1], v_t)
+        ctx.set_materialize_grads(False)
+        return kgu, vs
+
+    @staticmethod
+    def backward(ctx, dkgu, dvs):
+        (active,) = ctx.saved_tensors
+        block, n_blocks, D, v_t = ctx.meta
+        gate, up, v = ctx.needs_input_grad[:3]
+        gate, up, v = gate and dkgu is not None, up and dkgu is not None, v and dvs is not None
+        if not (gate or up or v):
+            return None, None, None, None, None
+        if torch.is_grad_enabled():
+            rows = (active.view(-1, 1).long() * block + torch.arange(block, device=active.device)).flatten()
+            full = lambda d: d.new_zeros((n_blocks * block, D)).index_add(0, rows, d)  # noqa: E731
+            n = rows.numel()
+            return (full(dkgu[:n]) if gate else None, full(dkgu[n:]) if up else None,
+                    full(dvs.t() if v_t else dvs) if v else None, None, None)
+        dg, du, dv = _train_scatter_op(dkgu, dvs, active, block, n_blocks, D, v_t, gate, up, v)
+        return dg if gate else None, du if up else None, (dv.t() if v_t else dv) if v else None, None, None
+
+
+@_lib.fsi_op("swiglu_pair", lambda gu: gu.new_empty((gu.shape[0], gu.shape[1] // 2)))
+def _swiglu_pair_op(gu: Tensor) -> Tensor:
+    """fsi_swiglu_pair: silu(g) * u of contiguous [g | u] rows."""
+    M, n = gu.shape[0], gu.shape[1] // 2
+    act = torch.empty((M, n), dtype=gu.dtype, device=gu.device)
+    st = _lib.lib().fsi_swiglu_pair(gu.data_ptr(), M, n, _lib.dtype_code(gu.dtype, "swiglu"), act.data_ptr(),
+                                    _lib.stream_handle(gu.device))
+    _lib.check(st, "swiglu")
+    return act
+
+
+@_lib.fsi_op("swiglu_pair_bwd", lambda dact, gu: torch.empty_like(gu))
+def _swiglu_pair_bwd_op(dact: Tensor, gu: Tensor) -> Tensor:
+    """fsi_swiglu_pair_bwd: [dg | du] rows."""
+    d = _aligned_rows(dact).contiguous()
+    dgu = torch.empty_like(gu)
+    st = _lib.lib().fsi_swiglu_pair_bwd(d.data_ptr(), gu.data_ptr(), gu.shape[0], gu.shape[1] // 2,
+                                        _lib.dtype_code(gu.dtype, "swiglu backward"), dgu.data_ptr(),
+                                        _lib.stream_handle(gu.device))
+    _lib.check(st, "swiglu backward")
+    return dgu
+
+
+class _TrainPattFn(torch.autograd.Function):
+    """y = (silu(x Kg^T) * (x Ku^T)) V over gathered rows [Kg; Ku] and V (foveal_pattention.py:
+    328-335): gate and up are one library GEMM, and so are their parts of dx and of the
+    weight gradients.  A backward that is itself differentiated runs on torch ops."""
+
+    @staticmethod
+    def forward(ctx, x, kgu, vs, v_t):
+        gu = torch.mm(x, kgu.t())
+        act = _swiglu_pair_op(gu)
+        ctx.save_for_backward(x, kgu, vs, gu, act)
+        ctx.v_t = v_t
+        return torch.mm(act, vs.t() if v_t else vs)
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, kgu, vs, gu, act = ctx.saved_tensors
+        v_t = ctx.v_t
+        need = ctx.needs_input_grad[:3]
+        if torch.is_grad_enabled():
+            n = kgu.shape[0] // 2
+            a = triton_fused_swiglu(F.linear(x, kgu[:n]), F.linear(x, kgu[n:]))
+            y = torch.mm(a, vs.t() if v_t else vs)
+            wanted = [t for t, w in zip((x, kgu, vs), need) if w]
+            got = iter(torch.autograd.grad(y, wanted, dy, create_graph=True))
+            return (*(next(got) if w else None for w in need), None)
+        dx = dkgu = dvs = None
+        if need[0] or need[1]:
+            dgu = _swiglu_pair_bwd_op(torch.mm(dy, vs if v_t else vs.t()), gu)
+            if need[0]:
+                dx = torch.mm(dgu, kgu)
+            if need[1]:
+                dkgu = torch.mm(dgu.t(), x)
+        if need[2]:
+            dvs = torch.mm(dy.t(), act) if v_t else torch.mm(act.t(), dy)
+        return dx, dkgu, dvs, None
 
 
 class FovealPattentionMLP(nn.Module):
@@ -479,6 +715,13 @@ class FovealPattentionMLP(nn.Module):
         reach k_gate, k_up, v (active rows), q_proj_16d, block_keys_16d and
         out_proj_16d as in the reference."""
         _lib.require_gpu(x_2d, what="FovealPattentionMLP training forward")
+        if self._train_fused(x_2d):
+            scores, context_16d, active_blocks = _TrainRouteFn.apply(
+                self.q_proj_16d(x_2d), self.block_keys_16d, self.base_blocks, self.remote_blocks,
+                float(self.temperature))
+            kgu, vs = _TrainGatherFn.apply(self.k_gate, self.k_up, self.v, active_blocks, self.block_size)
+            out_patt = _TrainPattFn.apply(x_2d, kgu, vs, _v_transposed(self.v))
+            return self._train_finish(out_patt, context_16d, scores, active_blocks, orig_shape, return_router_info)
         scores = self.compute_router_scores(x_2d)
         mean_scores = scores.mean(dim=0)
         _, top_remote = torch.topk(mean_scores[self.base_blocks:], k=self.remote_blocks)
@@ -499,6 +742,10 @@ class FovealPattentionMLP(nn.Module):
         out_patt = F.linear(act, self.v[indices].t())
         soft = F.softmax(scores / self.temperature, dim=-1)
         context_16d = torch.matmul(soft, self.block_keys_16d)
+        return self._train_finish(out_patt, context_16d, scores, active_blocks, orig_shape, return_router_info)
+
+    def _train_finish(self, out_patt: Tensor, context_16d: Tensor, scores: Tensor, active_blocks: Tensor, orig_shape,
+                      return_router_info: bool):
         out = (out_patt + self.out_proj_16d(context_16d)).reshape(*orig_shape)
         if return_router_info:
             return out, {
@@ -507,6 +754,22 @@ class FovealPattentionMLP(nn.Module):
                 "sparsity": (1.0 - self.total_active_blocks / self.num_blocks) * 100.0,
             }
         return out
+
+    def _train_fused(self, x_2d: Tensor) -> bool:
+        """Whether the training forward runs on csrc/mlp_train.hip: the fused SwiGLU (the eager
+        one rounds in between), one dtype, a 16-D index over at most 256 blocks, rows and
+        blocks of whole 16-byte vectors, and no autocast (which picks each op's type)."""
+        dt = x_2d.dtype
+        weights = (self.k_gate, self.k_up, self.v, self.q_proj_16d.weight, self.block_keys_16d)
+        return (self.use_fused_kernel and dt in (torch.bfloat16, torch.float32)
+                and all(w.dtype == dt and w.is_cuda for w in weights)
+                and self.index_dim == 16 and self.num_blocks <= 256 and x_2d.shape[0] > 0
+                and 0 < self.total_active_blocks and 0 <= self.base_blocks
+                and 0 <= self.remote_blocks <= self.num_blocks - self.base_blocks
+                and self.hidden_dim % 8 == 0 and self.block_size % 8 == 0 and self.temperature > 0
+                and self.intermediate_dim % self.block_size == 0
+                and tuple(self.v.shape) == tuple(self.k_gate.shape)
+                and not torch.is_autocast_enabled("cuda"))
 
     def forward(self, x: Tensor, return_router_info: bool = False):
         if self.training:

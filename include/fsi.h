@@ -155,6 +155,49 @@ FSI_API int fsi_swiglu_bwd(const void* dout, const void* g, const void* u, void*
                            void* stream);
 
 /* ------------------------------------------------------------------------- *
+ * Training path of FovealPattentionMLP beside its GEMMs
+ * (foveal_indexer/foveal_pattention.py:257-262, 292-307, 328-342).
+ *
+ * fsi_mlp_train_route: from the projected queries q (M, 16) and block keys (n_blocks, 16),
+ * scores = rms_norm(q) . keys^T / 4 (M, n_blocks), ctx = softmax(scores / temperature) . keys
+ * (M, 16) and the active list [0 .. base) ++ (topk(mean over tokens of scores[base:]) + base),
+ * largest first, equal means lower block first.  n_blocks <= 256.  _bwd: dq and dkeys from
+ * dscores and / or dctx (null: no gradient).  All arrays contiguous, of `dtype`.
+ *
+ * fsi_mlp_train_gather: kgu (2 n, D) = the active blocks' rows of k_gate, then of k_up
+ * (n = n_active * block), vs = v's, (n, D) or with v_transposed (v stored (D, N_p)) (D, n).
+ * fsi_mlp_train_scatter: the inverse for gradients, into whole contiguous (N_p, D) arrays (dv
+ * (D, N_p) with v_transposed), zero outside the active blocks; null outputs are skipped.
+ * Out-of-range block ids read as zero rows and are not written.  D and block multiples of 16
+ * bytes, 16-byte aligned rows.
+ *
+ * fsi_swiglu_pair: act (M, n) = silu(g) * u of gu (M, 2 n) = [g | u] rows, and its backward
+ * dgu = [dg | du]; fp32 arithmetic, one rounding.
+ * ------------------------------------------------------------------------- */
+FSI_API size_t fsi_mlp_train_route_workspace_size(int64_t M, int64_t n_blocks, int backward);
+
+FSI_API int fsi_mlp_train_route(const void* q, const void* keys, int64_t M, int64_t n_blocks, int64_t base_blocks,
+                                int64_t remote_blocks, float temperature, int dtype, void* scores, void* ctx,
+                                int32_t* active, void* workspace, size_t workspace_bytes, void* stream);
+
+FSI_API int fsi_mlp_train_route_bwd(const void* q, const void* keys, const void* dscores, const void* dctx, int64_t M,
+                                    int64_t n_blocks, float temperature, int dtype, void* dq, void* dkeys,
+                                    void* workspace, size_t workspace_bytes, void* stream);
+
+FSI_API int fsi_mlp_train_gather(const void* k_gate, const void* k_up, int64_t ldk, const void* v, int64_t ldv,
+                                 int v_transposed, const int32_t* active, int64_t n_active, int64_t block,
+                                 int64_t n_blocks, int64_t D, int dtype, void* kgu, void* vs, void* stream);
+
+FSI_API int fsi_mlp_train_scatter(const void* dkgu, const void* dvs, int v_transposed, const int32_t* active,
+                                  int64_t n_active, int64_t block, int64_t n_blocks, int64_t D, int dtype, void* dgate,
+                                  void* dup, void* dv, void* stream);
+
+FSI_API int fsi_swiglu_pair(const void* gu, int64_t M, int64_t n, int dtype, void* act, void* stream);
+
+FSI_API int fsi_swiglu_pair_bwd(const void* dact, const void* gu, int64_t M, int64_t n, int dtype, void* dgu,
+                                void* stream);
+
+/* ------------------------------------------------------------------------- *
  * Pooled 16-D router of FovealPattentionMLP in eval mode
  * (foveal_indexer/foveal_pattention.py:310-322):
  *   q = rms_norm(q_proj(mean_tokens(x))); s = q . block_keys^T * score_scale
