@@ -90,3 +90,43 @@ def test_decode_step_traces_to_fsi_ops(fsi):
         gm = make_fx(step, tracing_mode="fake")(*args)
     targets = [str(n.target) for n in gm.graph.nodes if n.op == "call_function"]
     assert any("fsi.mlp_router" in t for t in targets) and any("fsi.pattention_packed" in t for t in targets)
+
+
+def test_plain_call_only_where_the_dispatcher_has_nothing_to_do(fsi):
+    """A launch function is called past torch.ops only for plain tensors that autograd would
+    not record, outside every tracing, mode and transform."""
+    import torch.autograd.forward_ad as fwad
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    plain = fsi._lib._plain_call
+    t = torch.zeros(3)
+    leaf = torch.zeros(3, requires_grad=True)
+    assert plain((t, 1, None, torch.nn.Parameter(t, requires_grad=False)))
+    assert not plain((t, leaf))
+    with torch.no_grad():
+        assert plain((t, leaf))
+
+    class Sub(torch.Tensor):
+        pass
+
+    assert not plain((t.as_subclass(Sub),))
+    with FakeTensorMode() as mode:
+        fake = mode.from_tensor(t)
+        assert not plain((fake,))
+    assert not plain((fake,))
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    with Mode():
+        assert not plain((t,))
+    with torch.overrides.TorchFunctionMode():
+        assert not plain((t,))
+    with fwad.dual_level():
+        assert not plain((t,))
+    seen = []
+    torch.func.vmap(lambda a: (seen.append(plain((a,))), a)[1])(torch.zeros(2, 3))
+    torch.func.grad(lambda a: (seen.append(plain((t,))), a.sum())[1])(t)
+    assert seen == [False, False]
