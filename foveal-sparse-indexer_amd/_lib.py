@@ -200,6 +200,22 @@ SIGNATURES: dict[str, tuple] = {
         [_c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int,
          _c_ptr, _c_i64, _c_ptr, _c_size, _c_ptr],
     ),
+    "fsi_index_proj": (
+        _c_int,
+        [_c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr],
+    ),
+    "fsi_index_proj_dw_workspace_size": (_c_size, [_c_i64, _c_i64, _c_int]),
+    "fsi_index_proj_dw": (
+        _c_int,
+        [_c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_size,
+         _c_ptr],
+    ),
+    "fsi_index_expand": (_c_int, [_c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_int, _c_ptr, _c_ptr]),
+    "fsi_index_expand_bwd_workspace_size": (_c_size, [_c_i64, _c_i64]),
+    "fsi_index_expand_bwd": (
+        _c_int,
+        [_c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_size, _c_ptr],
+    ),
     "fsi_mlp_train_route_workspace_size": (_c_size, [_c_i64, _c_i64, _c_int]),
     "fsi_mlp_train_route": (
         _c_int,

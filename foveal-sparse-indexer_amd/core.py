@@ -307,6 +307,8 @@ class FovealIndexer(nn.Module):
     def compute_query_16d(self, x: Tensor) -> Tensor:
         """rms_norm(q_proj(x)) (core.py:214-222)."""
         what = "compute_query_16d"
+        if _projects_here(x, self.q_proj):
+            return index_rms_norm(_Proj16Fn.apply(x, self.q_proj.weight, None)[0], what)
         q = self.q_proj(x)
         return index_rms_norm(q, what)
 
@@ -318,8 +320,11 @@ class FovealIndexer(nn.Module):
         batch, n_elements, _ = x.shape
         if n_elements % self.block_size != 0:
             raise ValueError(f"Element length {n_elements} must be divisible by block_size={self.block_size}")
-        k_lin = self.k_proj(x)
-        v_lin = self.v_proj(x)
+        if _projects_here(x, self.k_proj, self.v_proj):
+            k_lin, v_lin = _Proj16Fn.apply(x, self.k_proj.weight, self.v_proj.weight)
+        else:
+            k_lin = self.k_proj(x)
+            v_lin = self.v_proj(x)
         _lib.require_gpu(k_lin, v_lin, what=what)
         _lib.dtype_code(k_lin.dtype, what)
         return _PoolKVFn.apply(k_lin.contiguous(), v_lin.contiguous(), self.block_size)
@@ -361,6 +366,8 @@ class FovealIndexer(nn.Module):
         if tuple(v.shape) != (B, Nb, self.index_dim):
             raise ValueError(f"{what}: values {tuple(v.shape)} != {(B, Nb, self.index_dim)}")
         context = _AdditiveContextFn.apply(s, v, self.causal)
+        if _plain_linear(self.out_proj, context) and self.out_proj.out_features % 8 == 0 and self.block_size > 0:
+            return _Expand16Fn.apply(context, self.out_proj.weight, self.block_size)
         out_blocks = self.out_proj(context)
         return out_blocks.repeat_interleave(self.block_size, dim=1)
 
@@ -454,6 +461,163 @@ class _DistillKLFn(torch.autograd.Function):
     def backward(ctx, g: Tensor):
         s, t, m8, n_rows = ctx.saved_tensors
         return _distill_kl_bwd_op(s, t, ctx.mode, m8, ctx.temperature, g, n_rows), None, None, None, None
+
+
+def _plain_linear(m: nn.Module, x: Tensor) -> bool:
+    """Whether m(x) is nothing but x W^T in x's type: a plain nn.Linear without bias or hooks
+    over 16 features on one side, outside autocast (which picks the type)."""
+    return (type(m) is nn.Linear and m.bias is None and type(m.weight) is nn.Parameter and m.weight.dtype == x.dtype
+            and x.dtype in (torch.float32, torch.bfloat16) and x.is_cuda and m.weight.device == x.device
+            and 16 in m.weight.shape
+            and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+            and not nn.modules.module._has_any_global_hook() and "forward" not in m.__dict__
+            and x.numel() > 0 and not torch.is_autocast_enabled("cuda"))
+
+
+def _projects_here(x: Tensor, *linears: nn.Module) -> bool:
+    """Whether the D -> 16 projections of x run on csrc/index_proj.hip: D a multiple of 128 (the
+    weight gradient's columns per wave); anything else is the linear layer's own GEMM."""
+    return (x.dim() in (2, 3) and x.shape[-1] % 128 == 0
+            and all(_plain_linear(m, x) and tuple(m.weight.shape) == (16, x.shape[-1]) for m in linears))
+
+
+def _rows_3d(x: Tensor) -> Tensor:
+    """x as (B, T, D) with unit stride over D and 16-byte aligned rows, copied if it must be."""
+    x = x if x.dim() == 3 else x.unsqueeze(0)
+    vec = 16 // x.element_size()
+    if x.stride(2) != 1 or x.stride(0) % vec or x.stride(1) % vec or x.data_ptr() % 16:
+        x = x.contiguous()
+        x = x if x.data_ptr() % 16 == 0 else x.clone()
+    return x
+
+
+def _aligned_contiguous(t: Tensor) -> Tensor:
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+@_lib.fsi_op("index_proj", lambda x, w0, w1: (x.new_empty((*x.shape[:-1], 16)),
+                                             x.new_empty((*x.shape[:-1], 16) if w1 is not None else (0,))))
+def _proj_op(x: Tensor, w0: Tensor, w1: Optional[Tensor]) -> Tuple[Tensor, Tensor]:
+    """fsi_index_proj: (x w0^T, x w1^T or empty)."""
+    what = "index projection"
+    dev = _lib.require_gpu(x, w0, w1, what=what)
+    lead = x.shape[:-1]
+    x3 = _rows_3d(x)
+    w0 = _aligned_contiguous(w0)
+    w1 = _aligned_contiguous(w1) if w1 is not None else None
+    y0 = torch.empty((*lead, 16), dtype=x.dtype, device=dev)
+    y1 = torch.empty((*lead, 16) if w1 is not None else (0,), dtype=x.dtype, device=dev)
+    B, T, D = x3.shape
+    st = _lib.lib().fsi_index_proj(x3.data_ptr(), x3.stride(0), x3.stride(1), B, T, D, w0.data_ptr(), _lib.ptr(w1),
+                                   _lib.dtype_code(x.dtype, what), y0.data_ptr(),
+                                   y1.data_ptr() if w1 is not None else None, _lib.stream_handle(dev))
+    _lib.check(st, what)
+    return y0, y1
+
+
+@_lib.fsi_op("index_proj_dw", lambda x, g0, g1: (x.new_empty((16, x.shape[-1])),
+                                                x.new_empty((16, x.shape[-1]) if g1 is not None else (0,))))
+def _proj_dw_op(x: Tensor, g0: Tensor, g1: Optional[Tensor]) -> Tuple[Tensor, Tensor]:
+    """fsi_index_proj_dw: (g0^T x, g1^T x or empty)."""
+    what = "index projection backward"
+    dev = _lib.require_gpu(x, g0, g1, what=what)
+    x3 = _rows_3d(x)
+    g0 = g0.contiguous()
+    g1 = g1.contiguous() if g1 is not None else None
+    B, T, D = x3.shape
+    nw = 2 if g1 is not None else 1
+    dw0 = torch.empty((16, D), dtype=x.dtype, device=dev)
+    dw1 = torch.empty((16, D) if g1 is not None else (0,), dtype=x.dtype, device=dev)
+    L = _lib.lib()
+    stream = _lib.stream_handle(dev)
+    ws = _lib.workspace(dev, L.fsi_index_proj_dw_workspace_size(B * T, D, nw), stream)
+    st = L.fsi_index_proj_dw(x3.data_ptr(), x3.stride(0), x3.stride(1), B, T, D, g0.data_ptr(), _lib.ptr(g1),
+                             _lib.dtype_code(x.dtype, what), dw0.data_ptr(), dw1.data_ptr() if nw == 2 else None,
+                             ws.data_ptr(), ws.numel(), stream)
+    _lib.check(st, what)
+    return dw0, dw1
+
+
+class _Proj16Fn(torch.autograd.Function):
+    """(x w0^T, x w1^T) over (.., D) x in one pass, w0 and w1 (16, D); w1 may be None."""
+
+    @staticmethod
+    def forward(ctx, x: Tensor, w0: Tensor, w1: Optional[Tensor]):
+        ctx.save_for_backward(x, w0, w1)
+        ctx.set_materialize_grads(False)
+        y0, y1 = _proj_op(x, w0, w1)
+        return (y0, y1) if w1 is not None else (y0, None)
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, g0: Optional[Tensor], g1: Optional[Tensor]):
+        x, w0, w1 = ctx.saved_tensors
+        need_x, need0, need1 = ctx.needs_input_grad
+        dx = dw0 = dw1 = None
+        if g0 is not None and need0 and g1 is not None and need1:
+            dw0, dw1 = _proj_dw_op(x, g0, g1)
+        elif g0 is not None and need0:
+            dw0 = _proj_dw_op(x, g0, None)[0]
+        elif g1 is not None and need1:
+            dw1 = _proj_dw_op(x, g1, None)[0]
+        if need_x:
+            for g, w in ((g0, w0), (g1, w1)):
+                if g is not None:
+                    d = torch.matmul(g, w)
+                    dx = d if dx is None else dx + d
+        return dx, dw0, dw1
+
+
+@_lib.fsi_op("index_expand", lambda ctx16, w, block: ctx16.new_empty(
+    (ctx16.shape[0], ctx16.shape[1] * block, w.shape[0])))
+def _expand_op(ctx16: Tensor, w: Tensor, block: int) -> Tensor:
+    """fsi_index_expand: (ctx16 w^T) of every block repeated over its elements."""
+    what = "additive_stream"
+    dev = _lib.require_gpu(ctx16, w, what=what)
+    c, w = _aligned_contiguous(ctx16), _aligned_contiguous(w)
+    B, nb = c.shape[:2]
+    D = w.shape[0]
+    out = torch.empty((B, nb * block, D), dtype=c.dtype, device=dev)
+    st = _lib.lib().fsi_index_expand(c.data_ptr(), w.data_ptr(), B * nb, block, D, _lib.dtype_code(c.dtype, what),
+                                     out.data_ptr(), _lib.stream_handle(dev))
+    _lib.check(st, what)
+    return out
+
+
+@_lib.fsi_op("index_expand_bwd", lambda dy, ctx16, w, block: (torch.empty_like(ctx16), torch.empty_like(w)))
+def _expand_bwd_op(dy: Tensor, ctx16: Tensor, w: Tensor, block: int) -> Tuple[Tensor, Tensor]:
+    """fsi_index_expand_bwd: (dctx16, dw)."""
+    what = "additive_stream backward"
+    dev = _lib.require_gpu(dy, ctx16, w, what=what)
+    dy, c, w = (_aligned_contiguous(t) for t in (dy.to(ctx16.dtype), ctx16, w))
+    n, D = c.shape[0] * c.shape[1], w.shape[0]
+    dc, dw = torch.empty_like(c), torch.empty_like(w)
+    L = _lib.lib()
+    stream = _lib.stream_handle(dev)
+    ws = _lib.workspace(dev, L.fsi_index_expand_bwd_workspace_size(n, D), stream)
+    st = L.fsi_index_expand_bwd(dy.data_ptr(), c.data_ptr(), w.data_ptr(), n, block, D,
+                                _lib.dtype_code(c.dtype, what), dc.data_ptr(), dw.data_ptr(), ws.data_ptr(),
+                                ws.numel(), stream)
+    _lib.check(st, what)
+    return dc, dw
+
+
+class _Expand16Fn(torch.autograd.Function):
+    """out_proj of the block context, repeated over each block's elements (core.py:310-312)."""
+
+    @staticmethod
+    def forward(ctx, context: Tensor, w: Tensor, block: int) -> Tensor:
+        ctx.save_for_backward(context, w)
+        ctx.block = block
+        return _expand_op(context, w, block)
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, dy: Tensor):
+        context, w = ctx.saved_tensors
+        dc, dw = _expand_bwd_op(dy, context, w, ctx.block)
+        return dc, dw, None
 
 
 @_lib.fsi_op("index_rms_norm", lambda xc, what: torch.empty_like(xc))

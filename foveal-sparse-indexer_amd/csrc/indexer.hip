@@ -1,11 +1,11 @@
 // 16-D indexer representations on MI355X (gfx950): the non-GEMM parts of
 // FovealIndexer (foveal_indexer/core.py:214-312).  The D -> 16 projections are
-// plain library GEMMs; everything after them runs here, with the reference's
+// products of their own (csrc/index_proj.hip); everything after them runs here, with the reference's
 // rounding points for bf16 tensors:
 //   * rms_norm over the 16 components: fp32, x * (1 / sqrt(mean(x^2) + FLT_EPSILON)),
 //     rounded once (F.rms_norm, core.py:222,241);
-//   * block pooling: mean over the block's tokens accumulated in fp32 in token
-//     order, divided by the block size, rounded (core.py:245-246); pooled keys
+//   * block pooling: mean over the block's tokens accumulated in fp32, divided by
+//     the block size, rounded (core.py:245-246); pooled keys
 //     are then L2-normalised in fp32 and rounded again (core.py:249);
 //   * cosine block scores: both sides L2-normalised in fp32 and rounded to the
 //     tensor dtype, dot products accumulated in fp32 and rounded, then divided
@@ -68,51 +68,75 @@ __global__ __launch_bounds__(256) void rms_norm_rows_kernel(const void* __restri
   for (int c = 0; c < IX_D; ++c) st<BF16>(out, r * IX_D + c, v[c]);
 }
 
-// One thread per (batch, block): pooled normalised key and mean value.
+// Sum over the 16 lanes l ^ 4, l ^ 8, l ^ 16, l ^ 32 (equal l & 3).
+__device__ __forceinline__ float sum_tokens16(float v) {
+#pragma unroll
+  for (int off = 4; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);
+  return v;
+}
+// Sum over four neighbouring lanes.
+__device__ __forceinline__ float sum_quad(float v) {
+  v += __shfl_xor(v, 1, 64);
+  return v + __shfl_xor(v, 2, 64);
+}
+// Four consecutive components.
+template <bool BF16>
+__device__ __forceinline__ f32x4_t ld4(const void* p, int64_t i) {
+  f32x4_t v;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) v[c] = ld<BF16>(p, i + c);
+  return v;
+}
+
+// One wave per (batch, block): pooled normalised key and mean value.  Lane l holds components
+// 4 (l & 3) .. of tokens l / 4, l / 4 + 16, .. so a wave reads 1 KiB of consecutive tokens at
+// once; a thread per block had walked its tokens one dependent load at a time (256 blocks of
+// 64 tokens: 77 -> 5 us).
 //   RMS: rms-normalise (and round) every token's key first (compute_kv_blocks_16d);
 //        off for FovealKVCache pages, whose keys arrive normalised (attention.py:305).
 //   KF32: write the normalised key in fp32 without rounding (FovealKVCache.kp_cache
 //        is fp32, attention.py:52,89-90); otherwise round to the input dtype.
 // Outputs are written at row stride out_stride (elements) per pooled row.
+constexpr int PK_WAVES = 4;
 template <bool BF16, bool RMS, bool KF32>
-__global__ __launch_bounds__(256) void pool_kv_kernel(const void* __restrict__ k_lin, const void* __restrict__ v_lin,
-                                                     int64_t n_pool, int block, int64_t in_group_stride,
-                                                     int64_t groups_per_batch, int64_t out_batch_stride,
-                                                     void* __restrict__ k_out, void* __restrict__ v_out) {
-  const int64_t pb = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;  // flat (batch, block)
-  if (pb >= n_pool) return;
+__global__ __launch_bounds__(64 * PK_WAVES) void pool_kv_kernel(
+    const void* __restrict__ k_lin, const void* __restrict__ v_lin, int64_t n_pool, int block, int64_t in_group_stride,
+    int64_t groups_per_batch, int64_t out_batch_stride, void* __restrict__ k_out, void* __restrict__ v_out) {
+  const int64_t pb = static_cast<int64_t>(blockIdx.x) * PK_WAVES + (threadIdx.x >> 6);  // flat (batch, block)
+  if (pb >= n_pool) return;  // whole waves exit together; no barrier below
+  const int lane = threadIdx.x & 63, c0 = 4 * (lane & 3);
   const int64_t bb = pb / groups_per_batch, gi = pb % groups_per_batch;
   const int64_t t0 = (bb * groups_per_batch + gi) * in_group_stride;  // element offset of the first token
-  const int64_t o = bb * out_batch_stride + gi * IX_D;
-  float ks[IX_D], vs[IX_D];
-#pragma unroll
-  for (int c = 0; c < IX_D; ++c) ks[c] = vs[c] = 0.f;
-  for (int t = 0; t < block; ++t) {
-    float kv[IX_D];
-#pragma unroll
-    for (int c = 0; c < IX_D; ++c) kv[c] = ld<BF16>(k_lin, t0 + t * IX_D + c);
+  const int64_t o = bb * out_batch_stride + gi * IX_D + c0;
+  f32x4_t ks = f32x4_t{0.f, 0.f, 0.f, 0.f}, vs = ks;
+  for (int t = lane >> 2; t < block; t += 16) {  // the four lanes of a token leave together
+    f32x4_t kv = ld4<BF16>(k_lin, t0 + static_cast<int64_t>(t) * IX_D + c0);
+    vs += ld4<BF16>(v_lin, t0 + static_cast<int64_t>(t) * IX_D + c0);
     if (RMS) {
-      rms_norm16(kv);
+      float ss = 0.f;
 #pragma unroll
-      for (int c = 0; c < IX_D; ++c) kv[c] = rnd<BF16>(kv[c]);
-    }
+      for (int c = 0; c < 4; ++c) ss = fmaf(kv[c], kv[c], ss);
+      const float r = 1.0f / sqrtf(sum_quad(ss) / static_cast<float>(IX_D) + FLT_EPS);
 #pragma unroll
-    for (int c = 0; c < IX_D; ++c) {
-      ks[c] += kv[c];
-      vs[c] += ld<BF16>(v_lin, t0 + t * IX_D + c);
+      for (int c = 0; c < 4; ++c) kv[c] = rnd<BF16>(kv[c] * r);
     }
+    ks += kv;
   }
   const float n = static_cast<float>(block);
+  float ss = 0.f;
 #pragma unroll
-  for (int c = 0; c < IX_D; ++c) {
-    ks[c] = rnd<BF16>(ks[c] / n);
-    st<BF16>(v_out, o + c, vs[c] / n);
+  for (int c = 0; c < 4; ++c) {
+    ks[c] = rnd<BF16>(sum_tokens16(ks[c]) / n);
+    vs[c] = sum_tokens16(vs[c]) / n;
+    ss = fmaf(ks[c], ks[c], ss);
   }
-  l2_normalize16(ks);
+  const float norm = fmaxf(sqrtf(sum_quad(ss)), 1e-12f);
+  if (lane >= 4) return;
 #pragma unroll
-  for (int c = 0; c < IX_D; ++c) {
-    if (KF32) static_cast<float*>(k_out)[o + c] = ks[c];
-    else st<BF16>(k_out, o + c, ks[c]);
+  for (int c = 0; c < 4; ++c) {
+    st<BF16>(v_out, o + c, vs[c]);
+    if (KF32) static_cast<float*>(k_out)[o + c] = ks[c] / norm;
+    else st<BF16>(k_out, o + c, ks[c] / norm);
   }
 }
 
@@ -320,84 +344,114 @@ __global__ __launch_bounds__(64 * PB_WAVES) void pool_kv_bwd_kernel(const void* 
 
 // Block-score backward.  With qn, kn the normalised (rounded) operands and
 // g = dscores / sqrt(d):  dqn = g kn,  dkn = g^T qn  (rounded, as the bmm's
-// gradients), then each through the normalisation.  One 64-lane workgroup per
-// (batch, 64-row tile); the other side is staged through LDS 64 rows at a time.
+// gradients), then each through the normalisation.  A workgroup owns 16 rows of
+// its side, 16 threads each; the other side is staged through LDS 64 rows at a
+// time (64 rows and one wave a workgroup left all but a few compute units idle
+// and read the gradient row by row: 4 x 64 x 64 blocks 26 + 17 -> 8 + 8 us).
 constexpr int SB_T = 64;
+constexpr int SB_R = 16;
+constexpr int SB_THREADS = 256;
 
+// Rows [r0, r0 + 64) of a (n, 16) operand, normalised and rounded, into LDS by the first wave.
 template <bool BF16>
-__global__ __launch_bounds__(SB_T) void block_scores_dq_kernel(const void* __restrict__ q, const void* __restrict__ k,
-                                                              const void* __restrict__ ds, int Q, int N, float sqrt_d,
-                                                              void* __restrict__ dq) {
-  __shared__ float kn[SB_T][IX_D];
-  __shared__ float tile[SB_T][SB_T + 1];
-  const int b = blockIdx.y, q0 = blockIdx.x * SB_T, lane = threadIdx.x;
-  const int nq = Q - q0 < SB_T ? Q - q0 : SB_T;
-  float acc[IX_D];
+__device__ __forceinline__ void stage_normalized(const void* x, int64_t base, int r0, int n, float (&out)[SB_T][IX_D + 1]) {
+  if (threadIdx.x >= SB_T) return;
+  const int r = r0 + static_cast<int>(threadIdx.x);
+  float v[IX_D];
 #pragma unroll
-  for (int c = 0; c < IX_D; ++c) acc[c] = 0.f;
-  for (int n0 = 0; n0 < N; n0 += SB_T) {
-    const int j = n0 + lane;
-    float kv[IX_D];
+  for (int c = 0; c < IX_D; ++c) v[c] = r < n ? ld<BF16>(x, (base + r) * IX_D + c) : 0.f;
+  l2_normalize16(v);
 #pragma unroll
-    for (int c = 0; c < IX_D; ++c) kv[c] = j < N ? ld<BF16>(k, (static_cast<int64_t>(b) * N + j) * IX_D + c) : 0.f;
-    l2_normalize16(kv);
-#pragma unroll
-    for (int c = 0; c < IX_D; ++c) kn[lane][c] = rnd<BF16>(kv[c]);
-    for (int r = 0; r < nq; ++r)
-      tile[r][lane] = j < N ? ld<BF16>(ds, (static_cast<int64_t>(b) * Q + q0 + r) * N + j) / sqrt_d : 0.f;
-    __syncthreads();
-    if (lane < nq) {
-      for (int jj = 0; jj < SB_T; ++jj) {
-        const float gg = tile[lane][jj];
-#pragma unroll
-        for (int c = 0; c < IX_D; ++c) acc[c] = fmaf(gg, kn[jj][c], acc[c]);
-      }
-    }
-    __syncthreads();
-  }
-  if (lane >= nq) return;
-  const int64_t row = static_cast<int64_t>(b) * Q + q0 + lane;
-  float qv[IX_D], out[IX_D];
-#pragma unroll
-  for (int c = 0; c < IX_D; ++c) {
-    qv[c] = ld<BF16>(q, row * IX_D + c);
-    acc[c] = rnd<BF16>(acc[c]);
-  }
-  l2_normalize16_bwd(qv, acc, out);
-#pragma unroll
-  for (int c = 0; c < IX_D; ++c) st<BF16>(dq, row * IX_D + c, out[c]);
+  for (int c = 0; c < IX_D; ++c) out[threadIdx.x][c] = rnd<BF16>(v[c]);
 }
 
 template <bool BF16>
-__global__ __launch_bounds__(SB_T) void block_scores_dk_kernel(const void* __restrict__ q, const void* __restrict__ k,
-                                                              const void* __restrict__ ds, int Q, int N, float sqrt_d,
-                                                              void* __restrict__ dk) {
-  __shared__ float qn[SB_T][IX_D];
-  const int b = blockIdx.y, lane = threadIdx.x;
-  const int j = blockIdx.x * SB_T + lane;
-  float acc[IX_D];
+__global__ __launch_bounds__(SB_THREADS) void block_scores_dq_kernel(const void* __restrict__ q,
+                                                                    const void* __restrict__ k,
+                                                                    const void* __restrict__ ds, int Q, int N,
+                                                                    float sqrt_d, void* __restrict__ dq) {
+  __shared__ float kn[SB_T][IX_D + 1];
+  const int b = blockIdx.y, part = threadIdx.x & 15;
+  const int qi = blockIdx.x * SB_R + (threadIdx.x >> 4);
+  const int64_t row = static_cast<int64_t>(b) * Q + (qi < Q ? qi : Q - 1);
+  float acc[IX_D] = {};
+  for (int n0 = 0; n0 < N; n0 += SB_T) {
+    float g[SB_T / 16];
 #pragma unroll
-  for (int c = 0; c < IX_D; ++c) acc[c] = 0.f;
-  for (int q0 = 0; q0 < Q; q0 += SB_T) {
-    const int qi = q0 + lane;
-    float qv[IX_D];
-#pragma unroll
-    for (int c = 0; c < IX_D; ++c) qv[c] = qi < Q ? ld<BF16>(q, (static_cast<int64_t>(b) * Q + qi) * IX_D + c) : 0.f;
-    l2_normalize16(qv);
-#pragma unroll
-    for (int c = 0; c < IX_D; ++c) qn[lane][c] = rnd<BF16>(qv[c]);
-    __syncthreads();
-    const int nq = Q - q0 < SB_T ? Q - q0 : SB_T;
-    if (j < N) {
-      for (int r = 0; r < nq; ++r) {
-        const float gg = ld<BF16>(ds, (static_cast<int64_t>(b) * Q + q0 + r) * N + j) / sqrt_d;
-#pragma unroll
-        for (int c = 0; c < IX_D; ++c) acc[c] = fmaf(gg, qn[r][c], acc[c]);
-      }
+    for (int i = 0; i < SB_T / 16; ++i) {
+      const int j = n0 + part + 16 * i;
+      g[i] = j < N ? ld<BF16>(ds, row * N + j) / sqrt_d : 0.f;
     }
+    stage_normalized<BF16>(k, static_cast<int64_t>(b) * N, n0, N, kn);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < SB_T / 16; ++i)
+#pragma unroll
+      for (int c = 0; c < IX_D; ++c) acc[c] = fmaf(g[i], kn[part + 16 * i][c], acc[c]);
     __syncthreads();
   }
-  if (j >= N) return;
+  float qv[IX_D], out[IX_D];
+#pragma unroll
+  for (int c = 0; c < IX_D; ++c) {
+#pragma unroll
+    for (int off = 1; off < 16; off <<= 1) acc[c] += __shfl_xor(acc[c], off, 64);
+    acc[c] = rnd<BF16>(acc[c]);
+    qv[c] = ld<BF16>(q, row * IX_D + c);
+  }
+  l2_normalize16_bwd(qv, acc, out);
+  if (qi >= Q) return;
+#pragma unroll
+  for (int c = 0; c < IX_D; ++c)
+    if (c == part) st<BF16>(dq, row * IX_D + c, out[c]);
+}
+
+// Sums of acc over the 16 threads of a key (threads t, t + 16, ..) for the first 16 threads:
+// 4 lanes of each wave, then the four waves through LDS.
+__device__ __forceinline__ void sum_key_threads(float (&acc)[IX_D], float (&red)[SB_THREADS / 64][SB_R][IX_D]) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int c = 0; c < IX_D; ++c) {
+    acc[c] += __shfl_xor(acc[c], 16, 64);
+    acc[c] += __shfl_xor(acc[c], 32, 64);
+    if (lane < SB_R) red[wave][lane][c] = acc[c];
+  }
+  __syncthreads();
+  if (threadIdx.x < SB_R)
+#pragma unroll
+    for (int c = 0; c < IX_D; ++c) {
+      acc[c] = red[0][lane][c];
+#pragma unroll
+      for (int w = 1; w < SB_THREADS / 64; ++w) acc[c] += red[w][lane][c];
+    }
+}
+
+template <bool BF16>
+__global__ __launch_bounds__(SB_THREADS) void block_scores_dk_kernel(const void* __restrict__ q,
+                                                                    const void* __restrict__ k,
+                                                                    const void* __restrict__ ds, int Q, int N,
+                                                                    float sqrt_d, void* __restrict__ dk) {
+  __shared__ float qn[SB_T][IX_D + 1];
+  __shared__ float red[SB_THREADS / 64][SB_R][IX_D];
+  const int b = blockIdx.y, part = threadIdx.x >> 4;
+  const int j = blockIdx.x * SB_R + (threadIdx.x & 15), jl = j < N ? j : N - 1;
+  float acc[IX_D] = {};
+  for (int q0 = 0; q0 < Q; q0 += SB_T) {
+    float g[SB_T / 16];
+#pragma unroll
+    for (int i = 0; i < SB_T / 16; ++i) {
+      const int r = q0 + part + 16 * i;
+      g[i] = r < Q ? ld<BF16>(ds, (static_cast<int64_t>(b) * Q + r) * N + jl) / sqrt_d : 0.f;
+    }
+    stage_normalized<BF16>(q, static_cast<int64_t>(b) * Q, q0, Q, qn);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < SB_T / 16; ++i)
+#pragma unroll
+      for (int c = 0; c < IX_D; ++c) acc[c] = fmaf(g[i], qn[part + 16 * i][c], acc[c]);
+    __syncthreads();
+  }
+  sum_key_threads(acc, red);
+  if (threadIdx.x >= SB_R || j >= N) return;
   const int64_t row = static_cast<int64_t>(b) * N + j;
   float kv[IX_D], out[IX_D];
 #pragma unroll
@@ -461,44 +515,49 @@ __global__ __launch_bounds__(AC_THREADS) void additive_context_bwd_rows_kernel(
 }
 
 // Additive-context backward, values: dv_j = sum_q p_qj dctx_q with the rounded
-// probabilities of the forward.  One 64-lane workgroup per (batch, 64-key tile);
-// the query rows' dctx and softmax statistics are staged through LDS.
+// probabilities of the forward.  16 keys a workgroup, 16 threads each; the query
+// rows' dctx and softmax statistics are staged through LDS (one wave per 64 keys:
+// 24 -> 5.4 us at 4 x 64 x 64).
 template <bool BF16>
-__global__ __launch_bounds__(SB_T) void additive_context_dv_kernel(const void* __restrict__ scores,
-                                                                  const void* __restrict__ dctx,
-                                                                  const float2* __restrict__ stats, int Q, int N,
-                                                                  int causal, void* __restrict__ dv) {
-  __shared__ float gs[SB_T][IX_D];
+__global__ __launch_bounds__(SB_THREADS) void additive_context_dv_kernel(const void* __restrict__ scores,
+                                                                        const void* __restrict__ dctx,
+                                                                        const float2* __restrict__ stats, int Q, int N,
+                                                                        int causal, void* __restrict__ dv) {
+  __shared__ float gs[SB_T][IX_D + 1];
   __shared__ float2 ms[SB_T];
-  const int b = blockIdx.y, lane = threadIdx.x;
-  const int j0 = blockIdx.x * SB_T, j = j0 + lane;
-  float acc[IX_D];
-#pragma unroll
-  for (int c = 0; c < IX_D; ++c) acc[c] = 0.f;
+  __shared__ float red[SB_THREADS / 64][SB_R][IX_D];
+  const int b = blockIdx.y, part = threadIdx.x >> 4;
+  const int j0 = blockIdx.x * SB_R, j = j0 + (threadIdx.x & 15), jl = j < N ? j : N - 1;
+  float acc[IX_D] = {};
   const int q_first = causal ? (j0 + 1) / SB_T * SB_T : 0;  // rows q <= j see no key j when causal
   for (int q0 = q_first; q0 < Q; q0 += SB_T) {
-    const int qi = q0 + lane;
-    if (qi < Q) {
-      const int64_t row = static_cast<int64_t>(b) * Q + qi;
+    float x[SB_T / 16];
 #pragma unroll
-      for (int c = 0; c < IX_D; ++c) gs[lane][c] = ld<BF16>(dctx, row * IX_D + c);
-      ms[lane] = stats[row];
+    for (int i = 0; i < SB_T / 16; ++i) {
+      const int r = q0 + part + 16 * i;
+      x[i] = r < Q ? ld<BF16>(scores, (static_cast<int64_t>(b) * Q + r) * N + jl) : 0.f;
+    }
+    if (threadIdx.x < SB_T) {
+      const int qi = q0 + static_cast<int>(threadIdx.x);
+      const int64_t row = static_cast<int64_t>(b) * Q + (qi < Q ? qi : Q - 1);
+#pragma unroll
+      for (int c = 0; c < IX_D; ++c) gs[threadIdx.x][c] = qi < Q ? ld<BF16>(dctx, row * IX_D + c) : 0.f;
+      ms[threadIdx.x] = stats[row];
     }
     __syncthreads();
-    const int nq = Q - q0 < SB_T ? Q - q0 : SB_T;
-    if (j < N) {
-      for (int r = 0; r < nq; ++r) {
-        if (causal && j >= q0 + r) continue;
-        const float2 st2 = ms[r];
-        const float p = rnd<BF16>(expf(ld<BF16>(scores, (static_cast<int64_t>(b) * Q + q0 + r) * N + j) - st2.x) /
-                                  st2.y);
+#pragma unroll
+    for (int i = 0; i < SB_T / 16; ++i) {
+      const int r = part + 16 * i;
+      if (q0 + r < Q && !(causal && j >= q0 + r)) {
+        const float p = rnd<BF16>(expf(x[i] - ms[r].x) / ms[r].y);
 #pragma unroll
         for (int c = 0; c < IX_D; ++c) acc[c] = fmaf(p, gs[r][c], acc[c]);
       }
     }
     __syncthreads();
   }
-  if (j >= N) return;
+  sum_key_threads(acc, red);
+  if (threadIdx.x >= SB_R || j >= N) return;
 #pragma unroll
   for (int c = 0; c < IX_D; ++c) st<BF16>(dv, (static_cast<int64_t>(b) * N + j) * IX_D + c, acc[c]);
 }
@@ -536,7 +595,7 @@ FSI_API int fsi_index_pool_kv(const void* k_lin, const void* v_lin, int dtype, i
   if (n_pool == 0) return FSI_OK;
   FSI_CHECK_ARG(k_lin && v_lin && k_blocks && v_blocks, FSI_ERR_INVALID_ARG, "index_pool_kv: null pointer");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const unsigned grid = static_cast<unsigned>((n_pool + 255) / 256);
+  const unsigned grid = static_cast<unsigned>((n_pool + PK_WAVES - 1) / PK_WAVES);
   const int64_t gs = block_size * IX_D;
   if (dtype == FSI_DTYPE_BF16)
     pool_kv_kernel<true, true, false><<<grid, 256, 0, st>>>(k_lin, v_lin, n_pool, (int)block_size, gs, nb, nb * IX_D,
@@ -559,7 +618,7 @@ FSI_API int fsi_kv_page_pool(const void* partial_k, const void* partial_v, int d
   if (B == 0) return FSI_OK;
   FSI_CHECK_ARG(partial_k && partial_v && kp_out && vp_out, FSI_ERR_INVALID_ARG, "kv_page_pool: null pointer");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const unsigned grid = static_cast<unsigned>((B + 255) / 256);
+  const unsigned grid = static_cast<unsigned>((B + PK_WAVES - 1) / PK_WAVES);
   const int64_t gs = page_size * IX_D;
   if (dtype == FSI_DTYPE_BF16)
     pool_kv_kernel<true, false, true><<<grid, 256, 0, st>>>(partial_k, partial_v, B, (int)page_size, gs, 1,
@@ -674,19 +733,19 @@ FSI_API int fsi_block_scores_bwd(const void* q, const void* k, const void* dscor
   const float sqrt_d = static_cast<float>(sqrt(static_cast<double>(index_dim)));
   // Q == 0 or N == 0: the kernels still run on the other side and write zero gradients.
   if (Q > 0) {
-    const dim3 gq(static_cast<unsigned>((Q + SB_T - 1) / SB_T), static_cast<unsigned>(B));
+    const dim3 gq(static_cast<unsigned>((Q + SB_R - 1) / SB_R), static_cast<unsigned>(B));
     if (dtype == FSI_DTYPE_BF16)
-      block_scores_dq_kernel<true><<<gq, SB_T, 0, st>>>(q, k, dscores, (int)Q, (int)N, sqrt_d, dq);
+      block_scores_dq_kernel<true><<<gq, SB_THREADS, 0, st>>>(q, k, dscores, (int)Q, (int)N, sqrt_d, dq);
     else
-      block_scores_dq_kernel<false><<<gq, SB_T, 0, st>>>(q, k, dscores, (int)Q, (int)N, sqrt_d, dq);
+      block_scores_dq_kernel<false><<<gq, SB_THREADS, 0, st>>>(q, k, dscores, (int)Q, (int)N, sqrt_d, dq);
     FSI_HIP_LAUNCH_CHECK("block_scores_bwd (dq)");
   }
   if (N > 0) {
-    const dim3 gk(static_cast<unsigned>((N + SB_T - 1) / SB_T), static_cast<unsigned>(B));
+    const dim3 gk(static_cast<unsigned>((N + SB_R - 1) / SB_R), static_cast<unsigned>(B));
     if (dtype == FSI_DTYPE_BF16)
-      block_scores_dk_kernel<true><<<gk, SB_T, 0, st>>>(q, k, dscores, (int)Q, (int)N, sqrt_d, dk);
+      block_scores_dk_kernel<true><<<gk, SB_THREADS, 0, st>>>(q, k, dscores, (int)Q, (int)N, sqrt_d, dk);
     else
-      block_scores_dk_kernel<false><<<gk, SB_T, 0, st>>>(q, k, dscores, (int)Q, (int)N, sqrt_d, dk);
+      block_scores_dk_kernel<false><<<gk, SB_THREADS, 0, st>>>(q, k, dscores, (int)Q, (int)N, sqrt_d, dk);
     FSI_HIP_LAUNCH_CHECK("block_scores_bwd (dk)");
   }
   return FSI_OK;
@@ -728,12 +787,12 @@ FSI_API int fsi_additive_context_bwd(const void* scores, const void* v_blocks, c
     FSI_HIP_LAUNCH_CHECK("additive_context_bwd (rows)");
   }
   if (N > 0) {
-    const dim3 gv(static_cast<unsigned>((N + SB_T - 1) / SB_T), static_cast<unsigned>(B));
+    const dim3 gv(static_cast<unsigned>((N + SB_R - 1) / SB_R), static_cast<unsigned>(B));
     if (dtype == FSI_DTYPE_BF16)
-      additive_context_dv_kernel<true><<<gv, SB_T, 0, st>>>(scores, dcontext, stats, (int)Q, (int)N, causal,
+      additive_context_dv_kernel<true><<<gv, SB_THREADS, 0, st>>>(scores, dcontext, stats, (int)Q, (int)N, causal,
                                                             dv_blocks);
     else
-      additive_context_dv_kernel<false><<<gv, SB_T, 0, st>>>(scores, dcontext, stats, (int)Q, (int)N, causal,
+      additive_context_dv_kernel<false><<<gv, SB_THREADS, 0, st>>>(scores, dcontext, stats, (int)Q, (int)N, causal,
                                                              dv_blocks);
     FSI_HIP_LAUNCH_CHECK("additive_context_bwd (values)");
   }

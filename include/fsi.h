@@ -296,6 +296,32 @@ FSI_API int fsi_decode_route(const void* qi, const float* kp, const void* vp, in
  * points apply everything after them with the reference's bf16 rounding points.
  * All tensors contiguous and of `dtype`.
  * ------------------------------------------------------------------------- */
+/* ------------------------------------------------------------------------- *
+ * Products around the 16-D index (core.py:214-250, 288-312).
+ * fsi_index_proj: y_i = x w_i^T for one or two (16, D) weights (w1 / y1 null: one); x row
+ * (b, t) at x + b xs_b + t xs_t, y (B T, 16) contiguous.  fsi_index_proj_dw: dw_i = g_i^T x
+ * from g_i (B T, 16).  fsi_index_expand: out[p block + t] = ctx[p] w^T for t < block, w
+ * (D, 16), out (n_pool block, D); _bwd: dctx and dw from dy.  D a multiple of 128
+ * (projections) or 8, 16-byte aligned rows, fp32 sums.
+ * ------------------------------------------------------------------------- */
+FSI_API int fsi_index_proj(const void* x, int64_t xs_b, int64_t xs_t, int64_t B, int64_t T, int64_t D, const void* w0,
+                           const void* w1, int dtype, void* y0, void* y1, void* stream);
+
+FSI_API size_t fsi_index_proj_dw_workspace_size(int64_t M, int64_t D, int n_weights);
+
+FSI_API int fsi_index_proj_dw(const void* x, int64_t xs_b, int64_t xs_t, int64_t B, int64_t T, int64_t D,
+                              const void* g0, const void* g1, int dtype, void* dw0, void* dw1, void* workspace,
+                              size_t workspace_bytes, void* stream);
+
+FSI_API int fsi_index_expand(const void* ctx, const void* w, int64_t n_pool, int64_t block, int64_t D, int dtype,
+                             void* out, void* stream);
+
+FSI_API size_t fsi_index_expand_bwd_workspace_size(int64_t n_pool, int64_t D);
+
+FSI_API int fsi_index_expand_bwd(const void* dy, const void* ctx, const void* w, int64_t n_pool, int64_t block,
+                                 int64_t D, int dtype, void* dctx, void* dw, void* workspace, size_t workspace_bytes,
+                                 void* stream);
+
 /* F.rms_norm over the 16 components (eps = FLT_EPSILON), x/out: (M, 16).
  * Replaces the norm of compute_query_16d (core.py:221-222) and of decode_step's
  * index key (attention.py:305). */
