@@ -33,6 +33,14 @@ int down_gather(const fsi::bf16_t* H, int64_t ldh, const fsi::bf16_t* wd, int64_
                 int n_active, int block_n, int M, int D, fsi::bf16_t* out, int64_t ldo, int* err, hipStream_t st);
 }  // namespace fsi_gemm
 
+namespace fsi_mid {  // csrc/pattention_mid.hip: 65 .. 255 tokens
+size_t workspace_bytes(int64_t M, int64_t K, int64_t D_out, int64_t n_channels);
+int run(const fsi::bf16_t* x, int64_t ldx, const fsi::bf16_t* kg, const fsi::bf16_t* ku, int64_t ldk,
+        const fsi::bf16_t* vt, int64_t ldv, const int32_t* active, int64_t n_blocks, int log2bn, int64_t M, int64_t K,
+        int64_t n_ch, int64_t D, int rounding, fsi::bf16_t* out, int64_t ldo, void* workspace, size_t ws_bytes,
+        int* err, hipStream_t st);
+}  // namespace fsi_mid
+
 namespace fsi_dec {
 size_t workspace_bytes(int64_t M, int64_t K, int64_t D, int64_t n_ch, int log2bn);
 int run(const fsi::bf16_t* x, int64_t ldx, const fsi::bf16_t* kg, const fsi::bf16_t* ku, int64_t ldk,
@@ -588,7 +596,9 @@ size_t fsi_pattention_workspace_size(int64_t M, int64_t K, int64_t D_out, int64_
   const size_t skinny = make_plan_bf16(M, D_out, n_channels).total;
   // the decode path (M <= 64) needs its split partials too; block sizes >= 32 only
   const size_t dec = fsi_dec::workspace_bytes(M, K, D_out, n_channels, 5);
-  return skinny > dec ? skinny : dec;
+  const size_t mid = fsi_mid::workspace_bytes(M, K, D_out, n_channels);
+  const size_t most = skinny > dec ? skinny : dec;
+  return most > mid ? most : mid;
 }
 
 int fsi_pattention_fwd(const void* x, int64_t ldx, const void* k_gate, const void* k_up, int64_t ldk,
@@ -695,6 +705,20 @@ int fsi_pattention_fwd(const void* x, int64_t ldx, const void* k_gate, const voi
                                rounding, static_cast<bf16_t*>(out), ldo, workspace, workspace_bytes, err, st);
     if (r < 0) {
       fsi_host::set_last_error("pattention: decode launch failed: %s", hipGetErrorString(hipGetLastError()));
+      return FSI_ERR_HIP;
+    }
+    if (r == 0) return FSI_OK;
+  }
+
+  // 65 .. 255 tokens: all of them against a few weight rows and a range of the contraction
+  // (csrc/pattention_mid.hip); falls through when its shape conditions do not hold.
+  if (M > 64 && M < GEMM_MIN_M && activation == FSI_ACT_SWIGLU && v_transposed && block_n >= 64 &&
+      N_p % block_n == 0 && ldv % 8 == 0 && (uintptr_t)v % 16 == 0) {
+    const int r = fsi_mid::run(xb, ldx, kgb, kub, ldk, static_cast<const bf16_t*>(v), ldv, active_blocks, cm.n_blocks,
+                               cm.log2bn, M, K, n_channels, D_out, rounding, static_cast<bf16_t*>(out), ldo, workspace,
+                               workspace_bytes, err, st);
+    if (r < 0) {
+      fsi_host::set_last_error("pattention: mid launch failed: %s", hipGetErrorString(hipGetLastError()));
       return FSI_ERR_HIP;
     }
     if (r == 0) return FSI_OK;
