@@ -9,7 +9,7 @@
 // gathers them).
 //
 //   dec32_partial_kernel: wave (split s, b Hkv + g, head group) takes keys
-//     [128 s, 128 s + 128) of that list for up to 16 query heads of KV head g.
+//     [SPLIT s, SPLIT s + SPLIT) of that list for up to 16 query heads of KV head g.
 //     Scores and products on v_mfma_f32_16x16x4_f32: S^T[key][head] with
 //     A = K rows (16-byte loads: 4 dims a lane) and B = q^T; the softmax
 //     probabilities of the lane's accumulator are, element by element, the A
@@ -17,10 +17,13 @@
 //     16-key tile takes keys 4 (lane / 16) + kk), B = V rows read 16 dims
 //     at a time.  The split's max, sum and unnormalised output go to the
 //     workspace (log2 units).
-//   dec32_merge_kernel: wave (b, h) combines the splits of its sequence.
+//   dec32_merge_kernel: one wave (four with the short splits) of (b, h) combines the
+//     splits of its sequence.
 // The K / V stream is read once per KV head (the query heads of a group share
 // it), which makes the step HBM-bound; the unused MFMA columns of groups of
 // fewer than 16 heads cost MFMA time the stream leaves free.
+#include <type_traits>
+
 #include "fsi_common.h"
 
 using namespace fsi;
@@ -30,13 +33,18 @@ namespace {
 // 96 keys per wave: at the C4 shape (3072 keys per sequence and KV head) 32 splits fill
 // the chip's 4096 wave slots (four per SIMD) in two whole rounds; 128 (1.5 rounds)
 // measured 0.197-0.203 ms against 0.188-0.189, 64 / 80 / 112 no better than 128 and
-// 192 (two waves per SIMD) 0.245.
+// 192 (two waves per SIMD) 0.245.  Where that leaves many of the slots
+// empty, the step waits for one wave's chain of loads, so it takes 32 keys per wave:
+// 4 sequences x 8 KV heads (1024 waves of 96), 100 MB: partial kernel 35.9 -> 22.9 us,
+// 4.4 TB/s.  The line lies where the two meet, whole step at hd 128 / 64: 2304 waves
+// 84 -> 74 / 51.5 -> 40.7 us, 3072 waves 83.9 both, 4096 waves 98.5 -> 106.
 #ifndef FSI_D32_SPLIT
 #define FSI_D32_SPLIT 96
 #endif
 constexpr int D_SPLIT = FSI_D32_SPLIT;  // keys per split (one wave)
-constexpr int D_TILES = D_SPLIT / 16;
-static_assert(D_SPLIT % 16 == 0 && D_SPLIT >= 16, "a split is whole 16-key tiles");
+constexpr int D_SPLIT_SMALL = 32;
+constexpr int64_t D_SMALL_WAVES = 2560;  // waves of D_SPLIT keys up to which the short splits are taken
+static_assert(D_SPLIT % 16 == 0 && D_SPLIT_SMALL % 16 == 0, "a split is whole 16-key tiles");
 constexpr int D_WAVES = 4;    // splits per workgroup
 constexpr int D_HG = 16;      // query heads per MFMA column block
 constexpr float D_LOG2E = 1.4426950408889634f;
@@ -101,9 +109,9 @@ __device__ __forceinline__ f32x4_t mfma4(float a, float b, f32x4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-template <int HD>
+template <int HD, int SPLIT>
 __global__ __launch_bounds__(64 * D_WAVES) void dec32_partial_kernel(D32Params P) {
-  constexpr int DG = HD / 16;
+  constexpr int DG = HD / 16, D_TILES = SPLIT / 16;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 15, kg = lane >> 4;
   const int s = blockIdx.x * D_WAVES + wave;  // split
@@ -112,7 +120,7 @@ __global__ __launch_bounds__(64 * D_WAVES) void dec32_partial_kernel(D32Params P
   const int h0 = g * P.G + blockIdx.z * D_HG;  // first query head of this column block
   const int nh = P.G - blockIdx.z * D_HG < D_HG ? P.G - blockIdx.z * D_HG : D_HG;
   const KeyList L = key_list(P, b);
-  if (s * D_SPLIT >= L.total) return;  // whole wave; no barriers in this kernel
+  if (s * SPLIT >= L.total) return;  // whole wave; no barriers in this kernel
   const float* kb = P.k + b * P.ks_b + g * P.ks_h;
   const float* vb = P.v + b * P.vs_b + g * P.vs_h;
 
@@ -130,7 +138,7 @@ __global__ __launch_bounds__(64 * D_WAVES) void dec32_partial_kernel(D32Params P
   int tok[D_TILES][4];  // token of key 16 t + 4 kg + e (-1: masked)
 #pragma unroll
   for (int t = 0; t < D_TILES; ++t) {
-    const int i0 = s * D_SPLIT + 16 * t;
+    const int i0 = s * SPLIT + 16 * t;
     const int tr = key_token(P, L, b, i0 + r, bad);  // the K row this lane loads
     const float* krow = kb + static_cast<int64_t>(tr >= 0 ? tr : 0) * P.ks_t + 4 * kg;
     f32x4_t kf[DG];
@@ -204,35 +212,39 @@ __global__ __launch_bounds__(64 * D_WAVES) void dec32_partial_kernel(D32Params P
   }
 }
 
-// Lane j of the wave takes splits j, j + 64, ...: the maximum and the split
-// weights exp2(m_s - M) come out of two wave reductions, then every lane adds
-// its dims of the weighted split outputs, the splits' loads issued together.
-template <int HD>
-__global__ __launch_bounds__(64 * D_WAVES) void dec32_merge_kernel(D32Params P) {
-  const int lane = threadIdx.x & 63;
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * D_WAVES + (threadIdx.x >> 6);  // (b, h)
-  if (row >= static_cast<int64_t>(P.B) * P.Hq) return;
-  const int b = static_cast<int>(row / P.Hq);
+// WPR waves a row (b, h), each over a contiguous part of the splits: the maximum over
+// all splits, then lane j of a wave takes the split weights exp2(m_s - M) of its part 64
+// at a time and every lane adds its dims of the weighted split outputs, eight splits'
+// loads issued together; the parts meet in LDS.
+template <int HD, int WPR>
+__global__ __launch_bounds__(64 * D_WAVES) void dec32_merge_kernel(D32Params P, int split) {
+  constexpr int DPL = (HD + 63) / 64;
+  __shared__ float red[D_WAVES][HD + 1];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t row = (static_cast<int64_t>(blockIdx.x) * D_WAVES + wave) / WPR;  // (b, h)
+  const bool live = row < static_cast<int64_t>(P.B) * P.Hq;
+  if (WPR == 1 && !live) return;
+  const int b = live ? static_cast<int>(row / P.Hq) : 0;
   const KeyList L = key_list(P, b);
-  const int ns = (L.total + D_SPLIT - 1) / D_SPLIT;
-  const float* pp = P.part + row * P.n_split * (HD + 2);
+  const int ns = live ? (L.total + split - 1) / split : 0;
+  const float* pp = P.part + (live ? row : 0) * P.n_split * (HD + 2);
   float M = -INFINITY;
   for (int s = lane; s < ns; s += 64) M = __builtin_fmaxf(M, pp[s * (HD + 2)]);
   M = wave_max(M);
-  constexpr int DPL = (HD + 63) / 64;
+  const int per = (ns + WPR - 1) / WPR, first = wave % WPR * per, last = first + per < ns ? first + per : ns;
   float o[DPL] = {};
   float lsum = 0.f;
   if (M != -INFINITY) {
-    for (int s0 = 0; s0 < ns; s0 += 64) {
-      // lane j: weight of split s0 + j (0 for splits with no key or past the count)
+    for (int s0 = first; s0 < last; s0 += 64) {
+      // lane j: weight of split s0 + j (0 for splits with no key or past the part)
       float wj = 0.f, lj = 0.f;
-      if (s0 + lane < ns) {
+      if (s0 + lane < last) {
         const float ms = pp[(s0 + lane) * (HD + 2)];
         wj = ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - M);
         lj = pp[(s0 + lane) * (HD + 2) + 1];
       }
       lsum += wave_sum(wj * lj);
-      const int n = ns - s0 < 64 ? ns - s0 : 64;
+      const int n = last - s0 < 64 ? last - s0 : 64;
       // eight splits' loads issued together, then added in split order (the same
       // fmaf chain as one split at a time; one at a time left a load latency per split)
       int j = 0;
@@ -268,6 +280,23 @@ __global__ __launch_bounds__(64 * D_WAVES) void dec32_merge_kernel(D32Params P) 
       }
     }
   }
+  if constexpr (WPR > 1) {
+    if (wave % WPR) {
+#pragma unroll
+      for (int e = 0; e < DPL; ++e)
+        if (lane + 64 * e < HD) red[wave][lane + 64 * e] = o[e];
+      if (lane == 0) red[wave][HD] = lsum;
+    }
+    __syncthreads();
+    if (wave % WPR || !live) return;
+#pragma unroll
+    for (int w = 1; w < WPR; ++w) {
+#pragma unroll
+      for (int e = 0; e < DPL; ++e)
+        if (lane + 64 * e < HD) o[e] += red[wave + w][lane + 64 * e];
+      lsum += red[wave + w][HD];
+    }
+  }
   const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
 #pragma unroll
   for (int e = 0; e < DPL; ++e) {
@@ -281,13 +310,19 @@ __global__ __launch_bounds__(64 * D_WAVES) void dec32_merge_kernel(D32Params P) 
 namespace fsi_dec32 {
 
 // Split-key count and workspace bytes for a call (an upper bound over the batch).
-int64_t n_split(int64_t window, int64_t capacity, int64_t page_size, int64_t max_seq) {
+int64_t n_split(int64_t window, int64_t capacity, int64_t page_size, int64_t max_seq, int64_t split) {
   const int64_t keys = (window < max_seq ? window : max_seq) + capacity * page_size;
-  return keys <= 0 ? 1 : (keys + D_SPLIT - 1) / D_SPLIT;
+  return keys <= 0 ? 1 : (keys + split - 1) / split;
+}
+size_t part_bytes_for(int64_t B, int64_t Hq, int64_t head_dim, int64_t ns) {
+  return static_cast<size_t>(B * Hq * ns * (head_dim + 2)) * sizeof(float);
 }
 size_t workspace_bytes(int64_t B, int64_t Hq, int64_t head_dim, int64_t window, int64_t capacity, int64_t page_size,
                        int64_t max_seq) {
-  return static_cast<size_t>(B * Hq * n_split(window, capacity, page_size, max_seq) * (head_dim + 2)) * sizeof(float);
+  const int64_t ns = n_split(window, capacity, page_size, max_seq, D_SPLIT);
+  // the short splits' partials where some grouping of the heads would take them
+  const bool small = B * ((Hq + D_HG - 1) / D_HG) * ns <= D_SMALL_WAVES;
+  return part_bytes_for(B, Hq, head_dim, small ? n_split(window, capacity, page_size, max_seq, D_SPLIT_SMALL) : ns);
 }
 
 // fp32, head_dim 64 or 128, 16-byte aligned K rows: the split kernels; returns 1
@@ -297,14 +332,19 @@ int run(const float* q, const float* k, const float* v, int64_t ks_b, int64_t ks
         int64_t page_size, const int32_t* remote_pages, const int32_t* remote_counts, int64_t capacity, int64_t B,
         int64_t Hq, int64_t Hkv, int64_t head_dim, float scale, float* out, float* part, size_t part_bytes, int* err,
         hipStream_t st) {
-  const int64_t ns = n_split(window, capacity, page_size, max_seq);
   const int64_t G = Hq / Hkv;
+  int64_t ns = n_split(window, capacity, page_size, max_seq, D_SPLIT);
+  const int64_t ns_small = n_split(window, capacity, page_size, max_seq, D_SPLIT_SMALL);
   const bool fits = (head_dim == 64 || head_dim == 128) && ks_t % 4 == 0 && ks_h % 4 == 0 && ks_b % 4 == 0 &&
                     reinterpret_cast<uintptr_t>(k) % 16 == 0 && reinterpret_cast<uintptr_t>(q) % 16 == 0 &&
                     part != nullptr &&
-                    part_bytes >= workspace_bytes(B, Hq, head_dim, window, capacity, page_size, max_seq) &&
+                    part_bytes >= part_bytes_for(B, Hq, head_dim, ns) &&
                     (ns + D_WAVES - 1) / D_WAVES <= 0x7fffffff && B * Hkv <= 65535 && (G + D_HG - 1) / D_HG <= 65535;
   if (!fits) return 1;
+  const bool small = B * Hkv * ((G + D_HG - 1) / D_HG) * ns <= D_SMALL_WAVES &&
+                     part_bytes >= part_bytes_for(B, Hq, head_dim, ns_small);
+  const int split = small ? D_SPLIT_SMALL : D_SPLIT;
+  if (small) ns = ns_small;
   D32Params P{};
   P.q = q;
   P.k = k;
@@ -336,17 +376,20 @@ int run(const float* q, const float* k, const float* v, int64_t ks_b, int64_t ks
   P.err = err;
   const dim3 g1(static_cast<unsigned>((ns + D_WAVES - 1) / D_WAVES), static_cast<unsigned>(B * Hkv),
                 static_cast<unsigned>((G + D_HG - 1) / D_HG));
-  const dim3 g2(static_cast<unsigned>((B * Hq + D_WAVES - 1) / D_WAVES));
-  if (head_dim == 64) {
-    dec32_partial_kernel<64><<<g1, 64 * D_WAVES, 0, st>>>(P);
-    FSI_HIP_LAUNCH_CHECK("decode_attn_dense fp32 partials");
-    dec32_merge_kernel<64><<<g2, 64 * D_WAVES, 0, st>>>(P);
-  } else {
-    dec32_partial_kernel<128><<<g1, 64 * D_WAVES, 0, st>>>(P);
-    FSI_HIP_LAUNCH_CHECK("decode_attn_dense fp32 partials");
-    dec32_merge_kernel<128><<<g2, 64 * D_WAVES, 0, st>>>(P);
-  }
-  FSI_HIP_LAUNCH_CHECK("decode_attn_dense fp32 merge");
+  auto launch = [&](auto hd_tag) {
+    constexpr int HD = decltype(hd_tag)::value;
+    const int64_t rows = B * Hq;
+    if (small) {
+      dec32_partial_kernel<HD, D_SPLIT_SMALL><<<g1, 64 * D_WAVES, 0, st>>>(P);
+      dec32_merge_kernel<HD, D_WAVES><<<static_cast<unsigned>(rows), 64 * D_WAVES, 0, st>>>(P, split);
+    } else {
+      dec32_partial_kernel<HD, D_SPLIT><<<g1, 64 * D_WAVES, 0, st>>>(P);
+      dec32_merge_kernel<HD, 1><<<static_cast<unsigned>((rows + D_WAVES - 1) / D_WAVES), 64 * D_WAVES, 0, st>>>(P, split);
+    }
+  };
+  if (head_dim == 64) launch(std::integral_constant<int, 64>{});
+  else launch(std::integral_constant<int, 128>{});
+  FSI_HIP_LAUNCH_CHECK("decode_attn_dense fp32");
   return FSI_OK;
 }
 
