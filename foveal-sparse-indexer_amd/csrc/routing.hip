@@ -13,14 +13,15 @@
 //   2. every candidate gets an order-preserving 32-bit key (prob bits + 1;
 //      0 = not a candidate; probabilities are >= 0 so their bit patterns sort
 //      like the values);
-//   3. the R-th largest key T is found exactly by bisection over key values;
+//   3. the R-th largest key T is found exactly by bisection over key values (long
+//      rows: over the few hundred keys that can be among the R);
 //      keys > T are taken and the rest of the R come from keys == T in
 //      ascending index order;
 //   4. the R winners are sorted by (prob desc, index asc) with a bitonic network
 //      across lanes and register slots;
-//   5. their running mass is accumulated sequentially in fp64 and rounded to
-//      fp32 per element (ATen's CPU cumsum of fp32 accumulates in double), and
-//      the reference's count rule is applied.
+//   5. their running mass is accumulated in fp64, with the sums of the sequential
+//      order, and rounded to fp32 per element (ATen's CPU cumsum of fp32
+//      accumulates in double), and the reference's count rule is applied.
 // torch.sort leaves the order of equal probabilities unspecified; lower index
 // first is used here.  That, and ulp-level exp/sum differences, are the only
 // ways a selection can differ from the CPU reference (near-ties).
@@ -198,20 +199,108 @@ __device__ __forceinline__ void sort_taken(int R, uint64_t (&out)[E], const uint
   bitonic_desc<E>(out);
 }
 
+// Slots of the dense candidate list that rank_top searches instead of a long row,
+// and the (key, index) entries its scratch holds (one 64-lane write of slack).
+constexpr int CAND_SLOTS = 8;
+constexpr int CAND_ENTRIES = 64 * CAND_SLOTS + 64;
+// Shortest rows, in slots of 64 keys, that are compacted: with 16 slots the passes saved
+// pay for little more than the compaction (8000 rows of 1024 keys 36.5 us without, 36.0 with).
+constexpr int CAND_MIN_PL = 32;
+
 // The R largest keys (0 < R <= min(64 E, #candidates)), sorted descending into
 // out[] (element k at lane k % 64, slot k / 64); entries k >= R hold 0.
-// lds_k / lds_i: this wave's 64 E words each.
+// lds_k / lds_i: this wave's 64 E words each.  cand (optional): CAND_ENTRIES
+// entries of this wave.
+//
+// Every pass over the keys is 2 VALU operations a slot, so a bisection of ten-odd
+// counts over 64 slots is most of the ranking.  With cand and R <= 64 the keys
+// at or above the smallest lane maximum (at least 64 of them; about 300 of 4096
+// keys in random order) are first compacted in index order, and the search runs
+// over CAND_SLOTS slots.  Rows with more keys than that at the top, or with a lane
+// of no key, take the whole row.  With div_by and the prefix scan of running_mass:
+// 8192 rows of 4096 keys, 64 ranked, 160 -> 130 us; 2 x 2000 rows of 2000 keys 39.6 ->
+// 32.4 us.  Still bound by VALU issue, at two waves per SIMD (64 keys a lane).
 template <int PL, int E>
-__device__ void rank_top(const uint32_t (&key)[PL], int R, uint64_t (&out)[E], uint32_t* lds_k, uint32_t* lds_i) {
+__device__ __forceinline__ void rank_top(const uint32_t (&key)[PL], int R, uint64_t (&out)[E], uint32_t* lds_k, uint32_t* lds_i,
+                         uint2* cand = nullptr) {
   const int lane = lane_id();
 #pragma unroll
   for (int e = 0; e < E; ++e) out[e] = 0;
   if (R <= 0) return;
   uint32_t T;
   int clo;
+  if constexpr (PL > CAND_SLOTS) {
+    if (cand != nullptr && R <= 64) {  // uniform
+      uint32_t mn = 0;
+#pragma unroll
+      for (int i = 0; i < PL; ++i) mn = key[i] > mn ? key[i] : mn;
+      for (int off = 32; off > 0; off >>= 1) {
+        const uint32_t o = __shfl_xor(mn, off, 64);
+        mn = o < mn ? o : mn;
+      }
+      mn = __builtin_amdgcn_readfirstlane(mn);
+      int base = 0;
+      if (mn > 0) {
+#pragma unroll
+        for (int i = 0; i < PL; ++i) {
+          const bool take = key[i] >= mn;
+          const uint64_t m = __ballot(take);
+          if (base <= 64 * CAND_SLOTS && take)
+            cand[base + lanes_below(m)] = make_uint2(key[i], static_cast<uint32_t>(i * 64 + lane));
+          base += __popcll(m);
+        }
+      }
+      if (base > 0 && base <= 64 * CAND_SLOTS) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        uint32_t ck[CAND_SLOTS], ci[CAND_SLOTS];
+#pragma unroll
+        for (int i = 0; i < CAND_SLOTS; ++i) {
+          const uint2 c = cand[i * 64 + lane];
+          ck[i] = i * 64 + lane < base ? c.x : 0u;
+          ci[i] = c.y;
+        }
+        top_threshold<CAND_SLOTS>(ck, R, T, clo);
+        take_top<CAND_SLOTS>(ck, R, T, clo, lds_k, lds_i, [&](int i) { return ci[i]; });
+        sort_taken<E>(R, out, lds_k, lds_i);
+        return;
+      }
+    }
+  }
   top_threshold<PL>(key, R, T, clo);
   take_top<PL>(key, R, T, clo, lds_k, lds_i, [&](int i) { return static_cast<uint32_t>(i * 64 + lane); });
   sort_taken<E>(R, out, lds_k, lds_i);
+}
+
+// x / d, correctly rounded, from r = the correctly rounded 1 / d: the first step makes
+// the quotient faithful, the second rounds it (Markstein's theorem).  Holds
+// while neither the quotient nor a remainder (a multiple of 2^-47 x) leaves the normal
+// range; the callers check |x| >= 2^-60 or x = 0 and 2^-40 <= d <= 2^20.
+__device__ __forceinline__ float div_by(float x, float d, float r) {
+  float q = x * r;
+  q = fmaf(fmaf(-d, q, x), r, q);
+  return fmaf(fmaf(-d, q, x), r, q);
+}
+constexpr float DIV_MIN_X = 0x1p-60f, DIV_MIN_D = 0x1p-40f, DIV_MAX_D = 0x1p20f;
+
+// v[c] / nrm for the components of a key (nrm = its norm, so |v[c]| <= about nrm).
+template <int D>
+__device__ __forceinline__ void normalise(float (&v)[D], float nrm) {
+  uint32_t mn = 0xffffffffu;  // smallest non-zero magnitude (zero wraps to the largest)
+#pragma unroll
+  for (int c = 0; c < D; ++c) {
+    const uint32_t m = (__float_as_uint(v[c]) << 1) - 1u;
+    mn = m < mn ? m : mn;
+  }
+  if (mn >= (__float_as_uint(DIV_MIN_X) << 1) - 1u && nrm >= DIV_MIN_D && nrm <= DIV_MAX_D) {
+    const float r = 1.f / nrm;
+#pragma unroll
+    for (int c = 0; c < D; ++c) v[c] = div_by(v[c], nrm, r);
+  } else {
+#pragma unroll
+    for (int c = 0; c < D; ++c) v[c] = v[c] / nrm;
+  }
 }
 
 // Running mass of the sorted probabilities for k < n; 0 elsewhere.
@@ -222,6 +311,24 @@ __device__ void rank_top(const uint32_t (&key)[PL], int R, uint64_t (&out)[E], u
 template <int E, bool RB>
 __device__ __forceinline__ void running_mass(const uint64_t (&sorted)[E], int n, float (&cum)[E]) {
   const int lane = lane_id();
+  if constexpr (E == 1 && !RB) {
+    // No fp64 sum rounds while every p is a multiple of 2^-24 p_min and the total stays
+    // below 2^29 p_min, so any order gives the sequential result: a prefix scan of
+    // 6 steps instead of n.
+    const float p = comp_prob(sorted[0]);
+    const float top = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p), 0));
+    const float low = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p), n > 0 && n <= 64 ? n - 1 : 0));
+    if (n > 0 && n <= 64 && low >= 0x1p-100f && low >= 0x1p-20f * top && top <= 1.f) {  // uniform
+      double x = lane < n ? static_cast<double>(p) : 0.0;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const double y = __shfl_up(x, off, 64);
+        x += lane >= off ? y : 0.0;
+      }
+      cum[0] = lane < n ? static_cast<float>(x) : 0.f;
+      return;
+    }
+  }
   double acc = 0.0;
   float accf = 0.f;
 #pragma unroll
@@ -294,9 +401,10 @@ struct SelectParams {
 // (core.py:43,103,111 evaluated in bfloat16).  Writes indices[capacity], count
 // and (optionally) mass = local mass + cum[count-1].
 template <int PL, int E, bool RB>
-__device__ void select_row(float (&s)[PL], int N, int qb, int64_t row, const SelectParams& sp,
+__device__ __forceinline__ void select_row(float (&s)[PL], int N, int qb, int64_t row, const SelectParams& sp,
                            int32_t* __restrict__ out_idx, int32_t* __restrict__ out_cnt,
-                           float* __restrict__ out_mass, uint32_t* lds_k, uint32_t* lds_i) {
+                           float* __restrict__ out_mass, uint32_t* lds_k, uint32_t* lds_i,
+                           uint2* cand) {
   const int lane = lane_id();
   const float top_p = sp.top_p_rows ? sp.top_p_rows[row] : sp.top_p;
   const int k_min = sp.k_min_rows ? sp.k_min_rows[row] : sp.k_min;
@@ -322,11 +430,24 @@ __device__ void select_row(float (&s)[PL], int N, int qb, int64_t row, const Sel
       z += s[i];
     }
     z = fmaxf(wave_sum(z), 1e-20f);
+    float small = s[0];
 #pragma unroll
-    for (int i = 0; i < PL; ++i) {
-      float p = s[i] / z;
-      if (RB) p = round_bf16(p);
-      key[i] = __float_as_uint(p) + 1u;
+    for (int i = 1; i < PL; ++i) small = fminf(small, s[i]);
+    if (__all(small >= DIV_MIN_X) && z >= 1.f && z <= DIV_MAX_D) {  // uniform
+      const float r = 1.f / z;
+#pragma unroll
+      for (int i = 0; i < PL; ++i) {
+        float p = div_by(s[i], z, r);
+        if (RB) p = round_bf16(p);
+        key[i] = __float_as_uint(p) + 1u;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < PL; ++i) {
+        float p = s[i] / z;
+        if (RB) p = round_bf16(p);
+        key[i] = __float_as_uint(p) + 1u;
+      }
     }
     avail = 64 * PL;
   } else {
@@ -365,7 +486,7 @@ __device__ void select_row(float (&s)[PL], int N, int qb, int64_t row, const Sel
   R = R < avail ? R : avail;
   R = R < 64 * E ? R : 64 * E;  // the host guarantees this does not truncate
   uint64_t sorted[E];
-  rank_top<PL, E>(key, R, sorted, lds_k, lds_i);
+  rank_top<PL, E>(key, R, sorted, lds_k, lds_i, cand);
 
   // counts (core.py:107-119)
   const float target = RB ? fmaxf(round_bf16(round_bf16(top_p) - lmass), 0.0f) : fmaxf(top_p - lmass, 0.0f);
@@ -428,6 +549,7 @@ __global__ __launch_bounds__(64 * RS_WAVES) void route_scores_kernel(const void*
                                                                      int32_t* __restrict__ out_cnt,
                                                                      float* __restrict__ out_mass) {
   __shared__ uint32_t lk[RS_WAVES][64 * E], li[RS_WAVES][64 * E];
+  __shared__ uint2 cand[CAND_MIN_PL <= PL ? RS_WAVES : 1][CAND_MIN_PL <= PL ? CAND_ENTRIES : 1];
   const int wave = threadIdx.x >> 6, lane = lane_id();
   const int64_t row = static_cast<int64_t>(blockIdx.x) * RS_WAVES + wave;
   if (row >= n_rows) return;  // whole wave leaves; no workgroup barrier follows
@@ -438,8 +560,8 @@ __global__ __launch_bounds__(64 * RS_WAVES) void route_scores_kernel(const void*
     if (BF16) s[i] = j < N ? bf16_to_f32(static_cast<const bf16_t*>(scores)[row * N + j]) : 0.f;
     else s[i] = j < N ? static_cast<const float*>(scores)[row * N + j] : 0.f;
   }
-  select_row<PL, E, BF16>(s, N, static_cast<int>(row % Qb), row, sp, out_idx, out_cnt, out_mass, lk[wave],
-                          li[wave]);
+  select_row<PL, E, BF16>(s, N, static_cast<int>(row % Qb), row, sp, out_idx, out_cnt, out_mass, lk[wave], li[wave],
+                          CAND_MIN_PL <= PL ? cand[wave] : nullptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -536,10 +658,9 @@ __global__ __launch_bounds__(64 * SR_WAVES) void score_route_kernel(const void* 
 #pragma unroll
         for (int c = 0; c < SR_D; ++c) v[c] = 0.f;
       }
-      const float nrm = fmaxf(sqrtf(ss), 1e-12f);
+      normalise(v, fmaxf(sqrtf(ss), 1e-12f));
 #pragma unroll
-      for (int w = 0; w < 4; ++w)
-        kn[w][t] = make_float4(v[4 * w] / nrm, v[4 * w + 1] / nrm, v[4 * w + 2] / nrm, v[4 * w + 3] / nrm);
+      for (int w = 0; w < 4; ++w) kn[w][t] = make_float4(v[4 * w], v[4 * w + 1], v[4 * w + 2], v[4 * w + 3]);
     }
     __syncthreads();
 #pragma unroll
@@ -569,9 +690,13 @@ __global__ __launch_bounds__(64 * SR_WAVES) void score_route_kernel(const void* 
 #pragma unroll
     for (int i = 0; i < PL; ++i) sa[i] /= sqrt_d;
   }
+  // the key chunk's LDS is free once every wave has scored: the candidate lists take it
+  static_assert(sizeof(uint2) * CAND_ENTRIES * SR_WAVES <= sizeof(kn), "candidate lists fit the key chunk");
+  if constexpr (CAND_MIN_PL <= PL) __syncthreads();
   if (row_q < Q)
-    select_row<PL, E, false>(sa, N, row_q, static_cast<int64_t>(b) * Q + row_q, sp, out_idx, out_cnt, out_mass, lk[wave],
-                      li[wave]);
+    select_row<PL, E, false>(
+        sa, N, row_q, static_cast<int64_t>(b) * Q + row_q, sp, out_idx, out_cnt, out_mass, lk[wave], li[wave],
+        CAND_MIN_PL <= PL ? reinterpret_cast<uint2*>(&kn[0][0]) + wave * CAND_ENTRIES : nullptr);
 }
 
 // ---------------------------------------------------------------------------
