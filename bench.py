@@ -213,8 +213,8 @@ def bench_routing(fsi, args, dev):
                        "valu_issue": {"achieved": round(gips, 1), "peak": VALU_PEAK_GIPS,
                                       "unit": "G VALU wave-instructions/s", "frac": round(gips / VALU_PEAK_GIPS, 4),
                                       "valu_insts_per_launch": C2_VALU_INSTS},
-                       "note": "not HBM-bound: 33.5 M scores, exps and a top-64 rank per launch; the rank "
-                               "(threshold bisection) takes most of the VALU issue"}
+                       "note": "not HBM-bound: 33.5 M scores, exps and a top-64 rank per launch; exps, "
+                               "scores and the rank share the VALU issue"}
     if not args.no_cpu_baseline:
         from oracle import routing as R
 
@@ -452,8 +452,8 @@ def bench_prefill_attn(fsi, args, dev):
     res["backward"] = {"ms": round(bwd_ms, 3), "tflops": round(bwd_tf, 1), "peak": BF16_PEAK_TFLOPS,
                        "frac": round(bwd_tf / BF16_PEAK_TFLOPS, 4),
                        "flops": int(2.5 * flops), "kernel": "sab_map + sab_q_bf (statistics, dQ) + sab_kv_bf (dK, dV)",
-                       "note": "every product on v_mfma_f32_16x16x32_bf16 over bf16 LDS tiles (row-major and "
-                               "transposed); P and dS enter dV / dK / dQ as bf16 hi + lo pairs (~2^-17 relative), "
+                       "note": "every product on v_mfma_f32_16x16x32_bf16 over bf16 LDS tiles (direct-to-LDS; "
+                               "transposed operands by ds_read_b64_tr_b16); P and dS enter dV / dK / dQ as bf16 hi + lo pairs (~2^-17 relative), "
                                "fp32 accumulation; memory O(T hd), no (T, T) tensor"}
     res["roofline"] = {"bound": "mfma", "achieved": round(tfs, 1), "peak": BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                        "frac": round(tfs / BF16_PEAK_TFLOPS, 4), "traffic": PREFILL_ATTN_TRAFFIC_BYTES,

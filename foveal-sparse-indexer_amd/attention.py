@@ -852,8 +852,8 @@ class FovealSparseAttention(nn.Module):
     The prefill `forward` routes with the HIP indexer ops and runs one
     block-sparse attention launch (`sparse_attention`).  Both paths take the
     reference's dtypes (fp32 by default, bf16) and are differentiable: the
-    attention backward recomputes the sparse pattern densely (as the reference's
-    forward does), decode's gradient reaches q (the cache is inference state).
+    attention backward walks the sparse pattern in HIP kernels (head_dim up to
+    128; wider heads recompute it densely), decode's gradient reaches q (the cache is inference state).
     """
 
     def __init__(

@@ -4,8 +4,9 @@ Same names, signatures, defaults and return structures as the reference
 (`Route` core.py:23-33, `masked_softmax` :36-43, `select_blocks` :46-160,
 `FovealIndexer` :163-353).  Softmax, ranking, prefix mass, counts, scoring,
 pooling and the additive-stream contraction run in the HIP library
-(csrc/routing.hip, csrc/indexer.hip); the D -> 16 projections are library
-GEMMs (nn.Linear).  masked_softmax and the FovealIndexer representations
+(csrc/routing.hip, csrc/indexer.hip), and so do the D -> 16 projections and the
+stream's expansion of plain nn.Linear modules (csrc/index_proj.hip; other
+modules are called as they are).  masked_softmax and the FovealIndexer representations
 (compute_query_16d, compute_kv_blocks_16d, compute_block_scores,
 additive_stream) are differentiable through HIP backward kernels, as the
 reference's dual-gradient training needs (tests/test_indexer.py:63-101);

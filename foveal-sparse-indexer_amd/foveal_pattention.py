@@ -11,7 +11,8 @@ active-block cache and forward signature as the reference
     (fused SwiGLU, one rounding of silu(g)*u; :281-282) and its eager path
     otherwise (silu(g) and the product rounded separately; :283-284).
   * Training mode follows the reference's per-token routing and additive stream
-    with library GEMMs around the HIP SwiGLU forward / backward kernels.
+    with library GEMMs between the HIP router, gather / scatter and SwiGLU
+    kernels (csrc/mlp_train.hip).
 """
 from __future__ import annotations
 
