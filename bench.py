@@ -69,7 +69,7 @@ C5_TRAFFIC_BYTES = {0.10: (515 + 64) << 20, 0.25: (1175 + 64) << 20, 0.50: (2249
 # (873685.9 + 16425.7 + 16507.2) KiB x 1.99983 read + (131285.4 + 32 + 32768.1) KiB written
 PREFILL_ATTN_TRAFFIC_BYTES = int(906618.8 * 1.99983 * 1024 + 164085.5 * 1024)
 # C2: wave-level VALU instructions of one score_route_kernel launch (rocprofv3 SQ_INSTS_VALU)
-C2_VALU_INSTS = 70_114_379
+C2_VALU_INSTS = 47_169_428
 VALU_PEAK_GIPS = 256 * 4 * 2.4 / 4  # G wave64 VALU instructions/s: 256 CUs x 4 SIMDs x 2.4 GHz / 4 cycles
 
 

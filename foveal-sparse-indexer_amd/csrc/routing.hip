@@ -218,7 +218,8 @@ constexpr int CAND_MIN_PL = 32;
 // keys in random order) are first compacted in index order, and the search runs
 // over CAND_SLOTS slots.  Rows with more keys than that at the top, or with a lane
 // of no key, take the whole row.  With div_by and the prefix scan of running_mass:
-// 8192 rows of 4096 keys, 64 ranked, 160 -> 130 us; 2 x 2000 rows of 2000 keys 39.6 ->
+// 8192 rows of 4096 keys, 64 ranked, 160 -> 124-130 us (70.1 ->
+// 47.2 M VALU instructions); 2 x 2000 rows of 2000 keys 39.6 ->
 // 32.4 us.  Still bound by VALU issue, at two waves per SIMD (64 keys a lane).
 template <int PL, int E>
 __device__ __forceinline__ void rank_top(const uint32_t (&key)[PL], int R, uint64_t (&out)[E], uint32_t* lds_k, uint32_t* lds_i,
