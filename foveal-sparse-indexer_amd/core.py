@@ -27,6 +27,7 @@ from typing import Optional, Tuple
 
 import torch
 from torch import Tensor, nn
+from torch._subclasses.fake_tensor import FakeTensor
 
 from . import _lib
 
@@ -467,7 +468,8 @@ class _DistillKLFn(torch.autograd.Function):
 def _plain_linear(m: nn.Module, x: Tensor) -> bool:
     """Whether m(x) is nothing but x W^T in x's type: a plain nn.Linear without bias or hooks
     over 16 features on one side, outside autocast (which picks the type)."""
-    return (type(m) is nn.Linear and m.bias is None and type(m.weight) is nn.Parameter and m.weight.dtype == x.dtype
+    return (type(m) is nn.Linear and m.bias is None and type(m.weight) in (nn.Parameter, FakeTensor)
+            and m.weight.dtype == x.dtype
             and x.dtype in (torch.float32, torch.bfloat16) and x.is_cuda and m.weight.device == x.device
             and 16 in m.weight.shape
             and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)

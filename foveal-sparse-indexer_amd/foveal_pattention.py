@@ -26,6 +26,7 @@ import torch.nn.functional as F
 from torch import Tensor, nn
 
 from . import _lib
+from .core import _plain_linear
 from .pattention import (
     FusedSwiGLUFunction,
     PACKED_PREFILL_MIN_M,
@@ -140,6 +141,14 @@ class _SavedGU:
 # -- training path on the HIP kernels of csrc/mlp_train.hip -----------------------------
 
 
+def _check_route_operands(q: Tensor, keys: Tensor, what: str) -> None:
+    """The kernels read both as rows of 16 values of one type."""
+    if q.dtype != keys.dtype:
+        raise TypeError(f"{what}: dtype mismatch {q.dtype}/{keys.dtype}")
+    if q.dim() != 2 or keys.dim() != 2 or q.shape[1] != 16 or keys.shape[1] != 16:
+        raise ValueError(f"{what}: queries {tuple(q.shape)} and keys {tuple(keys.shape)} (rows of 16)")
+
+
 def _train_route_fake(q, keys, base, remote, temperature):
     return (q.new_empty((q.shape[0], keys.shape[0])), torch.empty_like(q),
             q.new_empty((base + remote,), dtype=torch.int32))
@@ -150,6 +159,7 @@ def _train_route_op(q: Tensor, keys: Tensor, base: int, remote: int,
                     temperature: float) -> Tuple[Tensor, Tensor, Tensor]:
     """fsi_mlp_train_route: (scores (M, n_blocks), context (M, 16), active blocks int32)."""
     what = "FovealPattentionMLP training routing"
+    _check_route_operands(q, keys, what)
     dev = _lib.require_gpu(q, keys, what=what)
     q, keys = q.contiguous(), keys.contiguous()
     M, nb = q.shape[0], keys.shape[0]
@@ -172,7 +182,8 @@ def _train_route_bwd_op(q: Tensor, keys: Tensor, dscores: Optional[Tensor], dctx
                         temperature: float) -> Tuple[Tensor, Tensor]:
     """fsi_mlp_train_route_bwd: (dq, dkeys)."""
     what = "FovealPattentionMLP training routing backward"
-    dev = _lib.require_gpu(q, keys, what=what)
+    _check_route_operands(q, keys, what)
+    dev = _lib.require_gpu(q, keys, dscores, dctx, what=what)
     q, keys = q.contiguous(), keys.contiguous()
     ds = dscores.to(q.dtype).contiguous() if dscores is not None else None
     dc = dctx.to(q.dtype).contiguous() if dctx is not None else None
@@ -758,13 +769,17 @@ class FovealPattentionMLP(nn.Module):
 
     def _train_fused(self, x_2d: Tensor) -> bool:
         """Whether the training forward runs on csrc/mlp_train.hip: the fused SwiGLU (the eager
-        one rounds in between), one dtype, a 16-D index over at most 256 blocks, rows and
+        one rounds in between), one dtype, queries from a plain linear layer (a hook or a
+        wrapper may give another type), a 16-D index over at most 256 blocks, rows and
         blocks of whole 16-byte vectors, and no autocast (which picks each op's type)."""
         dt = x_2d.dtype
-        weights = (self.k_gate, self.k_up, self.v, self.q_proj_16d.weight, self.block_keys_16d)
+        weights = (self.k_gate, self.k_up, self.v, self.block_keys_16d)
         return (self.use_fused_kernel and dt in (torch.bfloat16, torch.float32)
                 and all(w.dtype == dt and w.is_cuda for w in weights)
+                and _plain_linear(self.q_proj_16d, x_2d)
+                and tuple(self.q_proj_16d.weight.shape) == (16, self.hidden_dim)
                 and self.index_dim == 16 and self.num_blocks <= 256 and x_2d.shape[0] > 0
+                and tuple(self.block_keys_16d.shape) == (self.num_blocks, 16)
                 and 0 < self.total_active_blocks and 0 <= self.base_blocks
                 and 0 <= self.remote_blocks <= self.num_blocks - self.base_blocks
                 and self.hidden_dim % 8 == 0 and self.block_size % 8 == 0 and self.temperature > 0

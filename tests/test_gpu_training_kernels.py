@@ -125,3 +125,11 @@ def test_training_nan_tokens_route_in_range(fsi, dev):
     _, info = m(x, return_router_info=True)
     active = info["active_blocks"].tolist()
     assert len(set(active)) == 8 and 0 <= min(active) and max(active) < 24
+
+
+def test_training_queries_of_another_type(fsi, dev):
+    """A hook that widens the projected queries over bf16 keys is refused, as torch.matmul does."""
+    m, x, _ = _module(fsi, (64, 16, 24, 2, 6, 40), torch.bfloat16, dev)
+    m.q_proj_16d.register_forward_hook(lambda mod, a, out: out.float())
+    with pytest.raises(RuntimeError):
+        m(x)

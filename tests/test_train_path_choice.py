@@ -1,0 +1,76 @@
+"""Which FovealPattentionMLP training calls the fused kernels take (CPU only: FakeTensor
+tracing of the forward, no kernel runs).  Whatever the module's owner puts in the place of a
+part that the fused path would pass by keeps the torch form, which calls it."""
+import pytest
+import torch
+from torch import nn
+from torch._subclasses.fake_tensor import FakeTensorMode
+from torch.utils._python_dispatch import TorchDispatchMode
+
+
+class _Ops(TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.names = []
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.names.append(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+def _traced(fsi, change=None, dtype=torch.bfloat16):
+    """Names of the ops of one training forward after change(module)."""
+    with FakeTensorMode(), torch.device("cuda"):
+        m = fsi.FovealPattentionMLP(hidden_dim=256, intermediate_dim=1024, base_blocks=2, remote_blocks=4,
+                                    dtype=dtype).train()
+        if change is not None:
+            change(m)
+        with _Ops() as ops:
+            m(torch.empty(2, 8, 256, dtype=dtype))
+    return ops.names
+
+
+def _fused(names):
+    return any("fsi.mlp_train_route" in n for n in names)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
+def test_plain_module_is_fused(fsi, dtype):
+    assert _fused(_traced(fsi, dtype=dtype))
+
+
+def test_hooked_projection_keeps_torch_ops(fsi):
+    """A hook that returns fp32 queries over bf16 keys: torch.matmul decides on the pair; the
+    kernel would read the keys as fp32, past their end."""
+    assert not _fused(_traced(fsi, lambda m: m.q_proj_16d.register_forward_hook(lambda mod, a, out: out.float())))
+
+
+def test_route_op_refuses_mixed_operands(fsi):
+    route, bwd = fsi.foveal_pattention._train_route_op, fsi.foveal_pattention._train_route_bwd_op
+    q, keys = torch.zeros(3, 16), torch.zeros(4, 16)
+    for args in ((q, keys.bfloat16()), (q.bfloat16(), keys)):
+        with pytest.raises(TypeError, match="dtype mismatch"):
+            route(*args, 1, 2, 1.0)
+        with pytest.raises(TypeError, match="dtype mismatch"):
+            bwd(*args, None, None, 1.0)
+    for args in ((q[:, :8], keys), (q, keys[:, :8])):
+        with pytest.raises(ValueError, match="rows of 16"):
+            route(*args, 1, 2, 1.0)
+
+
+class _Wrapped(nn.Module):
+    """A projection without a weight of its own."""
+
+    def __init__(self, inner):
+        super().__init__()
+        self.inner = inner
+
+    def forward(self, x):
+        return self.inner(x) * 2
+
+
+def test_wrapped_projection_is_called(fsi):
+    def wrap(m):
+        m.q_proj_16d = _Wrapped(m.q_proj_16d)
+
+    assert not _fused(_traced(fsi, wrap))
