@@ -770,11 +770,14 @@ class FovealPattentionMLP(nn.Module):
     def _train_fused(self, x_2d: Tensor) -> bool:
         """Whether the training forward runs on csrc/mlp_train.hip: the fused SwiGLU (the eager
         one rounds in between), one dtype, queries from a plain linear layer (a hook or a
-        wrapper may give another type), a 16-D index over at most 256 blocks, rows and
-        blocks of whole 16-byte vectors, and no autocast (which picks each op's type)."""
+        wrapper may give another type), the class's own router scores, a 16-D index over at
+        most 256 blocks, rows and blocks of whole 16-byte vectors, and no autocast (which
+        picks each op's type)."""
         dt = x_2d.dtype
         weights = (self.k_gate, self.k_up, self.v, self.block_keys_16d)
         return (self.use_fused_kernel and dt in (torch.bfloat16, torch.float32)
+                and type(self).compute_router_scores is _ROUTER_SCORES
+                and "compute_router_scores" not in self.__dict__
                 and all(w.dtype == dt and w.is_cuda for w in weights)
                 and _plain_linear(self.q_proj_16d, x_2d)
                 and tuple(self.q_proj_16d.weight.shape) == (16, self.hidden_dim)
@@ -816,6 +819,11 @@ class FovealPattentionMLP(nn.Module):
                 "sparsity": (1.0 - self.total_active_blocks / self.num_blocks) * 100.0,
             }
         return out
+
+
+# What the fused training path computes in place of a call: a subclass, an instance or the
+# class itself may hold another (noise, a balancing bias), which is then called.
+_ROUTER_SCORES = FovealPattentionMLP.compute_router_scores
 
 
 def release_unpacked_weights(model: nn.Module) -> int:

@@ -74,3 +74,26 @@ def test_wrapped_projection_is_called(fsi):
         m.q_proj_16d = _Wrapped(m.q_proj_16d)
 
     assert not _fused(_traced(fsi, wrap))
+
+
+def _biased(self, x):
+    self.calls = getattr(self, "calls", 0) + 1
+    return torch.matmul(self.q_proj_16d(x), self.block_keys_16d.t()) + 1.0
+
+
+@pytest.mark.parametrize("where", ["subclass", "instance", "class"])
+def test_replaced_router_scores_are_called(fsi, where, monkeypatch):
+    """compute_router_scores is what the training forward routes on, whoever replaced it."""
+    seen = []
+
+    def change(m):
+        if where == "subclass":
+            m.__class__ = type("Biased", (fsi.FovealPattentionMLP,), {"compute_router_scores": _biased})
+        elif where == "instance":
+            m.compute_router_scores = _biased.__get__(m)
+        else:
+            monkeypatch.setattr(fsi.FovealPattentionMLP, "compute_router_scores", _biased)
+        seen.append(m)
+
+    assert not _fused(_traced(fsi, change))
+    assert seen[0].calls == 1
