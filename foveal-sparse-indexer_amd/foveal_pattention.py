@@ -770,7 +770,8 @@ class FovealPattentionMLP(nn.Module):
     def _train_fused(self, x_2d: Tensor) -> bool:
         """Whether the training forward runs on csrc/mlp_train.hip: the fused SwiGLU (the eager
         one rounds in between), one dtype, queries from a plain linear layer (a hook or a
-        wrapper may give another type), the class's own router scores, a 16-D index over at
+        wrapper may give another type), the class's own router scores, a temperature that is a
+        number (a tensor has a gradient) whose reciprocal fp32 holds, a 16-D index over at
         most 256 blocks, rows and blocks of whole 16-byte vectors, and no autocast (which
         picks each op's type)."""
         dt = x_2d.dtype
@@ -785,7 +786,8 @@ class FovealPattentionMLP(nn.Module):
                 and tuple(self.block_keys_16d.shape) == (self.num_blocks, 16)
                 and 0 < self.total_active_blocks and 0 <= self.base_blocks
                 and 0 <= self.remote_blocks <= self.num_blocks - self.base_blocks
-                and self.hidden_dim % 8 == 0 and self.block_size % 8 == 0 and self.temperature > 0
+                and self.hidden_dim % 8 == 0 and self.block_size % 8 == 0
+                and isinstance(self.temperature, (int, float)) and 1e-30 <= self.temperature <= 1e30
                 and self.intermediate_dim % self.block_size == 0
                 and tuple(self.v.shape) == tuple(self.k_gate.shape)
                 and not torch.is_autocast_enabled("cuda"))

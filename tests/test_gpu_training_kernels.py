@@ -133,3 +133,16 @@ def test_training_queries_of_another_type(fsi, dev):
     m.q_proj_16d.register_forward_hook(lambda mod, a, out: out.float())
     with pytest.raises(RuntimeError):
         m(x)
+
+
+def test_training_learnable_temperature(fsi, dev):
+    """A temperature parameter gets the gradient of softmax(scores / T)."""
+    m, x, dy = _module(fsi, (64, 16, 24, 2, 6, 40), torch.float32, dev)
+    m.temperature = torch.nn.Parameter(torch.tensor(0.7, device=dev))
+    out, info = m(x, return_router_info=True)
+    (got,) = torch.autograd.grad(out, [m.temperature], dy)
+    t = m.temperature.detach().double().requires_grad_()
+    w = {n: p.detach() for n, p in m.named_parameters()}
+    ref = torch.softmax(info["scores"].detach().double() / t, -1) @ w["block_keys_16d"].double()
+    (want,) = torch.autograd.grad(ref @ w["out_proj_16d.weight"].double().t(), [t], dy.double())
+    assert _close(got, want, 1e-4)

@@ -97,3 +97,23 @@ def test_replaced_router_scores_are_called(fsi, where, monkeypatch):
 
     assert not _fused(_traced(fsi, change))
     assert seen[0].calls == 1
+
+
+@pytest.mark.parametrize("temperature", ["parameter", "tensor", 0.0, -1.0, 1e-50, float("inf"), float("nan")])
+def test_temperature_keeps_torch_ops(fsi, temperature):
+    """A learnable or tensor temperature has its gradient through scores / temperature; numbers
+    whose reciprocal fp32 does not hold divide in torch."""
+    def change(m):
+        if temperature == "parameter":
+            m.temperature = nn.Parameter(torch.ones(()))
+        elif temperature == "tensor":
+            m.temperature = torch.ones((), requires_grad=True)
+        else:
+            m.temperature = temperature
+
+    assert not _fused(_traced(fsi, change))
+
+
+@pytest.mark.parametrize("temperature", [1, 0.5])
+def test_number_temperature_is_fused(fsi, temperature):
+    assert _fused(_traced(fsi, lambda m: setattr(m, "temperature", temperature)))
