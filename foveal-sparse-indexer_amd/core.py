@@ -543,7 +543,8 @@ def _proj_dw_op(x: Tensor, g0: Tensor, g1: Optional[Tensor]) -> Tuple[Tensor, Te
 
 
 class _Proj16Fn(torch.autograd.Function):
-    """(x w0^T, x w1^T) over (.., D) x in one pass, w0 and w1 (16, D); w1 may be None."""
+    """(x w0^T, x w1^T) over (.., D) x in one pass, w0 and w1 (16, D); w1 may be None.  A
+    backward that is itself differentiated forms its products in torch."""
 
     @staticmethod
     def forward(ctx, x: Tensor, w0: Tensor, w1: Optional[Tensor]):
@@ -553,16 +554,19 @@ class _Proj16Fn(torch.autograd.Function):
         return (y0, y1) if w1 is not None else (y0, None)
 
     @staticmethod
-    @torch.autograd.function.once_differentiable
     def backward(ctx, g0: Optional[Tensor], g1: Optional[Tensor]):
         x, w0, w1 = ctx.saved_tensors
         need_x, need0, need1 = ctx.needs_input_grad
+        want0, want1 = need0 and g0 is not None, need1 and g1 is not None
         dx = dw0 = dw1 = None
-        if g0 is not None and need0 and g1 is not None and need1:
+        if torch.is_grad_enabled():
+            product = lambda g: torch.matmul(g.reshape(-1, 16).t(), x.reshape(-1, x.shape[-1]))  # noqa: E731
+            dw0, dw1 = product(g0) if want0 else None, product(g1) if want1 else None
+        elif want0 and want1:
             dw0, dw1 = _proj_dw_op(x, g0, g1)
-        elif g0 is not None and need0:
+        elif want0:
             dw0 = _proj_dw_op(x, g0, None)[0]
-        elif g1 is not None and need1:
+        elif want1:
             dw1 = _proj_dw_op(x, g1, None)[0]
         if need_x:
             for g, w in ((g0, w0), (g1, w1)):
@@ -607,7 +611,8 @@ def _expand_bwd_op(dy: Tensor, ctx16: Tensor, w: Tensor, block: int) -> Tuple[Te
 
 
 class _Expand16Fn(torch.autograd.Function):
-    """out_proj of the block context, repeated over each block's elements (core.py:310-312)."""
+    """out_proj of the block context, repeated over each block's elements (core.py:310-312).  A
+    backward that is itself differentiated forms its sums and products in torch."""
 
     @staticmethod
     def forward(ctx, context: Tensor, w: Tensor, block: int) -> Tensor:
@@ -616,10 +621,14 @@ class _Expand16Fn(torch.autograd.Function):
         return _expand_op(context, w, block)
 
     @staticmethod
-    @torch.autograd.function.once_differentiable
     def backward(ctx, dy: Tensor):
         context, w = ctx.saved_tensors
-        dc, dw = _expand_bwd_op(dy, context, w, ctx.block)
+        if torch.is_grad_enabled():
+            sums = dy.to(context.dtype).reshape(*context.shape[:2], ctx.block, w.shape[0]).sum(2)
+            dc = torch.matmul(sums, w)
+            dw = torch.matmul(sums.flatten(0, 1).t(), context.flatten(0, 1))
+        else:
+            dc, dw = _expand_bwd_op(dy, context, w, ctx.block)
         return dc, dw, None
 
 

@@ -98,3 +98,25 @@ def test_indexer_paths_agree(fsi, dev, why):
     add = m.additive_stream(s, v.detach())
     assert add.shape == (2, 40, D)
     assert len(calls) == (4 if why == "hook" else 0)
+
+
+def test_additive_stream_second_derivative(fsi, dev):
+    """A penalty on out_proj's gradient reaches the scores and values, as through nn.Linear."""
+    torch.manual_seed(3)
+    m = fsi.FovealIndexer(hidden_size=128, block_size=8).to(dev)
+    with torch.no_grad():
+        m.out_proj.weight.normal_()
+    s, v = torch.randn(2, 5, 5, device=dev, requires_grad=True), torch.randn(2, 5, 16, device=dev, requires_grad=True)
+    dy = torch.randn(2, 40, 128, device=dev)
+
+    def second(stream, s, v, w, dy):
+        (dw,) = torch.autograd.grad(stream, w, dy, create_graph=True)
+        return torch.autograd.grad(dw.square().sum(), (s, v))
+
+    got = second(m.additive_stream(s, v), s, v, m.out_proj.weight, dy)
+    sd, vd, wd = (t.detach().double().requires_grad_() for t in (s, v, m.out_proj.weight))
+    valid = torch.arange(5, device=dev)[None] < torch.arange(5, device=dev)[:, None]
+    p = torch.nan_to_num(torch.softmax(sd.masked_fill(~valid, float("-inf")), -1))
+    ref = ((p @ vd) @ wd.t()).repeat_interleave(8, dim=1)
+    for a, b in zip(got, second(ref, sd, vd, wd, dy.double())):
+        assert b.any() and (a.double() - b).norm() <= 1e-5 * b.norm()

@@ -1,0 +1,53 @@
+"""Second derivatives of the 16-D index products (CPU only: the kernels' ops stand in as the
+torch products that they compute, in fp64).  As linear layers, which they replace, both can
+be differentiated twice."""
+import pytest
+import torch
+
+
+@pytest.fixture
+def core(fsi, monkeypatch):
+    c = fsi.core
+
+    def proj(x, w0, w1):
+        return x @ w0.t(), x @ w1.t() if w1 is not None else x.new_empty((0,))
+
+    def proj_dw(x, g0, g1):
+        d = lambda g: g.reshape(-1, 16).t() @ x.reshape(-1, x.shape[-1])  # noqa: E731
+        return d(g0), d(g1) if g1 is not None else x.new_empty((0,))
+
+    def expand_bwd(dy, context, w, block):
+        s = dy.reshape(*context.shape[:2], block, -1).sum(2)
+        return s @ w, s.flatten(0, 1).t() @ context.flatten(0, 1)
+
+    monkeypatch.setattr(c, "_proj_op", proj)
+    monkeypatch.setattr(c, "_proj_dw_op", proj_dw)
+    monkeypatch.setattr(c, "_expand_op", lambda ctx, w, n: (ctx @ w.t()).repeat_interleave(n, dim=1))
+    monkeypatch.setattr(c, "_expand_bwd_op", expand_bwd)
+    return c
+
+
+def _leaves(*shapes):
+    g = torch.Generator().manual_seed(0)
+    return [torch.randn(*s, generator=g, dtype=torch.float64).requires_grad_() for s in shapes]
+
+
+def test_projection_twice(core):
+    x, w0, w1 = _leaves((2, 3, 5), (16, 5), (16, 5))
+    both = lambda *a: core._Proj16Fn.apply(*a)  # noqa: E731
+    one = lambda x, w: core._Proj16Fn.apply(x, w, None)[0]  # noqa: E731
+    assert torch.autograd.gradcheck(both, (x, w0, w1)) and torch.autograd.gradgradcheck(both, (x, w0, w1))
+    assert torch.autograd.gradcheck(one, (x[0], w0)) and torch.autograd.gradgradcheck(one, (x[0], w0))
+
+
+def test_projection_gradient_of_one_output(core):
+    """The input's gradient from a constant incoming gradient keeps its graph."""
+    x, w0, w1 = _leaves((2, 3, 5), (16, 5), (16, 5))
+    (dx,) = torch.autograd.grad(core._Proj16Fn.apply(x, w0, w1)[1].sum(), x, create_graph=True)
+    assert torch.equal(torch.autograd.grad(dx.sum(), w1)[0], torch.full((16, 5), 6.0, dtype=torch.float64))
+
+
+def test_expansion_twice(core):
+    ctx, w = _leaves((2, 3, 16), (7, 16))
+    f = lambda c, w: core._Expand16Fn.apply(c, w, 4)  # noqa: E731
+    assert torch.autograd.gradcheck(f, (ctx, w)) and torch.autograd.gradgradcheck(f, (ctx, w))
