@@ -5,6 +5,8 @@ check that the expected ops exist, that their fake implementations give the
 shapes and dtypes the real launches produce, and that a routed decode step
 traces into a graph whose nodes are the fsi ops (what torch.compile / export
 see)."""
+import ctypes
+
 import pytest
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
@@ -130,3 +132,21 @@ def test_plain_call_only_where_the_dispatcher_has_nothing_to_do(fsi):
     torch.func.vmap(lambda a: (seen.append(plain((a,))), a)[1])(torch.zeros(2, 3))
     torch.func.grad(lambda a: (seen.append(plain((t,))), a.sum())[1])(t)
     assert seen == [False, False]
+
+
+def _toy(fsi, name):
+    """An op of the package's kind whose launch reads memory, as a kernel does."""
+    @fsi._lib.fsi_op(name, lambda x, n, s: torch.empty_like(x))
+    def launch(x: torch.Tensor, n: int, s: float) -> torch.Tensor:
+        raw = (ctypes.c_float * x.numel()).from_address(x.data_ptr())
+        return torch.tensor(list(raw)).view(x.shape) * (n * s)
+
+    return launch
+
+
+def test_negated_view_reaches_the_launch_materialised(fsi):
+    """A contiguous view with the negative bit set: its memory holds the other sign."""
+    t = torch.tensor([1.0, -2.0, 3.0])
+    view = torch._neg_view(t)
+    assert view.is_neg() and view.is_contiguous() and not fsi._lib._plain_call((view,))
+    assert torch.equal(_toy(fsi, "toy_negated")(view, 1, 1.0), -t)
