@@ -89,3 +89,32 @@ def test_compiled_indexer_loss_backward_matches_eager(fsi, dev):
         grads.append((loss.detach(), q.grad, k.grad))
     for a, b in zip(*grads):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("what", ["softmax", "mlp", "tile", "stream"])
+def test_batched_gradients(fsi, dev, what):
+    """Vector-Jacobian products of a batch of gradients at once equal one at a time."""
+    torch.manual_seed(0)
+    if what == "softmax":
+        x = torch.randn(2, 3, 20, device=dev)
+        fn = lambda x: fsi.masked_softmax(x, torch.ones(20, dtype=torch.bool, device=dev))  # noqa: E731
+    elif what == "mlp":
+        m = fsi.FovealPattentionMLP(hidden_dim=64, intermediate_dim=256, block_size=16, base_blocks=2, remote_blocks=3,
+                                    dtype=torch.float32).to(dev).train()
+        x, fn = torch.randn(5, 64, device=dev), m
+    elif what == "tile":
+        w, mask = torch.randn(128, 128, device=dev), torch.ones(1, 4, dtype=torch.bool, device=dev)
+        x, fn = torch.randn(5, 128, device=dev), lambda x: fsi.blockwise_matmul(x, w, mask, 64, 64, rows_per_group=128)
+    else:
+        m = fsi.FovealIndexer(hidden_size=128, block_size=8).to(dev)
+        with torch.no_grad():
+            m.out_proj.weight.normal_()
+        v = torch.randn(1, 4, 16, device=dev)
+        x, fn = torch.randn(1, 4, 4, device=dev), lambda s: m.additive_stream(s, v)
+    x.requires_grad_()
+    y = fn(x)
+    dy = torch.randn(3, *y.shape, device=dev)
+    (got,) = torch.autograd.grad(y, x, dy, is_grads_batched=True, retain_graph=True)
+    for i in range(3):
+        (want,) = torch.autograd.grad(y, x, dy[i], retain_graph=True)
+        assert want.any() and (got[i] - want).norm() <= 1e-5 * want.norm()

@@ -150,3 +150,22 @@ def test_negated_view_reaches_the_launch_materialised(fsi):
     view = torch._neg_view(t)
     assert view.is_neg() and view.is_contiguous() and not fsi._lib._plain_call((view,))
     assert torch.equal(_toy(fsi, "toy_negated")(view, 1, 1.0), -t)
+
+
+def test_batched_gradients_go_through_the_dispatcher(fsi):
+    """torch.autograd.grad(is_grads_batched=True) calls a backward once with a tensor that
+    stands for the batch and has no storage; the dispatcher splits it."""
+    op = _toy(fsi, "toy_batched")
+
+    class Fn(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x):
+            return op(x, 2, 1.0)
+
+        @staticmethod
+        def backward(ctx, g):
+            return op(g, 2, 1.0)
+
+    x = torch.ones(3, requires_grad=True)
+    (got,) = torch.autograd.grad(Fn.apply(x), x, torch.eye(3), is_grads_batched=True)
+    assert torch.equal(got, 2 * torch.eye(3))
