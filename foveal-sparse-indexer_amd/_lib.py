@@ -11,6 +11,7 @@ import ctypes
 import functools
 import os
 import threading
+import typing
 from pathlib import Path
 
 import torch
@@ -413,9 +414,11 @@ def fsi_op(name: str, fake, mutates_args=()):
         if mutates_args:  # the dispatcher bumps the mutated tensors' version counters
             return op
 
+        kinds = _argument_kinds(fn)
+
         @functools.wraps(fn)
         def call(*args):
-            return fn(*args) if _plain_call(args) else op(*args)
+            return fn(*args) if _plain_call(args, kinds) else op(*args)
 
         call.op = op
         return call
@@ -423,23 +426,42 @@ def fsi_op(name: str, fake, mutates_args=()):
     return deco
 
 
-def _plain_call(args) -> bool:
+_TENSOR_TYPES = frozenset((torch.Tensor, torch.nn.Parameter))
+_PLAIN_TYPES = _TENSOR_TYPES | {int, float, bool, str, type(None)}
+_C = torch._C
+_forward_ad = torch.autograd.forward_ad
+_pre_dispatch_modes = torch._ops._len_torch_dispatch_stack_pre_dispatch
+_BATCHING = _C._parse_dispatch_key("VmapMode")  # torch.autograd.grad(is_grads_batched=True)
+
+
+def _argument_kinds(fn) -> tuple[frozenset, ...]:
+    """The exact types that a launch function takes at each position, from its annotations."""
+    kinds = []
+    for hint in list(typing.get_type_hints(fn).values())[:fn.__code__.co_argcount]:
+        members = set(typing.get_args(hint)) or {hint}
+        kinds.append(frozenset(members | _TENSOR_TYPES if torch.Tensor in members else members))
+    return tuple(kinds)
+
+
+def _plain_call(args, kinds=None) -> bool:
     """Whether an op call has nothing for the dispatcher to do, so the launch function can be
     called as it is: no tracing, compilation, dispatch or function mode, functorch or batching
-    transform or forward-mode level is active, and every tensor is a plain one without a pending negation
-    that autograd would not record (an op that autograd records, to refuse its backward,
-    still goes through the op).
+    transform or forward-mode level is active, every argument has the type that the launch
+    takes (`kinds`; the dispatcher converts NumPy scalars, 0-d tensors and the like), and every
+    tensor is a plain one without a pending negation that autograd would not record (an op
+    that autograd records, to refuse its backward, still goes through the op).
     The dispatcher's Python route costs 5 us of the 13 that a small op took to issue."""
-    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
-            or torch._C._is_torch_function_mode_enabled() or torch._ops._len_torch_dispatch_stack_pre_dispatch()
-            or torch._C._functorch.peek_interpreter_stack() is not None
-            or torch.autograd.forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None):
+    kinds = (_PLAIN_TYPES,) * len(args) if kinds is None else kinds
+    if (torch.compiler.is_compiling() or _C._len_torch_dispatch_stack() or _C._is_torch_function_mode_enabled()
+            or _pre_dispatch_modes() or _C._functorch.peek_interpreter_stack() is not None
+            or _C._dispatch_tls_is_dispatch_key_included(_BATCHING) or _forward_ad._current_level >= 0
+            or _C._get_tracing_state() is not None or len(args) != len(kinds)):
         return False
     grad = torch.is_grad_enabled()
-    for a in args:
-        if isinstance(a, torch.Tensor):
-            if type(a) is not torch.Tensor and type(a) is not torch.nn.Parameter:
-                return False
-            if a.is_neg() or (grad and a.requires_grad) or torch._C._functorch.is_legacy_batchedtensor(a):
-                return False
+    for a, kind in zip(args, kinds):
+        t = type(a)
+        if t not in kind:
+            return False
+        if t in _TENSOR_TYPES and (a.is_neg() or (grad and a.requires_grad)):
+            return False
     return True

@@ -7,6 +7,7 @@ traces into a graph whose nodes are the fsi ops (what torch.compile / export
 see)."""
 import ctypes
 
+import numpy as np
 import pytest
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
@@ -169,3 +170,35 @@ def test_batched_gradients_go_through_the_dispatcher(fsi):
     x = torch.ones(3, requires_grad=True)
     (got,) = torch.autograd.grad(Fn.apply(x), x, torch.eye(3), is_grads_batched=True)
     assert torch.equal(got, 2 * torch.eye(3))
+
+
+@pytest.mark.parametrize("n", [np.int64(3), np.int32(3), torch.tensor(3)], ids=["int64", "int32", "tensor"])
+@pytest.mark.parametrize("s", [0.5, np.float32(0.5), torch.tensor(0.5)], ids=["float", "float32", "tensor"])
+def test_scalars_are_converted(fsi, n, s):
+    """A size or scale that is no Python number arrives at the launch (a ctypes call) as one."""
+    seen = []
+
+    @fsi._lib.fsi_op(f"toy_scalar_{type(n).__name__}_{type(s).__name__}", lambda x, n, s: torch.empty_like(x))
+    def launch(x: torch.Tensor, n: int, s: float) -> torch.Tensor:
+        seen.append((type(n), type(s), n, s))
+        return x * 2
+
+    launch(torch.ones(2), n, s)
+    assert seen == [(int, float, 3, 0.5)]
+
+
+def test_numbers_of_the_other_kind(fsi):
+    """What a schema refuses stays refused, and a whole number is a float where one is wanted."""
+    op = _toy(fsi, "toy_other")
+    with pytest.raises((RuntimeError, TypeError)):
+        op(torch.ones(2), 3.0, 1.0)
+    assert op(torch.ones(2), 2, 1).tolist() == [2.0, 2.0]
+
+
+def test_every_launch_annotates_its_arguments(fsi):
+    plain = {torch.Tensor, torch.nn.Parameter, int, float, bool, str, type(None)}
+    for name in ("attention", "block_matmul", "core", "foveal_pattention", "pattention"):
+        for f in vars(getattr(fsi, name)).values():
+            if hasattr(f, "op") and hasattr(f, "__wrapped__"):
+                kinds = fsi._lib._argument_kinds(f.__wrapped__)
+                assert len(kinds) == f.__wrapped__.__code__.co_argcount and all(k <= plain for k in kinds), f
