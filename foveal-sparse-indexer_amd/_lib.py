@@ -417,8 +417,8 @@ def fsi_op(name: str, fake, mutates_args=()):
         kinds = _argument_kinds(fn)
 
         @functools.wraps(fn)
-        def call(*args):
-            return fn(*args) if _plain_call(args, kinds) else op(*args)
+        def call(*args, **kwargs):
+            return fn(*args) if not kwargs and _plain_call(args, kinds) else op(*args, **kwargs)
 
         call.op = op
         return call

@@ -202,3 +202,7 @@ def test_every_launch_annotates_its_arguments(fsi):
             if hasattr(f, "op") and hasattr(f, "__wrapped__"):
                 kinds = fsi._lib._argument_kinds(f.__wrapped__)
                 assert len(kinds) == f.__wrapped__.__code__.co_argcount and all(k <= plain for k in kinds), f
+
+
+def test_keyword_arguments(fsi):
+    assert _toy(fsi, "toy_keyword")(torch.ones(2), s=0.5, n=4).tolist() == [2.0, 2.0]
