@@ -445,17 +445,18 @@ def _argument_kinds(fn) -> tuple[frozenset, ...]:
 
 def _plain_call(args, kinds=None) -> bool:
     """Whether an op call has nothing for the dispatcher to do, so the launch function can be
-    called as it is: no tracing, compilation, dispatch or function mode, functorch or batching
-    transform or forward-mode level is active, every argument has the type that the launch
-    takes (`kinds`; the dispatcher converts NumPy scalars, 0-d tensors and the like), and every
-    tensor is a plain one without a pending negation that autograd would not record (an op
-    that autograd records, to refuse its backward, still goes through the op).
+    called as it is: no profiler (which lists the ops by name), tracing, compilation, dispatch
+    or function mode, functorch or batching transform or forward-mode level is active, every
+    argument has the type that the launch takes (`kinds`; the dispatcher converts NumPy
+    scalars, 0-d tensors and the like), and every tensor is a plain one without a pending
+    negation that autograd would not record (an op that autograd records, to refuse its
+    backward, still goes through the op).
     The dispatcher's Python route costs 5 us of the 13 that a small op took to issue."""
     kinds = (_PLAIN_TYPES,) * len(args) if kinds is None else kinds
     if (torch.compiler.is_compiling() or _C._len_torch_dispatch_stack() or _C._is_torch_function_mode_enabled()
             or _pre_dispatch_modes() or _C._functorch.peek_interpreter_stack() is not None
             or _C._dispatch_tls_is_dispatch_key_included(_BATCHING) or _forward_ad._current_level >= 0
-            or _C._get_tracing_state() is not None or len(args) != len(kinds)):
+            or _C._get_tracing_state() is not None or _C._autograd._profiler_enabled() or len(args) != len(kinds)):
         return False
     grad = torch.is_grad_enabled()
     for a, kind in zip(args, kinds):

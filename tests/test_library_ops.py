@@ -206,3 +206,10 @@ def test_every_launch_annotates_its_arguments(fsi):
 
 def test_keyword_arguments(fsi):
     assert _toy(fsi, "toy_keyword")(torch.ones(2), s=0.5, n=4).tolist() == [2.0, 2.0]
+
+
+def test_profiler_lists_the_ops(fsi):
+    op = _toy(fsi, "toy_profiled")
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        op(torch.ones(2), 1, 1.0)
+    assert "fsi::toy_profiled" in {e.key for e in prof.key_averages()}
