@@ -484,14 +484,22 @@ def _projects_here(x: Tensor, *linears: nn.Module) -> bool:
             and all(_plain_linear(m, x) and tuple(m.weight.shape) == (16, x.shape[-1]) for m in linears))
 
 
-def _rows_3d(x: Tensor) -> Tensor:
-    """x as (B, T, D) with unit stride over D and 16-byte aligned rows, copied if it must be."""
+def _rows_3d(x: Tensor) -> Tuple[Tensor, int, int]:
+    """x as (B, T, D) with unit stride over D and 16-byte aligned rows, copied if it must be, and
+    its batch and row strides; those of a dimension of one entry (any number, and kept by
+    contiguous()) are replaced by the packed ones."""
     x = x if x.dim() == 3 else x.unsqueeze(0)
+    B, T, D = x.shape
     vec = 16 // x.element_size()
-    if x.stride(2) != 1 or x.stride(0) % vec or x.stride(1) % vec or x.data_ptr() % 16:
+
+    def strides():
+        xs_t = x.stride(1) if T > 1 else D
+        return x.stride(0) if B > 1 else T * xs_t, xs_t
+
+    if x.stride(2) != 1 or any(s % vec for s in strides()) or x.data_ptr() % 16:
         x = x.contiguous()
         x = x if x.data_ptr() % 16 == 0 else x.clone()
-    return x
+    return x, *strides()
 
 
 def _aligned_contiguous(t: Tensor) -> Tensor:
@@ -506,13 +514,13 @@ def _proj_op(x: Tensor, w0: Tensor, w1: Optional[Tensor]) -> Tuple[Tensor, Tenso
     what = "index projection"
     dev = _lib.require_gpu(x, w0, w1, what=what)
     lead = x.shape[:-1]
-    x3 = _rows_3d(x)
+    x3, xs_b, xs_t = _rows_3d(x)
     w0 = _aligned_contiguous(w0)
     w1 = _aligned_contiguous(w1) if w1 is not None else None
     y0 = torch.empty((*lead, 16), dtype=x.dtype, device=dev)
     y1 = torch.empty((*lead, 16) if w1 is not None else (0,), dtype=x.dtype, device=dev)
     B, T, D = x3.shape
-    st = _lib.lib().fsi_index_proj(x3.data_ptr(), x3.stride(0), x3.stride(1), B, T, D, w0.data_ptr(), _lib.ptr(w1),
+    st = _lib.lib().fsi_index_proj(x3.data_ptr(), xs_b, xs_t, B, T, D, w0.data_ptr(), _lib.ptr(w1),
                                    _lib.dtype_code(x.dtype, what), y0.data_ptr(),
                                    y1.data_ptr() if w1 is not None else None, _lib.stream_handle(dev))
     _lib.check(st, what)
@@ -525,7 +533,7 @@ def _proj_dw_op(x: Tensor, g0: Tensor, g1: Optional[Tensor]) -> Tuple[Tensor, Te
     """fsi_index_proj_dw: (g0^T x, g1^T x or empty)."""
     what = "index projection backward"
     dev = _lib.require_gpu(x, g0, g1, what=what)
-    x3 = _rows_3d(x)
+    x3, xs_b, xs_t = _rows_3d(x)
     g0 = g0.contiguous()
     g1 = g1.contiguous() if g1 is not None else None
     B, T, D = x3.shape
@@ -535,7 +543,7 @@ def _proj_dw_op(x: Tensor, g0: Tensor, g1: Optional[Tensor]) -> Tuple[Tensor, Te
     L = _lib.lib()
     stream = _lib.stream_handle(dev)
     ws = _lib.workspace(dev, L.fsi_index_proj_dw_workspace_size(B * T, D, nw), stream)
-    st = L.fsi_index_proj_dw(x3.data_ptr(), x3.stride(0), x3.stride(1), B, T, D, g0.data_ptr(), _lib.ptr(g1),
+    st = L.fsi_index_proj_dw(x3.data_ptr(), xs_b, xs_t, B, T, D, g0.data_ptr(), _lib.ptr(g1),
                              _lib.dtype_code(x.dtype, what), dw0.data_ptr(), dw1.data_ptr() if nw == 2 else None,
                              ws.data_ptr(), ws.numel(), stream)
     _lib.check(st, what)

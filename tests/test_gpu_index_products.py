@@ -120,3 +120,21 @@ def test_additive_stream_second_derivative(fsi, dev):
     ref = ((p @ vd) @ wd.t()).repeat_interleave(8, dim=1)
     for a, b in zip(got, second(ref, sd, vd, wd, dy.double())):
         assert b.any() and (a.double() - b).norm() <= 1e-5 * b.norm()
+
+
+@pytest.mark.parametrize("shape,strides", [((1, 1, 128), (130, 130, 1)), ((1, 4, 128), (514, 128, 1)),
+                                           ((3, 1, 128), (136, 130, 1))])
+def test_one_row_or_sequence_of_a_padded_buffer(fsi, dev, shape, strides):
+    """A dimension of one entry has a stride that no copy changes."""
+    torch.manual_seed(0)
+    m = fsi.FovealIndexer(hidden_size=128, block_size=1).to(dev)
+    x = torch.randn(600, device=dev).as_strided(shape, strides)
+    q, (k, v) = m.compute_query_16d(x), m.compute_kv_blocks_16d(x)
+    weights = [m.q_proj.weight, m.k_proj.weight, m.v_proj.weight]
+    dy = [torch.randn_like(t) for t in (q, k, v)]
+    got = torch.autograd.grad((q, k, v), weights, dy)
+    y = x.clone(memory_format=torch.contiguous_format)
+    q2, (k2, v2) = m.compute_query_16d(y), m.compute_kv_blocks_16d(y)
+    assert torch.equal(q, q2) and torch.equal(k, k2) and torch.equal(v, v2)
+    for a, b in zip(got, torch.autograd.grad((q2, k2, v2), weights, dy)):
+        assert torch.equal(a, b)

@@ -1,6 +1,6 @@
-"""Second derivatives of the 16-D index products (CPU only: the kernels' ops stand in as the
-torch products that they compute, in fp64).  As linear layers, which they replace, both can
-be differentiated twice."""
+"""Host side of the 16-D index products (CPU only): second derivatives (the kernels' ops stand
+in as the torch products that they compute, in fp64; linear layers, which they replace, can
+be differentiated twice) and the rows that the kernels are handed."""
 import pytest
 import torch
 
@@ -51,3 +51,27 @@ def test_expansion_twice(core):
     ctx, w = _leaves((2, 3, 16), (7, 16))
     f = lambda c, w: core._Expand16Fn.apply(c, w, 4)  # noqa: E731
     assert torch.autograd.gradcheck(f, (ctx, w)) and torch.autograd.gradgradcheck(f, (ctx, w))
+
+
+ROWS = {  # shape, strides, first element
+    "row": ((1, 1, 128), (130, 130, 1), 0),  # one row of a padded buffer
+    "row2d": ((1, 128), (130, 1), 0),
+    "batch": ((1, 4, 128), (516, 128, 1), 0),
+    "rows of one": ((3, 1, 128), (136, 130, 1), 0),
+    "odd rows": ((1, 4, 128), (520, 130, 1), 0),
+    "odd start": ((1, 4, 128), (512, 128, 1), 1),
+    "odd row start": ((1, 1, 128), (130, 130, 1), 1),
+    "expanded": ((3, 4, 128), (0, 128, 1), 0),
+    "turned": ((1, 4, 128), (512, 1, 4), 0),
+}
+
+
+@pytest.mark.parametrize("kind", ROWS)
+def test_rows_are_aligned(fsi, kind):
+    """What the kernels ask for: strides of whole 16-byte pieces, also where a dimension has one
+    entry and torch leaves its stride as it was, and the same values at them."""
+    x = torch.arange(1040).bfloat16().as_strided(*ROWS[kind])
+    y, xs_b, xs_t = fsi.core._rows_3d(x)
+    B, T, D = y.shape
+    assert xs_b % 8 == 0 and xs_t % 8 == 0 and y.data_ptr() % 16 == 0 and y.stride(2) == 1
+    assert torch.equal(y.as_strided((B, T, D), (xs_b, xs_t, 1), y.storage_offset()), x.reshape(B, T, D))
