@@ -191,7 +191,7 @@ def _expand_tiles(m: Tensor, N: int, K: int, block_k: int, block_n: int) -> Tens
     return m.view(nkb, nnb).t().repeat_interleave(block_n, 0).repeat_interleave(block_k, 1)
 
 
-def _tile_bwd_supported(M: int, N: int, groups: int, rpg: int, block_k: int, block_n: int) -> bool:
+def _tile_bwd_supported(M: int, N: int, K: int, groups: int, rpg: int, block_k: int, block_n: int) -> bool:
     """Tilings fsi_blockwise_matmul_bwd takes (include/fsi.h) and is the faster form of.
 
     One row group is the only form in which the library runs two whole dense products
@@ -206,7 +206,7 @@ def _tile_bwd_supported(M: int, N: int, groups: int, rpg: int, block_k: int, blo
     if groups == 1 and 64 in (block_k, block_n) and M > 1024:
         return False
     return (M > 0 and block(block_k) and block(block_n) and (groups == 1 or rpg % 128 == 0) and used <= 2048
-            and N // block_n <= 2048)
+            and N // block_n <= 2048 and max(N, K) // 64 <= 65535)
 
 
 def _aligned16(t: Tensor) -> Tensor:
@@ -263,7 +263,7 @@ class _BlockwiseMatmulFn(torch.autograd.Function):
         block_k, block_n, rpg = ctx.meta
         N, K = weight.shape
         M = x2d.shape[0]
-        if not torch.is_grad_enabled() and _tile_bwd_supported(M, N, m8.shape[0], rpg, block_k, block_n):
+        if not torch.is_grad_enabled() and _tile_bwd_supported(M, N, K, m8.shape[0], rpg, block_k, block_n):
             want_dx, want_dw = ctx.needs_input_grad[:2]
             dx, dw = _blockwise_bwd_op(x2d, weight, dy.to(x2d.dtype), m8, block_k, block_n, rpg, want_dx, want_dw)
             return dx if want_dx else None, dw if want_dw else None, None, None, None, None
