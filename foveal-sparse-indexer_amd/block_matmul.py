@@ -263,6 +263,8 @@ class _BlockwiseMatmulFn(torch.autograd.Function):
         block_k, block_n, rpg = ctx.meta
         N, K = weight.shape
         M = x2d.shape[0]
+        if M <= rpg:  # the first group has every row (the kernels pad rows to whole groups)
+            m8 = m8[:1]
         if not torch.is_grad_enabled() and _tile_bwd_supported(M, N, K, m8.shape[0], rpg, block_k, block_n):
             want_dx, want_dw = ctx.needs_input_grad[:2]
             dx, dw = _blockwise_bwd_op(x2d, weight, dy.to(x2d.dtype), m8, block_k, block_n, rpg, want_dx, want_dw)

@@ -24,6 +24,7 @@ CASES = [  # M, K, N, block_k, block_n, density, groups, rows_per_group
     (256, 3072, 3072, 64, 64, 0.2, 2, 128),     # and its quarters
     (96, 192, 96, 64, 48, 0.5, 1, 96),          # not taken: n blocks of 48
     (256, 256, 256, 32, 64, 0.5, 2, 128),       # not taken: k blocks of 32
+    (257, 256, 256, 128, 64, 0.5, 5, 128),      # two groups past the rows
 ]
 
 
