@@ -119,7 +119,7 @@ __global__ __launch_bounds__(RT_THREADS) void train_route_kernel(RouteArgs A) {
     float l = 0.f, c[RT_DIM] = {};
     for (int b = j; b < A.nb; b += 16) {
       const float* key = keys + b * RT_KS;
-      const float p = __expf((route_score<T>(z, key) - mx) * A.inv_t);
+      const float p = expf((route_score<T>(z, key) - mx) * A.inv_t);
       l += p;
 #pragma unroll
       for (int d = 0; d < RT_DIM; ++d) c[d] = fmaf(p, key[d], c[d]);
@@ -211,7 +211,7 @@ __global__ __launch_bounds__(RT_THREADS) void train_route_bwd_kernel(RouteArgs A
     float l = 0.f, pg = 0.f;
     for (int b = j; b < A.nb; b += 16) {
       const float* key = keys + b * RT_KS;
-      const float e = __expf((route_score<T>(z, key) - mx) * A.inv_t);
+      const float e = expf((route_score<T>(z, key) - mx) * A.inv_t);
       float g = 0.f;
 #pragma unroll
       for (int d = 0; d < RT_DIM; ++d) g = fmaf(key[d], dc[d], g);

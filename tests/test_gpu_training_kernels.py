@@ -146,3 +146,24 @@ def test_training_learnable_temperature(fsi, dev):
     ref = torch.softmax(info["scores"].detach().double() / t, -1) @ w["block_keys_16d"].double()
     (want,) = torch.autograd.grad(ref @ w["out_proj_16d.weight"].double().t(), [t], dy.double())
     assert _close(got, want, 1e-4)
+
+
+def test_training_softmax_tail(fsi, dev):
+    """Single probabilities of the fp32 router softmax, read off a context of one-hot keys.
+    Block 0 scores 2 z, blocks 1 .. 3 score -2 z, z and 0 with z of many values up to 4 sqrt(2), so
+    every difference to the maximum is exact in fp32.  Bound: expf 2^-23 (one ulp), the sum of
+    four terms and the quotient three roundings of 2^-24, the returned scores' own rounding none:
+    3.0e-7."""
+    m = fsi.FovealPattentionMLP(hidden_dim=64, intermediate_dim=64, block_size=16, base_blocks=1, remote_blocks=1,
+                                dtype=torch.float32).to(dev).train()
+    M = 2048
+    q = torch.zeros(M, 16, device=dev)
+    a = torch.linspace(0.0, 1.5, M, device=dev)
+    q[:, 0], q[:, 1] = a.sin(), a.cos()
+    keys = torch.zeros(4, 16, device=dev)
+    keys[:, 0] = torch.tensor([8.0, -8.0, 4.0, 0.0], device=dev)
+    keys[1, 5], keys[2, 6], keys[3, 7] = 1.0, 1.0, 1.0  # q is zero there
+    s, ctx, _ = fsi.foveal_pattention._train_route_op(q, keys, 1, 1, 1.0)
+    assert torch.equal(s[:, 1], -s[:, 0]) and torch.equal(2 * s[:, 2], s[:, 0]) and not s[:, 3].any()
+    p = torch.softmax(s.double(), -1)[:, 1:]
+    assert ((ctx[:, 5:8].double() - p) / p).abs().max() <= 3e-7
