@@ -795,11 +795,17 @@ __device__ __forceinline__ void bf_split8(const f32x4_t& a, const f32x4_t& b, u3
 
 // dQ and the row statistics (as sab_q_kernel).  A workgroup is HP query heads of one KV head
 // (they share the K / V tiles and the block lists) at 64 queries; wave (head, half) owns 32
-// of them.  Consecutive workgroups are consecutive KV heads (one XCD each when there are
-// eight), the latest query tiles first.
+// of them.  With one head (an odd number of them per KV head) four waves share it too: wave
+// (key half, query half) takes 32 keys of every tile, and the halves' statistics and dQ meet
+// in LDS.  Two waves a workgroup leave one wave per SIMD: whole backward, 32 / 32 heads of 128,
+// 8192 tokens 2583 us with two and 2095 with four; 4 x 2048 tokens, 4 / 4 heads of 32, blocks of
+// 10 (classes per element) 667 and 427.  Consecutive workgroups are consecutive KV heads (one
+// XCD each when there are eight), the latest query tiles first.
 template <int HD, int HP, int MIX>
-__global__ __launch_bounds__(128 * HP, 2) void sab_q_bf_kernel(AbParams P) {
-  constexpr int DG = HD / 16, KS32 = HD / 32, NT = 128 * HP, TB = sab_tile_bytes<HD>();
+__global__ __launch_bounds__(AB_THREADS, 2) void sab_q_bf_kernel(AbParams P) {
+  constexpr int DG = HD / 16, KS32 = HD / 32, NT = AB_THREADS, TB = sab_tile_bytes<HD>();
+  static_assert(HP == 1 || HP == 2, "four waves: two heads or two key halves");
+  constexpr int JN = HP;  // 32-key parts of a tile that a wave takes
   // one array: separate ones get alias scopes, and every LDS read would then wait for the
   // direct loads in flight
   __shared__ __attribute__((aligned(1024))) char smem[4 * TB];  // [stage][K, V]
@@ -807,7 +813,8 @@ __global__ __launch_bounds__(128 * HP, 2) void sab_q_bf_kernel(AbParams P) {
   const int t0 = (ntiles - 1 - static_cast<int>(blockIdx.x) / nhp) * AB_T;
   const int hp = static_cast<int>(blockIdx.x) % nhp, g = hp % P.Hkv;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int b = blockIdx.y, h = g * (P.Hq / P.Hkv) + hp / P.Hkv * HP + (wave >> 1);
+  const int b = blockIdx.y, h = g * (P.Hq / P.Hkv) + hp / P.Hkv * HP + (HP == 2 ? wave >> 1 : 0);
+  const int j0 = HP == 2 ? 0 : wave >> 1;  // first of them
   const int r = lane & 15, kg = lane >> 4;
   const int tw = t0 + 32 * (wave & 1);  // this wave's queries tw + 16 i + r
   const bf16_t* q = static_cast<const bf16_t*>(P.q) + b * P.qs_b + h * P.qs_h;
@@ -865,11 +872,11 @@ __global__ __launch_bounds__(128 * HP, 2) void sab_q_bf_kernel(AbParams P) {
       more = it.next();
       if (more) sab_dma<HD, NT>(k, P.ks_t, it.tile * AB_T, P.T, smem + stage * 2 * TB);
       const bool inner = t0 + AB_T <= P.T && s0 + AB_T <= P.T;
-      f32x4_t st[2][4];
+      f32x4_t st[2][2 * JN];
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int j = 0; j < JN; ++j) {
         f32x4_t x[2][2];
-        scores(x, ko + 32 * j * HD * 2, qb);
+        scores(x, ko + 32 * (j0 + j) * HD * 2, qb);
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
           st[i][2 * j] = x[i][0];
@@ -878,10 +885,10 @@ __global__ __launch_bounds__(128 * HP, 2) void sab_q_bf_kernel(AbParams P) {
       }
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        sab_logits2<4, MIX>(P, map_b, tw + 16 * i, r, kg, s0, tcls, inner, sl2, st[i]);
+        sab_logits2<2 * JN, MIX>(P, map_b, tw + 16 * i, r, kg, s0 + 32 * j0, tcls, inner, sl2, st[i]);
         float cm = -INFINITY;
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
+        for (int t = 0; t < 2 * JN; ++t)
 #pragma unroll
           for (int e = 0; e < 4; ++e) cm = fmaxf(cm, st[i][t][e]);
         cm = max_rows4(cm);
@@ -889,7 +896,7 @@ __global__ __launch_bounds__(128 * HP, 2) void sab_q_bf_kernel(AbParams P) {
           const float mn = fmaxf(m[i], cm);
           float add = 0.f;
 #pragma unroll
-          for (int t = 0; t < 4; ++t)
+          for (int t = 0; t < 2 * JN; ++t)
 #pragma unroll
             for (int e = 0; e < 4; ++e) add += __builtin_amdgcn_exp2f(st[i][t][e] - mn);
           lpart[i] = (m[i] > -INFINITY ? lpart[i] * __builtin_amdgcn_exp2f(m[i] - mn) : 0.f) + add;
@@ -903,8 +910,29 @@ __global__ __launch_bounds__(128 * HP, 2) void sab_q_bf_kernel(AbParams P) {
   // or past T (every P 0, no NaN)
   float lse2[2];
 #pragma unroll
+  for (int i = 0; i < 2; ++i) lpart[i] = sum_rows4(lpart[i]);
+  if constexpr (HP == 1) {  // [key half][max, sum][query]
+    float* sums = reinterpret_cast<float*>(smem) + 32 * (wave & 1) + r;
+    if (kg == 0)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        sums[2 * j0 * AB_T + 16 * i] = m[i];
+        sums[(2 * j0 + 1) * AB_T + 16 * i] = lpart[i];
+      }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const float* s = sums + 16 * i;
+      const float m0 = s[0], m1 = s[2 * AB_T];
+      m[i] = fmaxf(m0, m1);
+      lpart[i] = (m0 > -INFINITY ? s[AB_T] * __builtin_amdgcn_exp2f(m0 - m[i]) : 0.f) +
+                 (m1 > -INFINITY ? s[3 * AB_T] * __builtin_amdgcn_exp2f(m1 - m[i]) : 0.f);
+    }
+    __syncthreads();  // the tiles take the memory
+  }
+#pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const float l = sum_rows4(lpart[i]);
+    const float l = lpart[i];
     lse2[i] = l > 0.f && tw + 16 * i + r < P.T ? m[i] + __log2f(l) : INFINITY;
   }
 
@@ -932,7 +960,7 @@ __global__ __launch_bounds__(128 * HP, 2) void sab_q_bf_kernel(AbParams P) {
       if (more) load(stage);
       const bool inner = t0 + AB_T <= P.T && s0 + AB_T <= P.T;
 #pragma unroll 1
-      for (int j = 0; j < 2; ++j) {  // 32 keys at a time (not unrolled: register budget)
+      for (int j = j0; j < j0 + JN; ++j) {  // 32 keys at a time (not unrolled: register budget)
         f32x4_t st[2][2], dp[2][2];
         const uint32_t at = cur + 32 * j * HD * 2;
         scores(st, row_off + at, qb);
@@ -960,6 +988,20 @@ __global__ __launch_bounds__(128 * HP, 2) void sab_q_bf_kernel(AbParams P) {
       }
       __syncthreads();
     }
+  }
+  if constexpr (HP == 1) {  // the second key half hands its sums over, the first stores
+    f32x4_t* part = reinterpret_cast<f32x4_t*>(smem) + (wave & 1) * (2 * DG * 64) + lane;
+    if (j0 == 1)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int dt = 0; dt < DG; ++dt) part[(i * DG + dt) * 64] = dqa[i][dt];
+    __syncthreads();
+    if (j0 == 1) return;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int dt = 0; dt < DG; ++dt) dqa[i][dt] += part[(i * DG + dt) * 64];
   }
   const int64_t row0 = static_cast<int64_t>(b) * P.Hq + h;
 #pragma unroll
@@ -1266,8 +1308,8 @@ FSI_API int fsi_sparse_attn_bwd(const void* q, int64_t qs_b, int64_t qs_h, int64
             al8(v, vs_b, vs_h, vs_t) && al8(dout, ds_b, ds_h, ds_t)) {
           auto launch = [&](auto mix_tag) {
             constexpr int MIX = decltype(mix_tag)::value;
-            if ((Hq / Hkv) % 2 == 0) sab_q_bf_kernel<HD, 2, MIX><<<dim3(gq.x / 2, gq.y), 256, 0, st>>>(P);
-            else sab_q_bf_kernel<HD, 1, MIX><<<gq, 128, 0, st>>>(P);
+            if ((Hq / Hkv) % 2 == 0) sab_q_bf_kernel<HD, 2, MIX><<<dim3(gq.x / 2, gq.y), AB_THREADS, 0, st>>>(P);
+            else sab_q_bf_kernel<HD, 1, MIX><<<gq, AB_THREADS, 0, st>>>(P);
             sab_kv_bf_kernel<HD, MIX><<<gkv, AB_THREADS, 0, st>>>(P);
           };
           if (block % AB_T == 0) launch(sab_mix_t<SAB_TILE>{});

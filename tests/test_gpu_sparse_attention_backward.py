@@ -25,6 +25,11 @@ CASES = [  # B, Hq, Hkv, hd, T, block, window, cap, mode
     (1, 4, 2, 64, 160, 16, 0, 4, 1),
     (1, 2, 2, 32, 96, 8, 0, 4, 1),
     (1, 2, 1, 32, 4200, 64, 100, 2, 0),   # 66 tiles: a second list register
+    (1, 3, 1, 64, 70, 64, 5, 1, 0),       # one head a workgroup, its waves sharing a tile's keys:
+    (1, 1, 1, 128, 33, 16, 40, 3, 0),     # one key past a half
+    (1, 1, 1, 64, 96, 32, 0, 1, 1),       # halves that no query attends
+    (2, 3, 3, 32, 100, 10, 3, 2, 0),
+    (1, 3, 1, 128, 200, 24, 0, 3, 1),
 ]
 
 
