@@ -82,7 +82,7 @@ def test_sparse_attention_backward_bf16(fsi, dev, case):
 @pytest.mark.parametrize("pad", [4, 1])
 def test_sparse_attention_backward_short_alignment(fsi, dev, pad):
     """Operands whose rows start at a multiple of 4 elements (8 bytes) or of one element
-    only keep to the kernels that read them so."""
+    only (copied into aligned ones) give the same gradients."""
     case = (1, 2, 1, 64, 130, 64, 40, 2, 0)
     hd, blk, W = case[3], case[5], case[6]
     q, k, v, dout, idx, cnt = _inputs(case, 5)
