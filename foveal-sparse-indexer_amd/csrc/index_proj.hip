@@ -397,8 +397,11 @@ FSI_API int fsi_index_proj(const void* x, int64_t xs_b, int64_t xs_t, int64_t B,
   auto run = [&](auto tag, auto flat) {
     using E = decltype(tag);
     constexpr bool F = decltype(flat)::value;
-    // 64 rows a workgroup once that gives every compute unit one, 16 below
-    if (A.M >= 8192) {
+    // 16 rows a workgroup as long as all of them run at once (two of eight waves on each of 256
+    // compute units), 64 rows beyond.  us with 64 | 16, keys and values of 2048 columns in
+    // fp32: 4096 rows 27.3 | 13.5, 8192 27.5 | 23.9, 12288 27.8 | 34.4, 16384 28.1 | 45.2; bf16 14.1 |
+    // 12.4, 14.3 | 13.6, 14.6 | 19.0, 14.8 | 24.2.
+    if (A.M > 8192) {
       const unsigned g = static_cast<unsigned>((A.M + 63) / 64);
       if (w1) proj_kernel<E, 2, 4, 4, F><<<g, 256, 0, st>>>(A);
       else proj_kernel<E, 1, 4, 4, F><<<g, 256, 0, st>>>(A);
