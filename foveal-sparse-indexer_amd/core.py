@@ -368,8 +368,9 @@ class FovealIndexer(nn.Module):
         if tuple(v.shape) != (B, Nb, self.index_dim):
             raise ValueError(f"{what}: values {tuple(v.shape)} != {(B, Nb, self.index_dim)}")
         context = _AdditiveContextFn.apply(s, v, self.causal)
-        if _plain_linear(self.out_proj, context) and self.out_proj.out_features % 8 == 0 and self.block_size > 0:
-            return _Expand16Fn.apply(context, self.out_proj.weight, self.block_size)
+        w = self.out_proj.weight if _plain_linear(self.out_proj, context) else None
+        if w is not None and w.shape[0] % 8 == 0 and w.shape[1] == 16 and self.block_size > 0:
+            return _Expand16Fn.apply(context, w, self.block_size)
         out_blocks = self.out_proj(context)
         return out_blocks.repeat_interleave(self.block_size, dim=1)
 
@@ -507,11 +508,22 @@ def _aligned_contiguous(t: Tensor) -> Tensor:
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
+def _check_operands(what: str, like: Tensor, *operands) -> None:
+    """Each (tensor or None, its shape): the kernels read it as that, in like's type."""
+    for t, shape in operands:
+        if t is not None and t.dtype != like.dtype:
+            raise TypeError(f"{what}: dtype mismatch {t.dtype}/{like.dtype}")
+        if t is not None and tuple(t.shape) != tuple(shape):
+            raise ValueError(f"{what}: {tuple(t.shape)} != {tuple(shape)}")
+
+
 @_lib.fsi_op("index_proj", lambda x, w0, w1: (x.new_empty((*x.shape[:-1], 16)),
                                              x.new_empty((*x.shape[:-1], 16) if w1 is not None else (0,))))
 def _proj_op(x: Tensor, w0: Tensor, w1: Optional[Tensor]) -> Tuple[Tensor, Tensor]:
     """fsi_index_proj: (x w0^T, x w1^T or empty)."""
     what = "index projection"
+    D = x.shape[-1]
+    _check_operands(what, x, (w0, (16, D)), (w1, (16, D)))
     dev = _lib.require_gpu(x, w0, w1, what=what)
     lead = x.shape[:-1]
     x3, xs_b, xs_t = _rows_3d(x)
@@ -532,6 +544,8 @@ def _proj_op(x: Tensor, w0: Tensor, w1: Optional[Tensor]) -> Tuple[Tensor, Tenso
 def _proj_dw_op(x: Tensor, g0: Tensor, g1: Optional[Tensor]) -> Tuple[Tensor, Tensor]:
     """fsi_index_proj_dw: (g0^T x, g1^T x or empty)."""
     what = "index projection backward"
+    y_shape = (*x.shape[:-1], 16)
+    _check_operands(what, x, (g0, y_shape), (g1, y_shape))
     dev = _lib.require_gpu(x, g0, g1, what=what)
     x3, xs_b, xs_t = _rows_3d(x)
     g0 = g0.contiguous()
@@ -589,6 +603,7 @@ class _Proj16Fn(torch.autograd.Function):
 def _expand_op(ctx16: Tensor, w: Tensor, block: int) -> Tensor:
     """fsi_index_expand: (ctx16 w^T) of every block repeated over its elements."""
     what = "additive_stream"
+    _check_operands(what, ctx16, (ctx16, (*ctx16.shape[:2], 16)), (w, (w.shape[0], 16)))
     dev = _lib.require_gpu(ctx16, w, what=what)
     c, w = _aligned_contiguous(ctx16), _aligned_contiguous(w)
     B, nb = c.shape[:2]
@@ -604,6 +619,9 @@ def _expand_op(ctx16: Tensor, w: Tensor, block: int) -> Tensor:
 def _expand_bwd_op(dy: Tensor, ctx16: Tensor, w: Tensor, block: int) -> Tuple[Tensor, Tensor]:
     """fsi_index_expand_bwd: (dctx16, dw)."""
     what = "additive_stream backward"
+    _check_operands(what, ctx16, (ctx16, (*ctx16.shape[:2], 16)), (w, (w.shape[0], 16)))
+    if tuple(dy.shape) != (ctx16.shape[0], ctx16.shape[1] * block, w.shape[0]):
+        raise ValueError(f"{what}: gradient {tuple(dy.shape)}")
     dev = _lib.require_gpu(dy, ctx16, w, what=what)
     dy, c, w = (_aligned_contiguous(t) for t in (dy.to(ctx16.dtype), ctx16, w))
     n, D = c.shape[0] * c.shape[1], w.shape[0]

@@ -75,3 +75,38 @@ def test_rows_are_aligned(fsi, kind):
     B, T, D = y.shape
     assert xs_b % 8 == 0 and xs_t % 8 == 0 and y.data_ptr() % 16 == 0 and y.stride(2) == 1
     assert torch.equal(y.as_strided((B, T, D), (xs_b, xs_t, 1), y.storage_offset()), x.reshape(B, T, D))
+
+
+def test_ops_refuse_operands_of_other_shapes(fsi):
+    """The kernels read 16 columns, or 16 components a row, of one type, whatever the memory holds."""
+    core, z = fsi.core, torch.zeros
+    x, w, c = z(2, 3, 128), z(16, 128), z(2, 3, 16)
+    for call in (lambda: core._proj_op(x, w[:, :64], None), lambda: core._proj_op(x, w[:8], None),
+                 lambda: core._proj_op(x, w, w[:8]), lambda: core._proj_dw_op(x, c[:, :2], None),
+                 lambda: core._proj_dw_op(x, c, c[..., :8]), lambda: core._expand_op(c, z(16, 8), 4),
+                 lambda: core._expand_op(c[..., :8], z(16, 8), 4),
+                 lambda: core._expand_bwd_op(z(2, 12, 8), c, z(16, 16), 4),
+                 lambda: core._expand_bwd_op(z(2, 6, 16), c, z(16, 16), 4)):
+        with pytest.raises(ValueError):
+            call()
+    for call in (lambda: core._proj_op(x, w, w.bfloat16()), lambda: core._proj_dw_op(x, c.bfloat16(), None),
+                 lambda: core._expand_op(c, z(16, 16).bfloat16(), 4)):
+        with pytest.raises(TypeError, match="dtype mismatch"):
+            call()
+
+
+@pytest.mark.parametrize("shape", [(16, 8), (24, 16)])
+def test_stream_of_a_replaced_out_proj(fsi, shape):
+    """A projection of another input width is refused, as by the linear layer itself; 16 outputs
+    are not 16 inputs."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    with FakeTensorMode(), torch.device("cuda"):
+        m = fsi.FovealIndexer(hidden_size=128, block_size=8)
+        m.out_proj = torch.nn.Linear(shape[1], shape[0], bias=False)
+        s, v = torch.empty(1, 2, 2), torch.empty(1, 2, 16)
+        if shape[1] == 16:
+            assert m.additive_stream(s, v).shape == (1, 16, 24)
+        else:
+            with pytest.raises(RuntimeError):
+                m.additive_stream(s, v)
