@@ -248,6 +248,9 @@ def _train_gather_op(k_gate: Tensor, k_up: Tensor, v: Tensor, active: Tensor, bl
                      v_t: bool) -> Tuple[Tensor, Tensor]:
     """fsi_mlp_train_gather: the active rows of [k_gate; k_up] and of v ((D, n) with v_t)."""
     what = "FovealPattentionMLP training"
+    if not (k_gate.shape == k_up.shape == v.shape) or not (k_gate.dtype == k_up.dtype == v.dtype):
+        raise ValueError(f"{what}: weights {tuple(k_gate.shape)} {k_gate.dtype}, {tuple(k_up.shape)} {k_up.dtype}, "
+                         f"{tuple(v.shape)} {v.dtype}")
     dev = _lib.require_gpu(k_gate, k_up, v, active, what=what)
     kg, ku, vv = _aligned_rows(k_gate), _aligned_rows(k_up), _aligned_rows(v.t() if v_t else v)
     if kg.stride(0) != ku.stride(0):
@@ -769,7 +772,8 @@ class FovealPattentionMLP(nn.Module):
 
     def _train_fused(self, x_2d: Tensor) -> bool:
         """Whether the training forward runs on csrc/mlp_train.hip: the fused SwiGLU (the eager
-        one rounds in between), one dtype, queries from a plain linear layer (a hook or a
+        one rounds in between), one dtype, weights of the module's sizes,
+        queries from a plain linear layer (a hook or a
         wrapper may give another type), the class's own router scores, a temperature that is a
         number (a tensor has a gradient) whose reciprocal fp32 holds, a 16-D index over at
         most 256 blocks, rows and blocks of whole 16-byte vectors, and no autocast (which
@@ -780,6 +784,7 @@ class FovealPattentionMLP(nn.Module):
                 and type(self).compute_router_scores is _ROUTER_SCORES
                 and "compute_router_scores" not in self.__dict__
                 and all(w.dtype == dt and w.is_cuda for w in weights)
+                and all(tuple(w.shape) == (self.intermediate_dim, self.hidden_dim) for w in weights[:3])
                 and _plain_linear(self.q_proj_16d, x_2d)
                 and tuple(self.q_proj_16d.weight.shape) == (16, self.hidden_dim)
                 and self.index_dim == 16 and self.num_blocks <= 256 and x_2d.shape[0] > 0
@@ -789,7 +794,6 @@ class FovealPattentionMLP(nn.Module):
                 and self.hidden_dim % 8 == 0 and self.block_size % 8 == 0
                 and isinstance(self.temperature, (int, float)) and 1e-30 <= self.temperature <= 1e30
                 and self.intermediate_dim % self.block_size == 0
-                and tuple(self.v.shape) == tuple(self.k_gate.shape)
                 and not torch.is_autocast_enabled("cuda"))
 
     def forward(self, x: Tensor, return_router_info: bool = False):

@@ -117,3 +117,20 @@ def test_temperature_keeps_torch_ops(fsi, temperature):
 @pytest.mark.parametrize("temperature", [1, 0.5])
 def test_number_temperature_is_fused(fsi, temperature):
     assert _fused(_traced(fsi, lambda m: setattr(m, "temperature", temperature)))
+
+
+@pytest.mark.parametrize("name", ["k_gate", "k_up", "v"])
+def test_weights_of_another_size_keep_torch_ops(fsi, name):
+    """A shorter weight has no rows for some active blocks: indexing it is refused or not by
+    torch; the gather kernel would read past its end."""
+    def shorten(m):
+        setattr(m, name, nn.Parameter(getattr(m, name).detach()[:512]))
+
+    assert not _fused(_traced(fsi, shorten))
+
+
+def test_gather_op_refuses_weights_of_two_sizes_or_types(fsi):
+    w, active = torch.zeros(64, 16), torch.zeros(1, dtype=torch.int32)
+    for ws in ((w, w[:32], w), (w, w, w[:32]), (w, w.bfloat16(), w)):
+        with pytest.raises(ValueError, match="weights"):
+            fsi.foveal_pattention._train_gather_op(*ws, active, 16, False)
