@@ -24,6 +24,7 @@ from typing import Any, Dict, Iterable, List, Optional, Tuple
 import torch
 import torch.nn.functional as F
 from torch import Tensor, nn
+from torch._subclasses.fake_tensor import FakeTensor
 
 from . import _lib
 from .core import _plain_linear
@@ -772,8 +773,8 @@ class FovealPattentionMLP(nn.Module):
 
     def _train_fused(self, x_2d: Tensor) -> bool:
         """Whether the training forward runs on csrc/mlp_train.hip: the fused SwiGLU (the eager
-        one rounds in between), one dtype, weights of the module's sizes,
-        queries from a plain linear layer (a hook or a
+        one rounds in between), one dtype, weights of the module's sizes in no tensor class of
+        their own (which may gather in its own way), queries from a plain linear layer (a hook or a
         wrapper may give another type), the class's own router scores, a temperature that is a
         number (a tensor has a gradient) whose reciprocal fp32 holds, a 16-D index over at
         most 256 blocks, rows and blocks of whole 16-byte vectors, and no autocast (which
@@ -783,7 +784,7 @@ class FovealPattentionMLP(nn.Module):
         return (self.use_fused_kernel and dt in (torch.bfloat16, torch.float32)
                 and type(self).compute_router_scores is _ROUTER_SCORES
                 and "compute_router_scores" not in self.__dict__
-                and all(w.dtype == dt and w.is_cuda for w in weights)
+                and all(w.dtype == dt and w.is_cuda and type(w) in _WEIGHT_TYPES for w in weights)
                 and all(tuple(w.shape) == (self.intermediate_dim, self.hidden_dim) for w in weights[:3])
                 and _plain_linear(self.q_proj_16d, x_2d)
                 and tuple(self.q_proj_16d.weight.shape) == (16, self.hidden_dim)
@@ -830,6 +831,7 @@ class FovealPattentionMLP(nn.Module):
 # What the fused training path computes in place of a call: a subclass, an instance or the
 # class itself may hold another (noise, a balancing bias), which is then called.
 _ROUTER_SCORES = FovealPattentionMLP.compute_router_scores
+_WEIGHT_TYPES = (nn.Parameter, Tensor, FakeTensor)
 
 
 def release_unpacked_weights(model: nn.Module) -> int:

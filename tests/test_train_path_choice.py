@@ -134,3 +134,31 @@ def test_gather_op_refuses_weights_of_two_sizes_or_types(fsi):
     for ws in ((w, w[:32], w), (w, w, w[:32]), (w, w.bfloat16(), w)):
         with pytest.raises(ValueError, match="weights"):
             fsi.foveal_pattention._train_gather_op(*ws, active, 16, False)
+
+
+class _Stored(torch.Tensor):
+    """A weight in a storage form of its own (quantised, sharded) that indexing decodes."""
+
+    @staticmethod
+    def __new__(cls, like):
+        return torch.Tensor._make_wrapper_subclass(cls, like.shape, dtype=like.dtype, device=like.device)
+
+    def __init__(self, like):
+        self.inner = like
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        args = [a.inner if isinstance(a, _Stored) else a for a in args]
+        if func not in (torch.ops.aten.index.Tensor, torch.ops.aten.detach.default):
+            raise NotImplementedError(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("name", ["k_gate", "k_up", "v"])
+def test_weight_of_a_tensor_class_is_indexed(fsi, name):
+    def store(m):
+        w = getattr(m, name).detach()
+        del m._parameters[name]
+        setattr(m, name, _Stored(w))
+
+    assert not _fused(_traced(fsi, store))
