@@ -627,11 +627,11 @@ def _expand_bwd_op(dy: Tensor, ctx16: Tensor, w: Tensor, block: int) -> Tuple[Te
     n, D = c.shape[0] * c.shape[1], w.shape[0]
     dc, dw = torch.empty_like(c), torch.empty_like(w)
     L = _lib.lib()
-    stream = _lib.stream_handle(dev)
-    ws = _lib.workspace(dev, L.fsi_index_expand_bwd_workspace_size(n, D), stream)
+    # scratch of this call alone: with small blocks it is as large as dy, so it is not kept
+    ws = torch.empty(L.fsi_index_expand_bwd_workspace_size(n, D), dtype=torch.uint8, device=dev)
     st = L.fsi_index_expand_bwd(dy.data_ptr(), c.data_ptr(), w.data_ptr(), n, block, D,
                                 _lib.dtype_code(c.dtype, what), dc.data_ptr(), dw.data_ptr(), ws.data_ptr(),
-                                ws.numel(), stream)
+                                ws.numel(), _lib.stream_handle(dev))
     _lib.check(st, what)
     return dc, dw
 

@@ -53,6 +53,15 @@ def test_expansion(fsi, dev, dtype, B, nb, block, D):
     assert _close(dw, s.reshape(-1, D).t() @ c.reshape(-1, 16).double(), dtype)
 
 
+def test_expansion_backward_keeps_no_scratch(fsi, dev):
+    """With blocks of one element the block sums are as large as the gradient itself."""
+    c, w = torch.randn(2, 2000, 16, device=dev), torch.randn(2048, 16, device=dev)
+    kept = lambda: sum(b.numel() for b in fsi._lib._ws.values())  # noqa: E731
+    before = kept()
+    fsi.core._expand_bwd_op(torch.randn(2, 2000, 2048, device=dev), c, w, 1)
+    assert kept() == before
+
+
 @pytest.mark.parametrize("why", ["plain", "hook", "bias", "width", "autocast", "odd"])
 def test_indexer_paths_agree(fsi, dev, why):
     """The indexer's representations and gradients are those of its linear layers, whichever
