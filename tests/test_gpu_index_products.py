@@ -103,9 +103,17 @@ def test_indexer_paths_agree(fsi, dev, why):
     want = torch.autograd.grad((qr, kr, vr), leaves, (dq.double(), dk.double(), dv.double()))
     for a, b in zip(got, want):
         assert (a.double() - b).norm() <= 1e-5 * b.double().norm()
-    s = torch.randn(2, 5, 5, device=dev)
-    add = m.additive_stream(s, v.detach())
-    assert add.shape == (2, 40, D)
+    s, vv = torch.randn(2, 5, 5, device=dev, requires_grad=True), v.detach().requires_grad_()
+    valid = torch.arange(5, device=dev)[None] < torch.arange(5, device=dev)[:, None]
+    add = m.additive_stream(s, vv)
+    sd, vd, wd = (t.detach().double().requires_grad_() for t in (s, vv, m.out_proj.weight))
+    p = torch.nan_to_num(torch.softmax(sd.masked_fill(~valid, float("-inf")), -1))
+    ref = ((p @ vd) @ wd.t()).repeat_interleave(8, dim=1)
+    assert add.shape == (2, 40, D) and _close(add.detach(), ref.detach(), torch.float32)
+    dy = torch.randn_like(add)
+    for a, b in zip(torch.autograd.grad(add, (s, vv, m.out_proj.weight), dy),
+                    torch.autograd.grad(ref, (sd, vd, wd), dy.double())):
+        assert b.any() and (a.double() - b).norm() <= 1e-5 * b.norm()
     assert len(calls) == (4 if why == "hook" else 0)
 
 

@@ -8,6 +8,9 @@ that underflow, and non-finite scores (equal bits in, equal order out)."""
 import pytest
 import torch
 
+from oracle import routing as R
+from route_check import check_rows
+
 pytestmark = pytest.mark.gpu
 
 
@@ -52,8 +55,9 @@ def test_candidates_rank_as_the_row(fsi, dev, kind, N, dtype):
 @pytest.mark.parametrize("N", [1030, 2000, 4096])
 @pytest.mark.parametrize("keys", ["random", "repeated", "tiny", "wide"])
 def test_scored_candidates_rank_as_the_row(fsi, dev, N, keys):
-    """score_and_route: indices, counts and mass of the two searches agree exactly
-    (fp64 sums of these masses are exact in either order)."""
+    """score_and_route: indices, counts and mass of the two searches agree exactly (fp64 sums of
+    these masses are exact in either order), and with the oracle, whose normalisation and
+    softmax are plain fp32 divisions, up to near-ties."""
     print(f"[case] scored candidates {keys} {N}", flush=True)
     g = torch.Generator().manual_seed(N + len(keys))
     q, k = torch.randn(2, 37, 16, generator=g), torch.randn(2, N, 16, generator=g)
@@ -68,3 +72,11 @@ def test_scored_candidates_rank_as_the_row(fsi, dev, N, keys):
     ia, ca, ma = fsi.score_and_route(q.to(dev), k.to(dev), remote_capacity=64, **kw)
     ib, cb, mb = fsi.score_and_route(q.to(dev), k.to(dev), remote_capacity=128, **kw)
     assert torch.equal(ca, cb) and torch.equal(ma, mb) and torch.equal(ia, ib[..., :64])
+    ora = R.select_route(R.cosine_scores_f32(q, k), causal=False, top_p=0.9, min_remote_blocks=4, max_remote_blocks=64,
+                         remote_capacity=64)
+    bad = check_rows(ia, ca, ora, torch.ones(37, N, dtype=torch.bool), 1e-6, 1e-5)
+    assert not bad, bad
+    cnt = ora["remote_counts"].long()
+    want = ora["cumulative"].gather(2, (cnt - 1)[..., None])[..., 0]  # at least 4 are taken
+    same = ca.cpu().long() == cnt
+    assert same.any() and torch.allclose(ma.cpu()[same], want[same], atol=2e-6)
