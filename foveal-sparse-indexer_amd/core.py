@@ -510,10 +510,13 @@ def _aligned_contiguous(t: Tensor) -> Tensor:
 
 def _check_operands(what: str, like: Tensor, *operands) -> None:
     """Each (tensor or None, its shape): the kernels read it as that, in like's type."""
+    dtype = like.dtype
     for t, shape in operands:
-        if t is not None and t.dtype != like.dtype:
-            raise TypeError(f"{what}: dtype mismatch {t.dtype}/{like.dtype}")
-        if t is not None and tuple(t.shape) != tuple(shape):
+        if t is None:
+            continue
+        if t.dtype is not dtype:
+            raise TypeError(f"{what}: dtype mismatch {t.dtype}/{dtype}")
+        if t.shape != shape:
             raise ValueError(f"{what}: {tuple(t.shape)} != {tuple(shape)}")
 
 
@@ -598,12 +601,19 @@ class _Proj16Fn(torch.autograd.Function):
         return dx, dw0, dw1
 
 
+def _check_stream(what: str, ctx16: Tensor, w: Tensor) -> None:
+    if w.dtype is not ctx16.dtype:
+        raise TypeError(f"{what}: dtype mismatch {w.dtype}/{ctx16.dtype}")
+    if ctx16.dim() != 3 or w.dim() != 2 or ctx16.shape[2] != 16 or w.shape[1] != 16:
+        raise ValueError(f"{what}: context {tuple(ctx16.shape)} and weight {tuple(w.shape)} (rows of 16)")
+
+
 @_lib.fsi_op("index_expand", lambda ctx16, w, block: ctx16.new_empty(
     (ctx16.shape[0], ctx16.shape[1] * block, w.shape[0])))
 def _expand_op(ctx16: Tensor, w: Tensor, block: int) -> Tensor:
     """fsi_index_expand: (ctx16 w^T) of every block repeated over its elements."""
     what = "additive_stream"
-    _check_operands(what, ctx16, (ctx16, (*ctx16.shape[:2], 16)), (w, (w.shape[0], 16)))
+    _check_stream(what, ctx16, w)
     dev = _lib.require_gpu(ctx16, w, what=what)
     c, w = _aligned_contiguous(ctx16), _aligned_contiguous(w)
     B, nb = c.shape[:2]
@@ -619,7 +629,7 @@ def _expand_op(ctx16: Tensor, w: Tensor, block: int) -> Tensor:
 def _expand_bwd_op(dy: Tensor, ctx16: Tensor, w: Tensor, block: int) -> Tuple[Tensor, Tensor]:
     """fsi_index_expand_bwd: (dctx16, dw)."""
     what = "additive_stream backward"
-    _check_operands(what, ctx16, (ctx16, (*ctx16.shape[:2], 16)), (w, (w.shape[0], 16)))
+    _check_stream(what, ctx16, w)
     if tuple(dy.shape) != (ctx16.shape[0], ctx16.shape[1] * block, w.shape[0]):
         raise ValueError(f"{what}: gradient {tuple(dy.shape)}")
     dev = _lib.require_gpu(dy, ctx16, w, what=what)
