@@ -195,12 +195,14 @@ def _tile_bwd_supported(M: int, N: int, K: int, groups: int, rpg: int, block_k: 
     """Tilings fsi_blockwise_matmul_bwd takes (include/fsi.h) and is the faster form of.
 
     One row group is the only form in which the library runs two whole dense products
-    instead of two per group.  Its 128 x 128 output tiles hold up to four 64-wide mask tiles
-    there, so at density 0.5 nearly all of them have work, and many rows hide the library
-    form's masking passes: 64 x 64 tiles of 8192 x 8192 at density 0.5, forward and both
-    gradients, 0.57 / 0.72 / 1.27 ms here and 0.72 / 0.84 / 1.16 ms there for 512 / 1024 /
-    2048 rows (4096 x 4096: 0.23 / 0.26 / 0.345 and 0.245 / 0.27 / 0.34); 128 x 128 tiles
-    0.66 and 1.00 ms for 2048 rows."""
+    instead of two per group.  The library form's time hardly depends on the density, which the
+    host doesn't know; the 128 x 128 output tiles here hold up to four 64-wide mask tiles, so at
+    density 0.5 nearly all of them have work.  The line keeps dense masks from losing: 8192 x
+    8192 at density 0.1 / 0.25 / 0.5, forward and both gradients, 64 x 64 tiles 0.37 / 0.54 /
+    0.72 ms here and 0.73 / 0.78 / 0.85 there for 1024 rows, 0.59 / 0.91 / 1.27 and 0.95 /
+    1.06 / 1.21 for 2048, 1.04 / 1.67 / 2.36 and 1.46 / 1.67 / 1.95 for 4096 (sparse masks of
+    many rows thus stay with the slower form); 128 x 128 tiles 0.33 / 0.45 / 0.68 and 0.88 /
+    0.94 / 1.03 for 2048 rows, 0.53 / 0.76 / 1.24 and 1.35 / 1.45 / 1.63 for 4096."""
     block = lambda b: b == 64 or b % 128 == 0  # noqa: E731
     used = -(-M // rpg) if groups > 1 else 1
     if groups == 1 and 64 in (block_k, block_n) and M > 1024:

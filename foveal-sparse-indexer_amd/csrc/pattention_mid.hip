@@ -223,9 +223,10 @@ bool mid_plan(int64_t tiles, int64_t steps, MidPlan& p) {
   return false;
 }
 
-// Elements of one weight matrix's active rows from which these kernels are the faster ones:
-// below, the caches hold the weights that every 64-token workgroup of the other kernels reads
-// again.  us a pass, there -> here, for 65 / 150 / 255 tokens: 4096 x 4096 (16.8 M) 59 / 92 /
+// Elements of one weight matrix's active rows from which these kernels are the faster ones at
+// every token count: below, the caches hold the weights that every 64-token workgroup of the
+// other kernels reads again, and the partials weigh more.  At 8.4 M five of six points are
+// 3 to 13 % faster here, but one is 3 % slower and the line keeps it from losing.  us a pass, there -> here, for 65 / 150 / 255 tokens: 4096 x 4096 (16.8 M) 59 / 92 /
 // 111 -> 44 / 63 / 77; 4096 x 2048 and 2048 x 4096 (8.4 M) 36 / 54 / 61 -> 33 / 47 / 59 and
 // 38 / 53 / 60 -> 36 / 50 / 62; 2048 x 1536 (3.1 M) 22 / 30 / 32 -> 23 / 35 / 45.
 constexpr int64_t MD_MIN_WEIGHT = 12 << 20;
