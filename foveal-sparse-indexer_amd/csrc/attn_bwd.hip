@@ -543,12 +543,15 @@ __global__ __launch_bounds__(AB_THREADS) void sab_kv_kernel(AbParams P) {
 // v_mfma_f32_16x16x32_bf16 over 64-row tiles moved straight into LDS (no staging
 // registers), double-buffered: the next tile's loads run while this one is used.
 //
-// What bounds these kernels is LDS, not the matrix cores: an operand fragment is 1 KiB
-// (8 LDS clocks) and feeds a 16-clock MFMA on one of four SIMDs, so a fragment has to
-// serve two MFMAs at least.  Each wave therefore owns 32 rows (two 16-row operands in
-// registers) of its side, and P / dS enter their products as a pair of bf16 operands
-// hi + lo (hi = the value rounded to bf16, lo = the remainder rounded; ~2^-17 relative,
-// the other operand an exact bf16 input, fp32 accumulation), which makes it four there.
+// An operand fragment is 1 KiB (8 LDS clocks) and feeds a 16-clock MFMA on one of four SIMDs,
+// so a fragment has to serve two MFMAs at least or LDS bounds the kernel.  Each wave therefore
+// owns 32 rows (two 16-row operands in registers) of its side, and P / dS enter their products as
+// a pair of bf16 operands hi + lo (hi = the value rounded to bf16, lo = the remainder rounded;
+// ~2^-17 relative, the other operand an exact bf16 input, fp32 accumulation), which makes it four
+// there.  With that no unit is full (sab_q | sab_kv: MFMA 0.37 | 0.41 busy, VALU 0.55 | 0.44, LDS
+// 0.30 | 0.29 with half of it bank conflicts): what bounds them is the chain product, softmax
+// and split, product of every tile, at the two waves per SIMD that registers (204 | 256) and
+// LDS (64 | 65 KiB a workgroup) leave.
 // The tiles are stored row-major only: products that contract over a tile's rows read it
 // with ds_read_b64_tr_b16, so no transposed copy is written.
 // 8192 tokens, 32 / 8 heads of 128, window 1024 + 32 pages: sab_q 1521 -> 1026 us,

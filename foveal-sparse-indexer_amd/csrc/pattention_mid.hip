@@ -13,7 +13,9 @@
 //   mid_out_kernel    sums the splits -> out
 // The partials cost 30 MB of traffic each way at that size, less than the rows they save.
 // 150 tokens of the 8B layer (4096 hidden, 64 of 224 blocks): 92 -> 63 us, the two GEMMs
-// 31 and 21 (2.4 TB/s of weights; the token rows from L2 bound them).
+// 31 and 21 (2.1 - 2.4 TB/s of weights: the vector memory counter is in order, so waiting for a
+// step's token rows, loaded two steps ahead, also waits for the weight stages issued before
+// them, and two stages of the ring stay in flight).
 #include "fsi_common.h"
 
 using namespace fsi;
@@ -134,7 +136,7 @@ __global__ __launch_bounds__(MD_THREADS, 2) void mid_gemm_kernel(MidArgs A) {
   load_a(av[0], 0);
   load_a(av[1], 1);
   // One step: refill the stage read in the previous one, then multiply.  Counting the direct
-  // loads alone (the token rows in flight only make the wait stricter), the stage of `step`
+  // loads alone (the token rows in flight make the wait stricter), the stage of `step`
   // has landed once at most the STAGES - 2 later steps' are outstanding.
   auto run = [&](int step, u32x4_t (&x)[MT][2], u32x4_t (&next)[MT][2]) {
     if (step + STAGES - 2 < A.steps) md_wait<UNITS * (STAGES - 2)>();

@@ -778,9 +778,9 @@ FSI_API size_t fsi_blockwise_matmul_bwd_workspace_size(int64_t M, int64_t N, int
 // groups whose mask has the tile, so both do the forward's operations and sum in fp32 (the
 // masked dense products of the library form do 1 / density times as many and write W o T
 // for every group).  4096 x 8192 x 8192 at 25 % in 32 groups: 15.0 -> 0.52 ms for both
-// gradients, 225 us for each GEMM (610 TFLOP/s, as the forward: the operand stream of its
+// gradients, 195 us for each GEMM (700 TFLOP/s, as the forward: the operand stream of its
 // 128 x 128 tiles bounds it).  The GEMM wants both operands contraction-major, so W (for
-// dx), dy and x (for dW) are transposed first, 128 of the 520 us (4.2 TB/s).
+// dx), dy and x (for dW) are transposed first, 103 of the 520 us (5.2 TB/s).
 FSI_API int fsi_blockwise_matmul_bwd(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* dy,
                                      int64_t lddy, const uint8_t* tile_mask, int64_t groups, int64_t rows_per_group,
                                      int64_t block_k, int64_t block_n, int64_t M, int64_t N, int64_t K, int dtype,
