@@ -800,7 +800,7 @@ def main():
     EAGER = args.eager
     if args.gpus != 1:
         print(f"bench.py: this build runs on one GPU; --gpus {args.gpus} is not supported "
-              "(the multi-GPU sharding of this path is described in DESIGN.md, not run)", file=sys.stderr)
+              "(the multi-GPU sharding of this path is described, not run)", file=sys.stderr)
         sys.exit(2)
 
     import __graft_entry__
@@ -931,7 +931,7 @@ def main():
     torch.cuda.empty_cache()
 
     if not args.no_workloads:
-        # The other SURVEY configs, each one JSON sub-object with its own roofline and CPU baseline.
+        # The other workloads, each one JSON sub-object with its own roofline and CPU baseline.
         sub_args = argparse.Namespace(**vars(args))
         # 100 graph-replayed steps (20 measured 5-10 % slower per step than 200: the
         # shorter timed window starts on a GPU that idled through the CPU baselines)
