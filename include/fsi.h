@@ -291,12 +291,6 @@ FSI_API int fsi_decode_route(const void* qi, const float* kp, const void* vp, in
                              void* stream);
 
 /* ------------------------------------------------------------------------- *
- * FovealIndexer representations (foveal_indexer/core.py:214-312), index_dim 16.
- * The D -> 16 projections are plain GEMMs done by the caller; these entry
- * points apply everything after them with the reference's bf16 rounding points.
- * All tensors contiguous and of `dtype`.
- * ------------------------------------------------------------------------- */
-/* ------------------------------------------------------------------------- *
  * Products around the 16-D index (core.py:214-250, 288-312).
  * fsi_index_proj: y_i = x w_i^T for one or two (16, D) weights (w1 / y1 null: one); x row
  * (b, t) at x + b xs_b + t xs_t, y (B T, 16) contiguous.  fsi_index_proj_dw: dw_i = g_i^T x
@@ -322,6 +316,12 @@ FSI_API int fsi_index_expand_bwd(const void* dy, const void* ctx, const void* w,
                                  int64_t D, int dtype, void* dctx, void* dw, void* workspace, size_t workspace_bytes,
                                  void* stream);
 
+/* ------------------------------------------------------------------------- *
+ * FovealIndexer representations (foveal_indexer/core.py:214-312), index_dim 16.
+ * The D -> 16 projections are fsi_index_proj's or a GEMM's; these entry
+ * points apply everything after them with the reference's bf16 rounding points.
+ * All tensors contiguous and of `dtype`.
+ * ------------------------------------------------------------------------- */
 /* F.rms_norm over the 16 components (eps = FLT_EPSILON), x/out: (M, 16).
  * Replaces the norm of compute_query_16d (core.py:221-222) and of decode_step's
  * index key (attention.py:305). */
